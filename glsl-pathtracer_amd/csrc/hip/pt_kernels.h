@@ -44,6 +44,9 @@ struct ShadowBuf {
     float4* c;  // [2n]   ray k: contribution without the throughput
 };
 
+// LDS traversal-stack entries of k_finish (its blocks are one wave).
+constexpr int FINISH_S = 64;
+
 // Visibility record of the adjoint's primal pass: per path slot and bounce,
 // bit k of the bounce's two bits says NEE ray k (0 environment, 1 analytic
 // light) was valid and unoccluded. 16 bounces per 32-bit word; word array w
@@ -94,7 +97,8 @@ struct BatchBuf {
 
 namespace ptk {
 enum { KIND_PLAIN = 0, KIND_EXTEND = 1, KIND_SHADE = 2, KIND_SHADOW = 3, KIND_SHADE_BATCH = 4,
-       KIND_SHADE_INLINE = 5, KIND_SHADE_BATCH_INLINE = 6, KIND_REPLAY = 7, KIND_PLAIN_BATCH = 8 };
+       KIND_SHADE_INLINE = 5, KIND_SHADE_BATCH_INLINE = 6, KIND_REPLAY = 7, KIND_PLAIN_BATCH = 8,
+       KIND_FINISH = 9, KIND_FINISH_INLINE = 10 };
 
 // Resident blocks for a persistent launch (occupancy x CUs); extra_lds is the
 // replay stage's per-block gradient table.
@@ -106,7 +110,8 @@ void launch_extend(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, c
                    const ptd::PathBuf& pb, bool primary, const int* qin, const int* count_in, int npaths, int npix,
                    int first_sample, int* hitq, int* hit_count, int* work, int S, int* spill,
                    unsigned long long* counters, int* ovf, bool count, int budget = 0,
-                   const ptd::ContBuf* cb = nullptr, int* cont_count = nullptr);
+                   const ptd::ContBuf* cb = nullptr, int* cont_count = nullptr, int leave = 0);
+// leave: a later bounce that at most this many paths enter does nothing (launch_finish runs them).
 // A later bounce with budget > 0 (and not counting): traversals stop after
 // `budget` iterations into cb, each keeping a place in the hit queue;
 // launch_extend_resume then finishes them and fills those places (the slot,
@@ -114,6 +119,15 @@ void launch_extend(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, c
 void launch_extend_resume(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op,
                           const ptd::PathBuf& pb, const ptd::ContBuf& cb, const int* cont_count, int* hitq,
                           int* work, int S, int* spill, int* ovf);
+// Every path left after the stages of bounces [0, nb), run to its end (primary:
+// every path of the pass from its camera ray): the queue of the first bounce
+// whose entry count cells[b] is at most `limit`, or of bounce nb. qa, qb: the
+// queues of even and odd bounces; D: bounces of the pass in all; vis: the
+// adjoint's visibility words (arrays of vis_stride words), else null.
+void launch_finish(hipStream_t s, int blocks, const ptd::DevScene& sc, const ptd::DevOpts& op,
+                   const ptd::PathBuf& pb, const ptd::BatchBuf* bb, bool primary, bool inline_nee, const int* qa,
+                   const int* qb, const int* cells, int nb, int limit, int D, int npaths, int npix, int first_sample,
+                   int* work, int* spill, int* ovf, unsigned* vis = nullptr, int vis_stride = 0);
 // Shade stage; bb: the batched form's pass state (null: one frame); inline_nee:
 // NEE visibility resolved in the stage (stochastic alpha, volume MIS), else
 // queued as shadow records. S and spill: the traversal stack (inline_nee).

@@ -237,7 +237,8 @@ __device__ __forceinline__ void save_cont(const ContBuf& cb, int r, int slot, co
 // registers): at eight (64) more values spill and the traversal loop reloads
 // them around its stack pushes, which costs issue slots in a stage bound by
 // VALU issue (1080p: 19.6 -> 17.9 ms per frame; 4K heavy scene: 630 -> 569 ms;
-// six waves, 80 registers, is slower on both).
+// six waves, 80 registers, is slower on both). A later bounce that at most
+// `leave` paths enter is left to k_finish.
 // CAPPED (later bounces): a traversal runs at most `budget` loop iterations
 // here; a wave does not wait on its longest rays. Stopped traversals go to the
 // continuation buffer (while it has room and their stack is at most
@@ -251,7 +252,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
                                                 const int* count_in, int npaths, int npix, int first_sample,
                                                 int* hitq, int* hit_count, int* work, int S, int* spill,
                                                 unsigned long long* counters, int* ovf_flag, BatchBuf bb,
-                                                int budget, ContBuf cb, int* cont_count) {
+                                                int budget, ContBuf cb, int* cont_count, int leave) {
     static_assert(!CAPPED || (!COUNT && !PRIMARY), "only uninstrumented later bounces are capped");
     extern __shared__ int lds[];
     Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
@@ -259,7 +260,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
               static_cast<size_t>(gridDim.x) * blockDim.x};
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
-    const int count = PRIMARY ? (BATCH ? bb.cur[3] : npaths) : *count_in;
+    int count = PRIMARY ? (BATCH ? bb.cur[3] : npaths) : *count_in;
+    if (!PRIMARY && count <= leave) count = 0;  // few enough for k_finish
     for (WorkCursor<PRIMARY ? RUN_CAMERA : RUN_TRAVERSE> wc; wc.base < count; wc.next(work)) {
         const int i = wc.base + lane_id();
         bool keep = false, valid = false, done = false;
@@ -514,6 +516,87 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
         }
     }
     flush_counts<COUNT>(cnt, counters);
+    if (ovf) atomicOr(ovf_flag, 1);
+}
+
+// The rest of a pass's paths in one launch, once few are left (or, PRIMARY,
+// every path of a small pass from its camera ray on): each lane runs its path
+// to the end in registers (finish_path) and writes its radiance. What the
+// stages buy is full waves of paths at the same step; they pay with a launch
+// per stage and, per launch, the wait for its slowest ray. Once the paths left
+// fit the chip at once there is nothing to buy: a bounce's stage launches last
+// as long as their longest traversals, bounce after bounce, where a path that
+// goes on by itself waits for nobody. Few paths are spread over all waves (a
+// batch is count / waves lanes), so a wave's rays wait for fewer others and
+// mix fewer kinds of loop body. Measured, device time: the 640x360 preview of
+// 995 instances with alpha-tested foliage, whose paths may take 64 bounces
+// more than their depth, 43.2 -> 19.1 ms; 1280x720 spheres at one sample 3.0
+// -> 1.0; 256x256 Cornell box 0.61 -> 0.25; 4K foliage at four samples 428 ->
+// 395. One wave per block and the whole stack in LDS
+// (FINISH_S entries: at two waves per SIMD, all that 241 registers allow, LDS
+// has the room), so deep traversals do not go to the backing store.
+// The queue is that of the first bounce b in [1, nb] which the stages left
+// (count in cells[b] at most `limit`) or, at b == nb, could not start.
+// vis: visibility words as in k_shadow (array w at vis + w * vis_stride).
+template <bool PRIMARY, bool BATCH, bool INLINE_NEE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, const int* cells, int nb, int limit,
+         int D, int npaths, int npix, int first_sample, int* work, BatchBuf bb, int* spill, int* ovf_flag,
+         unsigned* vis, int vis_stride) {
+    extern __shared__ int lds[];
+    int b = 0, count = 0;
+    if (PRIMARY) {
+        count = BATCH ? bb.cur[3] : npaths;
+    } else {
+        for (b = 1; b <= nb; ++b) {
+            const int c = cells[b];
+            if (c > 0 && (c <= limit || b == nb)) { count = c; break; }
+        }
+    }
+    const int* q = (b & 1) ? qb : qa;
+    const int nw = static_cast<int>(gridDim.x);
+    const int per = min(64, (count + nw - 1) / nw);
+    Stack stk{lds, spill, static_cast<int>(threadIdx.x), 64, FINISH_S,
+              blockIdx.x * static_cast<size_t>(64) + threadIdx.x, static_cast<size_t>(gridDim.x) * 64};
+    bool ovf = false;
+    for (int base = static_cast<int>(blockIdx.x) * per; base < count;) {
+        const int l = lane_id(), i = base + l;
+        if (l < per && i < count) {
+            const int slot = PRIMARY ? i : q[i];
+            PathRegs p;
+            DevOpts op = op0;
+            bool valid = true;
+            if (BATCH) {
+                int job, smp, item;
+                batch_decode(bb, slot, job, smp, item);
+                const JobDev* J = bb.jobs + job;
+                if (PRIMARY) {
+                    const DevOpts oj = job_opts(op0, *J);
+                    int px, py;
+                    item_pixel(item, oj.width, px, py);
+                    valid = px < oj.width && py < oj.height;
+                    if (valid) primary_path(oj, px, py, smp, p);
+                }
+                op.max_depth = J->max_depth;
+            } else if (PRIMARY) {
+                int s, px, py;
+                valid = slot_pixel(op, slot, npix, s, px, py);
+                if (valid) primary_path(op, px, py, first_sample + s, p);
+            }
+            if (!PRIMARY) load_path(pb, slot, p);
+            if (valid) {
+                finish_path<INLINE_NEE>(sc, op, p, b, D, stk, ovf, [&](int bounce, int lit) {
+                    if (vis)
+                        vis[static_cast<size_t>(bounce / VIS_BOUNCES_PER_WORD) * vis_stride + slot] |=
+                            static_cast<unsigned>(lit) << (2 * (bounce % VIS_BOUNCES_PER_WORD));
+                });
+                pb.rad[slot] = F4(p.rad, p.alpha);
+            }
+        }
+        int next = 0;
+        if (l == 0) next = atomicAdd(work, per);
+        base = __builtin_amdgcn_readfirstlane(next) + nw * per;
+    }
     if (ovf) atomicOr(ovf_flag, 1);
 }
 
@@ -1293,6 +1376,8 @@ int persistent_blocks(int kind, int bs, int S, bool count, int num_cu, size_t ex
         case KIND_SHADE_BATCH: per_cu = max_blocks(k_shade<false, true, false>, bs, 0); break;
         case KIND_SHADE_INLINE: per_cu = max_blocks(k_shade<false, false, true>, bs, lds); break;
         case KIND_SHADE_BATCH_INLINE: per_cu = max_blocks(k_shade<false, true, true>, bs, lds); break;
+        case KIND_FINISH: per_cu = max_blocks(k_finish<false, false, false>, 64, FINISH_S * 64 * sizeof(int)); break;
+        case KIND_FINISH_INLINE: per_cu = max_blocks(k_finish<false, false, true>, 64, FINISH_S * 64 * sizeof(int)); break;
         case KIND_REPLAY: per_cu = max_blocks(k_replay_shade<false>, bs, extra_lds); break;
         default: break;
     }
@@ -1309,15 +1394,15 @@ void launch_plain(hipStream_t s, int blocks, int bs, const DevScene& sc, const D
 void launch_extend(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
                    bool primary, const int* qin, const int* count_in, int npaths, int npix, int first_sample,
                    int* hitq, int* hit_count, int* work, int S, int* spill, unsigned long long* counters, int* ovf,
-                   bool count, int budget, const ContBuf* cb, int* cont_count) {
+                   bool count, int budget, const ContBuf* cb, int* cont_count, int leave) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
     const BatchBuf nb{};
     const ContBuf nc{};
     if (budget > 0 && !primary && !count && cb && cont_count) {
-        hipLaunchKernelGGL((k_extend<false, false, false, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, budget, *cb, cont_count);
+        hipLaunchKernelGGL((k_extend<false, false, false, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, budget, *cb, cont_count, leave);
         return;
     }
-#define PT_EXT(C, P) hipLaunchKernelGGL((k_extend<C, P, false>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, 0, nc, nullptr)
+#define PT_EXT(C, P) hipLaunchKernelGGL((k_extend<C, P, false>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, 0, nc, nullptr, leave)
     if (count) { if (primary) PT_EXT(true, true); else PT_EXT(true, false); }
     else { if (primary) PT_EXT(false, true); else PT_EXT(false, false); }
 #undef PT_EXT
@@ -1328,6 +1413,23 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const DevScene& sc,
                           int* ovf) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
     hipLaunchKernelGGL(k_extend_resume, dim3(blocks), dim3(bs), lds, s, sc, op, pb, cb, cont_count, hitq, work, S, spill, ovf);
+}
+
+void launch_finish(hipStream_t s, int blocks, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
+                   const BatchBuf* bb, bool primary, bool inline_nee, const int* qa, const int* qb, const int* cells,
+                   int nb, int limit, int D, int npaths, int npix, int first_sample, int* work, int* spill, int* ovf,
+                   unsigned* vis, int vis_stride) {
+    const BatchBuf b = bb ? *bb : BatchBuf{};
+    const size_t lds = FINISH_S * 64 * sizeof(int);
+#define PT_FIN(P, B, I) hipLaunchKernelGGL((k_finish<P, B, I>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, vis, vis_stride)
+    if (bb) {
+        if (inline_nee) { if (primary) PT_FIN(true, true, true); else PT_FIN(false, true, true); }
+        else { if (primary) PT_FIN(true, true, false); else PT_FIN(false, true, false); }
+    } else {
+        if (inline_nee) { if (primary) PT_FIN(true, false, true); else PT_FIN(false, false, true); }
+        else { if (primary) PT_FIN(true, false, false); else PT_FIN(false, false, false); }
+    }
+#undef PT_FIN
 }
 
 void launch_shade(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
@@ -1369,7 +1471,7 @@ void launch_pass_end(hipStream_t s, const BatchBuf& bb) {
 void launch_extend_batch(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
                          const BatchBuf& bb, int* hitq, int* hit_count, int* work, int S, int* spill, int* ovf) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
-    hipLaunchKernelGGL((k_extend<false, true, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, nullptr, nullptr, 0, 0, 0, hitq, hit_count, work, S, spill, nullptr, ovf, bb, 0, ContBuf{}, nullptr);
+    hipLaunchKernelGGL((k_extend<false, true, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, nullptr, nullptr, 0, 0, 0, hitq, hit_count, work, S, spill, nullptr, ovf, bb, 0, ContBuf{}, nullptr, 0);
 }
 
 void launch_accum_batch(hipStream_t s, int blocks, const PathBuf& pb, const BatchBuf& bb) {

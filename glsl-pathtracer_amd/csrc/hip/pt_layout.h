@@ -122,6 +122,7 @@ struct Relayout {
     std::vector<int> inst_blas4_ref;        // each instance's four-wide BLAS root reference
     int tlas4_base = 0;                     // first four-wide TLAS entry in wide.nodes (at least max(n - 1, 1) follow)
     int root4 = 0;                          // four-wide TLAS root reference
+    long long traced_tris = 0;              // triangles over all instances (an estimate)
     // The TLAS as the device rebuild writes it: one instance per leaf, every
     // instance once, internal nodes numbered in preorder from tlas_base to the
     // end of the node array.
@@ -235,6 +236,14 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
         }
         R.tlas_rebuildable = ok && leaves == num_instances && internal == num_instances - 1 && base + internal == n;
         R.tlas_base = base;
+    }
+    {
+        // Triangles below every node, children first: the reference's trees are
+        // in preorder (another order only makes the estimate smaller).
+        std::vector<int> below(R.nodes.size(), 0);
+        auto tris_of = [&](int ref) { return ref < 0 ? (-1 - ref) & 3 : below[ref]; };
+        for (int i = n - 1; i >= 0; --i) below[i] = tris_of(R.nodes[i].d.x) + tris_of(R.nodes[i].d.y);
+        for (int i = 0; i < num_instances; ++i) R.traced_tris += tris_of(R.inst_blas_ref[i]);
     }
     R.inst_blas4_ref.assign(num_instances, 0);
     for (int i = 0; i < num_instances; ++i) {

@@ -101,6 +101,7 @@ struct pt_renderer_s {
     DevScene sc{};
     bool has_scene = false;
     int num_tris = 0, num_instances = 0, num_materials = 0;
+    long long traced_tris = 0;  // triangles over all instances (of the last full upload)
     bool any_alpha = false, any_medium = false, has_env = false;
     bool any_blend = false;  // a material with alphaMode BLEND (stochastic alpha)
     // host copy of the flat node array (for TLAS refresh) and node re-layout map
@@ -252,6 +253,7 @@ struct pt_renderer_s {
         root4_tlas = R.root4;
         t4_base = R.tlas4_base;
         t4_room = static_cast<int>(R.wide.nodes.size()) - R.tlas4_base;
+        traced_tris = R.traced_tris;
     }
     // Four-wide BLAS roots of BVH2 BLAS root references.
     std::vector<int> blas4_of(const std::vector<int>& blas2) const {
@@ -335,8 +337,19 @@ void check_ready(pt_renderer_s* h) {
 // Per pass: extend-queue counts [0, D], hit counts [D+1, 2D+1], shadow counts
 // [2D+2, 3D+2], three work counters per bounce [3D+3, 6D+3), then per bounce
 // the continuation count and the resume stage's work counter [6D+6, 8D+6).
-int counter_cells(int D) { return 8 * D + 6; }
+// Then the work counter of k_finish.
+int counter_cells(int D) { return 8 * D + 7; }
 int* cont_cells(int* cnt, int D, int b) { return cnt + 6 * D + 6 + 2 * b; }
+int* finish_cell(int* cnt, int D) { return cnt + 8 * D + 6; }
+
+// k_finish takes a pass over from the stages at the first later bounce whose
+// paths fill its grid at most once, and after FINISH_BOUNCES bounces at the
+// latest (alpha pass-through allows 64 bounces more than the path depth; that
+// late few paths are left, and a launch per stage would be made for nothing).
+// Measured on the 4K foliage frame of four samples: taken over at a quarter,
+// half, one, two and four fills 415, 412, 410, 412 and 421 ms (stages to the
+// end: 440); after 16, 30 and 40 bounces at the latest 461, 412 and 409.
+constexpr int FINISH_BOUNCES = 40;
 
 // NEE visibility is resolved inside the shade stage (shadow records are not
 // used) when AnyHit draws from the path's random numbers between NEE sampling
@@ -354,12 +367,47 @@ bool inline_nee(const pt_renderer_s* h, const DevOpts& op) {
     return needs_inline_nee(h, op) || h->opts.nee_inline == 1;
 }
 
+// Path state and queues of the stages (the radiance is p_rad).
+void ensure_paths(pt_renderer_s* h, size_t max_paths) {
+    h->p_ro.ensure(max_paths); h->p_rd.ensure(max_paths); h->p_thr.ensure(max_paths);
+    h->p_rng.ensure(max_paths); h->p_meta.ensure(max_paths); h->p_aux.ensure(max_paths);
+    if (h->any_medium) h->p_med.ensure(max_paths);
+    h->p_hit.ensure(max_paths); h->p_hit2.ensure(max_paths);
+    h->qa.ensure(max_paths); h->qb.ensure(max_paths); h->hq.ensure(max_paths);
+}
+
 void ensure_shadow(pt_renderer_s* h, size_t max_paths) {
     h->s_idx.ensure(max_paths); h->s_o.ensure(max_paths); h->s_t.ensure(max_paths);
     h->s_d.ensure(2 * max_paths); h->s_c.ensure(2 * max_paths);
 }
 
 ptd::ShadowBuf shadow_buf(pt_renderer_s* h) { return ptd::ShadowBuf{h->s_idx.p, h->s_o.p, h->s_t.p, h->s_d.p, h->s_c.p}; }
+
+// Use of k_finish in a pass: its blocks, the number of paths at or below which
+// it takes over from the stages and at or below which it runs the whole pass
+// (0: not used). Where the second line lies depends on how long a ray is:
+// stages pay off when many rays wait for long ones. Whole / staged in ms, with
+// the tail in k_finish either way (frames read back, depth 6), by paths:
+//   room or props of up to 4,000 triangles: 1M 2.6 / 3.6 (Cornell box), 2.2 /
+//     3.3 (sky), 2.6 / 6.0 (volume MIS); 8M 12.6 / 14.6, 9.1 / 9.2, 11.8 /
+//     15.2; 33M 46.8 / 49.6, 32.5 / 29.3, 43.1 / 39.3;
+//   0.2M to 1M triangles over all instances: 1M 3.6 / 4.9 and 2.0 / 2.9; 2M
+//     5.7 / 5.9 and 2.5 / 3.3; 4M 9.9 / 7.7 and 3.4 / 3.6;
+//   21M triangles with foliage: 0.23M 19.1 / 20.3; 0.5M 30 / 26; 1M 48 / 39.
+struct Finish { int blocks, leave, whole; };
+
+Finish finish_setup(pt_renderer_s* h, bool inl) {
+    Finish f{0, 0, 0};
+    // uncompacted queues and instrumented runs keep the stages throughout
+    if (std::max(1, h->opts.compact_every) != 1 || h->opts.count_work) return f;
+    f.blocks = ptk::persistent_blocks(inl ? ptk::KIND_FINISH_INLINE : ptk::KIND_FINISH, 64, ptd::FINISH_S, false,
+                                      h->num_cu);
+    h->spill.ensure(static_cast<size_t>(f.blocks) * 64 * (ptd::MAXD - ptd::FINISH_S + 1));
+    f.leave = f.blocks * 64;
+    const long long fills = h->traced_tris <= 16384 ? 64 : h->traced_tris <= 4000000 ? 16 : 2;
+    f.whole = static_cast<int>(std::min<long long>(fills * f.leave, INT32_MAX / 2));
+    return f;
+}
 
 // Launch shape and buffers of the wavefront form for passes of up to
 // spp_pass samples of every pixel.
@@ -369,6 +417,7 @@ struct Wavefront {
     size_t max_paths;
     int cap;            // extend_cap of later bounces (0: off)
     ptd::ContBuf cb;    // continuation buffer when cap > 0
+    Finish fin;
 };
 
 // adjoint: NEE always in the shadow stage, which records the visibility bits
@@ -382,13 +431,13 @@ Wavefront wavefront_setup(pt_renderer_s* h, const DevOpts& op, int num_samples, 
     const size_t max_paths = static_cast<size_t>(w.npix) * w.spp_pass;
     if (max_paths > static_cast<size_t>(INT32_MAX / 2)) throw ArgError(PT_ERR_OVERFLOW, "too many paths per pass");
     w.max_paths = max_paths;
-    h->p_ro.ensure(max_paths); h->p_rd.ensure(max_paths); h->p_thr.ensure(max_paths); h->p_rad.ensure(max_paths);
-    h->p_rng.ensure(max_paths); h->p_meta.ensure(max_paths); h->p_aux.ensure(max_paths);
-    if (h->any_medium) h->p_med.ensure(max_paths);
-    h->p_hit.ensure(max_paths); h->p_hit2.ensure(max_paths);
     w.inline_nee = adjoint ? false : inline_nee(h, op);
-    if (!w.inline_nee) ensure_shadow(h, max_paths);
-    h->qa.ensure(max_paths); h->qb.ensure(max_paths); h->hq.ensure(max_paths);
+    w.fin = finish_setup(h, w.inline_nee);
+    h->p_rad.ensure(max_paths);
+    // a pass that k_finish runs whole keeps no path state (the replay does)
+    const bool staged = max_paths > static_cast<size_t>(w.fin.whole);
+    if (staged || adjoint) ensure_paths(h, max_paths);
+    if (staged && !w.inline_nee) ensure_shadow(h, max_paths);
     // Bounce iterations: maxDepth + 1 closest hits; alpha pass-through repeats a depth.
     w.D = op.max_depth + 1 + ((op.flags & ptd::OPT_ALPHA_TEST) ? 64 : 0);
     h->counters.ensure(counter_cells(w.D));
@@ -399,7 +448,7 @@ Wavefront wavefront_setup(pt_renderer_s* h, const DevOpts& op, int num_samples, 
     w.b_ext = ptk::persistent_blocks(ptk::KIND_EXTEND, w.bs, w.S, w.cw, h->num_cu);
     // instrumented runs and the adjoint's passes traverse uncapped
     w.cap = (adjoint || w.cw) ? 0 : h->opts.extend_cap;
-    w.cb = w.cap > 0 ? h->cont_buf(max_paths) : ptd::ContBuf{};
+    w.cb = staged && w.cap > 0 ? h->cont_buf(max_paths) : ptd::ContBuf{};
     w.b_sha = ptk::persistent_blocks(w.inline_nee ? ptk::KIND_SHADE_INLINE : ptk::KIND_SHADE, w.bs, w.S, w.cw, h->num_cu);
     w.b_sdw = ptk::persistent_blocks(ptk::KIND_SHADOW, w.bs, w.S, w.cw, h->num_cu);
     // every traversing grid (extend, shadow, an inline-NEE shade) indexes the
@@ -422,7 +471,19 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
     int* qout = h->qb.p;
     int* c_ext = cnt;  // count of the current extend queue
     const int cadence = std::max(1, h->opts.compact_every);
-    for (int b = 0; b < D; ++b) {
+    auto finish = [&](bool primary, int nb) {
+        h->stage_begin(PT_STAGE_PLAIN, ev);
+        ptk::launch_finish(s, w.fin.blocks, h->sc, op, pb, nullptr, primary, w.inline_nee, h->qa.p, h->qb.p, cnt, nb,
+                           w.fin.leave, D, npaths, w.npix, fs, finish_cell(cnt, D), h->spill.p, h->ovf.p, vis,
+                           static_cast<int>(w.max_paths));
+        h->stage_end(PT_STAGE_PLAIN, ev);
+    };
+    if (w.fin.whole > 0 && w.max_paths <= static_cast<size_t>(w.fin.whole)) {
+        finish(true, 0);
+        return;
+    }
+    const int nb = w.fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
+    for (int b = 0; b < nb; ++b) {
         int* c_hit = cnt + (D + 1) + b;
         int* c_sh = cnt + 2 * (D + 1) + b;
         int* wk = cnt + 3 * (D + 1) + 3 * b;
@@ -437,7 +498,7 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
         h->stage_begin(PT_STAGE_EXTEND, ev);
         ptk::launch_extend(s, w.b_ext, w.bs, h->sc, op, pb, primary, qin, c_ext, npaths, w.npix, fs, h->hq.p, c_hit,
                            wk + 0, w.S, h->spill.p, h->work_counts.p, h->ovf.p, w.cw, capped ? w.cap : 0, &w.cb,
-                           c_cont);
+                           c_cont, w.fin.leave);
         if (capped)
             ptk::launch_extend_resume(s, w.b_ext, w.bs, h->sc, op, pb, w.cb, c_cont, h->hq.p, c_cont + 1, w.S,
                                       h->spill.p, h->ovf.p);
@@ -458,6 +519,7 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
             c_ext = c_next;
         }
     }
+    if (w.fin.leave > 0) finish(false, nb);
 }
 
 void render_wavefront(pt_renderer_s* h, int first_sample, int num_samples) {
@@ -687,14 +749,13 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     long long max_npix = 0;
     for (int j = 0; j < n; ++j)
         max_npix = std::max<long long>(max_npix, static_cast<long long>((jobs[j].width + 7) / 8) * ((jobs[j].height + 7) / 8) * 64);
+    const Finish fin = finish_setup(h, inl);
     const BatchPlan P = plan_batch(jobs, n, std::max(1, h->opts.wave_spp) * max_npix);
     const size_t max_paths = static_cast<size_t>(P.max_paths);
-    h->p_ro.ensure(max_paths); h->p_rd.ensure(max_paths); h->p_thr.ensure(max_paths); h->p_rad.ensure(max_paths);
-    h->p_rng.ensure(max_paths); h->p_meta.ensure(max_paths); h->p_aux.ensure(max_paths);
-    if (h->any_medium) h->p_med.ensure(max_paths);
-    h->p_hit.ensure(max_paths); h->p_hit2.ensure(max_paths);
-    if (!inl) ensure_shadow(h, max_paths);
-    h->qa.ensure(max_paths); h->qb.ensure(max_paths); h->hq.ensure(max_paths);
+    const bool whole = P.max_paths <= fin.whole;  // every pass in one launch of k_finish
+    h->p_rad.ensure(max_paths);
+    if (!whole) ensure_paths(h, max_paths);
+    if (!whole && !inl) ensure_shadow(h, max_paths);
     const int D = P.max_depth + 1 + ((op.flags & ptd::OPT_ALPHA_TEST) ? 64 : 0);
     const int ncells = counter_cells(D);
     h->counters.ensure(ncells);
@@ -702,7 +763,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     const int bs = h->block_size(), S = h->stack_S();
     const int b_ext = ptk::persistent_blocks(ptk::KIND_EXTEND, bs, S, false, h->num_cu);
     const int cap = h->opts.extend_cap;
-    const ptd::ContBuf cb = cap > 0 ? h->cont_buf(max_paths) : ptd::ContBuf{};
+    const ptd::ContBuf cb = cap > 0 && !whole ? h->cont_buf(max_paths) : ptd::ContBuf{};
     const int b_sha = ptk::persistent_blocks(inl ? ptk::KIND_SHADE_BATCH_INLINE : ptk::KIND_SHADE_BATCH, bs, S, false,
                                              h->num_cu);
     const int b_sdw = ptk::persistent_blocks(ptk::KIND_SHADOW, bs, S, false, h->num_cu);
@@ -737,7 +798,15 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
         int* qin = h->qa.p;
         int* qout = h->qb.p;
         int* c_ext = cnt;
-        for (int b = 0; b < D; ++b) {
+        auto finish = [&](bool primary, int nb) {
+            stage(PT_STAGE_PLAIN, [&] {
+                ptk::launch_finish(s, fin.blocks, h->sc, op, pb, &bb, primary, inl, h->qa.p, h->qb.p, cnt, nb, fin.leave,
+                                   D, 0, 0, 0, finish_cell(cnt, D), h->spill.p, h->ovf.p);
+            });
+        };
+        const int nb = whole ? 0 : fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
+        if (whole) finish(true, 0);
+        for (int b = 0; b < nb; ++b) {
             int* c_hit = cnt + (D + 1) + b;
             int* c_sh = cnt + 2 * (D + 1) + b;
             int* wk = cnt + 3 * (D + 1) + 3 * b;
@@ -750,7 +819,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
                     ptk::launch_extend_batch(s, b_ext, bs, h->sc, op, pb, bb, h->hq.p, c_hit, wk, S, h->spill.p, h->ovf.p);
                 } else {
                     ptk::launch_extend(s, b_ext, bs, h->sc, op, pb, false, qin, c_ext, 0, 0, 0, h->hq.p, c_hit, wk, S,
-                                       h->spill.p, h->work_counts.p, h->ovf.p, false, cap, &cb, c_cont);
+                                       h->spill.p, h->work_counts.p, h->ovf.p, false, cap, &cb, c_cont, fin.leave);
                     if (cap > 0)
                         ptk::launch_extend_resume(s, b_ext, bs, h->sc, op, pb, cb, c_cont, h->hq.p, c_cont + 1,
                                                   S, h->spill.p, h->ovf.p);
@@ -770,6 +839,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
                 c_ext = c_next;
             }
         }
+        if (!whole && fin.leave > 0) finish(false, nb);
         stage(PT_STAGE_ACCUM, [&] { ptk::launch_accum_batch(s, b_acc, pb, bb); });
         ptk::launch_pass_end(s, bb);
     };
