@@ -83,6 +83,7 @@ struct DevScene {
     const float* __restrict__ env_img;  // RGB32F
     const float* __restrict__ env_cdf;
     int root;                           // TLAS root reference (in nodes4 when that is set)
+    int far_nodes4;                     // 1: nodes4 holds 2^25 entries or more (beyond 32-bit byte offsets)
     int root_bin;                       // EMPTY4, or the BVH2 TLAS root that any-hit traversals drawing
                                         // random numbers walk (nodes4 set and a material blends)
     int num_lights;
@@ -731,7 +732,7 @@ struct Hit {
 
 struct TravCount { uint32_t nodes, tris, insts, lights, spills, rays; };
 
-// Traversal stack: entries [0, S) in LDS (entry i of lane tid at lds[i*bs + tid],
+// Traversal stack: entries [0, S) in LDS (entry i of a lane at lds[i*bs + lane],
 // conflict-free), deeper entries in a global backing store indexed by the
 // thread's slot. MAXD bounds the total depth; deeper trees set `overflow`.
 // The reference's binary traversal keeps 64 entries (closest_hit.glsl:89);
@@ -740,10 +741,10 @@ struct TravCount { uint32_t nodes, tris, insts, lights, spills, rays; };
 constexpr int MAXD = 96;
 
 struct Stack {
-    int* lds;          // this block's LDS array
+    int* lds;          // this wave's LDS entries
     int* spill;        // global backing store (MAXD - S entries per thread slot)
-    int lane;          // threadIdx.x
-    int bs;            // blockDim.x
+    int lane;          // lane of the wave
+    int bs;            // entry stride (64)
     int S;             // LDS entries
     size_t gslot;      // this thread's slot in the backing store
     size_t gstride;    // number of thread slots
@@ -759,6 +760,14 @@ struct Stack {
         return __hip_atomic_load(spill + static_cast<size_t>(sp - S) * gstride + gslot, __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_WAVEFRONT);
     }
+    // Cursors of the traversal loops: entry sp as its LDS index, so that a push
+    // or pop in LDS is one shift and add, and empty, full and in-LDS are
+    // compares with constants.
+    __device__ __forceinline__ int cursor(int sp) const { return sp * bs + lane; }
+    __device__ __forceinline__ int depth(int cur) const { return (cur - lane) / bs; }
+    __device__ __forceinline__ bool empty(int cur) const { return cur < bs; }
+    __device__ __forceinline__ bool room(int cur, int n) const { return cur < (S - n + 1) * bs; }  // n more in LDS
+    __device__ __forceinline__ void put(int cur, int v) { lds[cur] = v; }
 };
 
 __device__ __forceinline__ void inst_to_object(const GInst& I, vec3 o, vec3 d, vec3& oo, vec3& od) {
@@ -811,6 +820,80 @@ __device__ __forceinline__ bool alpha_transparent(const DevScene& sc, int row, i
 // the TLAS) and that instance. {root, 0, -1, -1} starts a traversal.
 struct TravState { int ref, sp, blas_base, cur_inst; };
 
+// Whether a ray's slab arithmetic can meet a NaN or leave the float range: a
+// direction component that is zero, tiny, infinite or NaN (its reciprocal is
+// then infinite, huge, zero or NaN), or an origin that is not finite or huge.
+__device__ __forceinline__ bool odd_ray(vec3 o, vec3 inv) {
+    const float big = 1e18f;
+    const bool d = fabsf(inv.x) <= big && fabsf(inv.y) <= big && fabsf(inv.z) <= big && inv.x != 0.0f &&
+                   inv.y != 0.0f && inv.z != 0.0f;
+    return !(d && fabsf(o.x) <= big && fabsf(o.y) <= big && fabsf(o.z) <= big);
+}
+
+// Four-wide node tests. A ray whose direction components are finite and not
+// zero enters a slab through the plane its sign says, so the near and far rows
+// are picked by address (one bit per axis, near ^ 16 is the far row) and the
+// per-axis min and max of slab() fall away: entry is the largest near distance,
+// exit the smallest far one, bit for bit what slab() gives (the smaller of two
+// products is the one the sign picks). Empty children hold a box that such a
+// ray misses (make_node4). A child is hit (slab()'s key > 0 and entry <= best)
+// when exit >= entry, exit > 0 and entry <= best; exit > 0 is folded into the
+// first compare (entry clamped to the smallest float above 0). k: the key of a
+// hit child, infinite for a child that is not hit. A traversing wave spends
+// its time on two things here: the issue slots of this code and the 112 bytes
+// a lane reads per node, which keep the CU's L1 return path busy (16 cycles per
+// 16-byte load of a wave, whatever lanes are active; measured busy 99% of the
+// closest-hit stage's cycles, with 1.2 VALU instructions per cycle and CU).
+// Against slab() per child, a count of hits before the sort and a bounds check
+// per push, the node step went from about 165 to 120 VALU instructions:
+// 1080p closest hits 16.3 -> 15.8 ms, tail of the 4K foliage frame 16.9 ->
+// 15.5, 995 moved instances 20.2 -> 18.1. Rays that may meet a NaN
+// (odd_ray: in a rendered image only for degenerate input) take slab() itself.
+struct Rows4 { uint32_t x, y, z; };  // byte offset of the near row of each axis
+__device__ __forceinline__ Rows4 near_rows(vec3 inv) {
+    return Rows4{inv.x < 0.0f ? 16u : 0u, inv.y < 0.0f ? 48u : 32u, inv.z < 0.0f ? 80u : 64u};
+}
+struct Kids4 { float k[4]; int4 ref; };
+
+__device__ __forceinline__ void test_node4(const GNode4* __restrict__ nodes, int ref, vec3 o, vec3 inv, Rows4 rows,
+                                           bool odd, float best, Kids4& c) {
+    const float none = __builtin_inff();
+    // 32-bit byte offsets: arrays of 2^25 nodes and more go through `odd` (the
+    // wrapped offset still lies in the array)
+    const char* base = reinterpret_cast<const char*>(nodes);
+    const uint32_t at = static_cast<uint32_t>(ref) << 7;
+    const uint32_t ax = at | rows.x, ay = at | rows.y, az = at | rows.z;
+    const float4 nx = *reinterpret_cast<const float4*>(base + ax), fx = *reinterpret_cast<const float4*>(base + (ax ^ 16u));
+    const float4 ny = *reinterpret_cast<const float4*>(base + ay), fy = *reinterpret_cast<const float4*>(base + (ay ^ 16u));
+    const float4 nz = *reinterpret_cast<const float4*>(base + az), fz = *reinterpret_cast<const float4*>(base + (az ^ 16u));
+    c.ref = *reinterpret_cast<const int4*>(base + (at | 96u));
+    const float n[4][3] = {{nx.x, ny.x, nz.x}, {nx.y, ny.y, nz.y}, {nx.z, ny.z, nz.z}, {nx.w, ny.w, nz.w}};
+    const float f[4][3] = {{fx.x, fy.x, fz.x}, {fx.y, fy.y, fz.y}, {fx.z, fy.z, fz.z}, {fx.w, fy.w, fz.w}};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float t0 = fmaxf((n[j][0] - o.x) * inv.x, fmaxf((n[j][1] - o.y) * inv.y, (n[j][2] - o.z) * inv.z));
+        const float t1 = fminf((f[j][0] - o.x) * inv.x, fminf((f[j][1] - o.y) * inv.y, (f[j][2] - o.z) * inv.z));
+        const bool hit = t1 >= fmaxf(t0, 0x1p-149f) && !(t0 > best);
+        c.k[j] = hit ? (t0 > 0.0f ? t0 : t1) : none;
+    }
+    if (odd) {
+        // one child after another: this path has no registers to spare
+        const float* g = reinterpret_cast<const float*>(nodes + ref);
+        c.ref = *reinterpret_cast<const int4*>(g + 24);
+#pragma unroll 1
+        for (int j = 0; j < 4; ++j) {
+            float t0;
+            float k = slab(g[j], g[8 + j], g[16 + j], g[4 + j], g[12 + j], g[20 + j], o, inv, t0);
+            const int r = reinterpret_cast<const int*>(g)[24 + j];
+            k = r != EMPTY4 && k > 0.0f && !(t0 > best) ? fminf(k, 3.40282347e38f) : none;
+            if (j == 0) c.k[0] = k;
+            if (j == 1) c.k[1] = k;
+            if (j == 2) c.k[2] = k;
+            if (j == 3) c.k[3] = k;
+        }
+    }
+}
+
 // Two-level traversal. ANY: return at the first accepted hit closer than
 // tmax; with `alpha` set, candidates are alpha-tested first (AnyHit with
 // OPT_ALPHA_TEST and no media).
@@ -825,69 +908,85 @@ struct TravState { int ref, sp, blas_base, cur_inst; };
 // hit does not depend on the order; what would is a stochastic alpha test,
 // whose draws follow the visit order, so callers that pass an RNG keep the
 // reference's order.
-template <bool ANY, bool COUNT, bool RESUME = false, bool UNORDERED = false>
-__device__ bool traverse(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& stk, Hit& h, TravCount& cnt,
-                         bool& overflow, bool alpha = false, Rng* rng = nullptr, TravState* ts = nullptr,
-                         int budget = -1) {
-    static_assert(!(ANY && RESUME), "only closest-hit traversals are resumed");
-    static_assert(!UNORDERED || ANY, "only any-hit traversals ignore the visit order");
+// WIDE: the four-wide form (one loop per form: in a common one the other
+// form's node test costs registers and moves in every iteration).
+template <bool WIDE, bool ANY, bool COUNT, bool RESUME, bool UNORDERED>
+__device__ __forceinline__ bool traverse_form(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& stk, Hit& h,
+                                              TravCount& cnt, bool& overflow, bool alpha, Rng* rng, TravState* ts,
+                                              int budget) {
     if (COUNT) cnt.rays++;
     const vec3 invD = V(1.0f / D.x, 1.0f / D.y, 1.0f / D.z);
     vec3 o = O, d = D, inv = invD;
     float best = tmax;
-    int sp = 0, blas_base = -1, cur_inst = -1, cur_mat = 0;
+    // top: cursor of the first free stack entry; blas_base: of the entry the
+    // current instance's BLAS began at (-1 in the TLAS)
+    int top = stk.cursor(0), blas_base = -1, cur_inst = -1, cur_mat = 0;
     int ref = sc.root;
     if (RESUME) {
-        ref = ts->ref; sp = ts->sp; blas_base = ts->blas_base; cur_inst = ts->cur_inst;
-        if (blas_base >= 0) {
+        ref = ts->ref; top = stk.cursor(ts->sp); cur_inst = ts->cur_inst;
+        if (ts->blas_base >= 0) {
+            blas_base = stk.cursor(ts->blas_base);
             inst_to_object(sc.inst[cur_inst], O, D, o, d);
             inv = V(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
         }
     }
+    Rows4 rows{0, 0, 0};
+    bool odd = false;
+    if (WIDE) {
+        rows = near_rows(inv);
+        odd = sc.far_nodes4 || odd_ray(o, inv);
+    }
     for (;;) {
         if (RESUME && budget-- == 0) {
-            ts->ref = ref; ts->sp = sp; ts->blas_base = blas_base; ts->cur_inst = cur_inst;
+            ts->ref = ref; ts->sp = stk.depth(top); ts->cur_inst = cur_inst;
+            ts->blas_base = blas_base < 0 ? -1 : stk.depth(blas_base);
             return false;
         }
         bool do_pop = false;
-        if (ref >= 0 && sc.nodes4) {
+        if (ref >= 0 && WIDE) {
             // Four-wide node (TLAS or BLAS): the hit children in order of the
             // reference's key (nearest first; equal keys in child order), the
             // nearest visited next, the others pushed farthest first.
             if (COUNT) cnt.nodes += 2;
-            const GNode4& n = sc.nodes4[ref];
-            const float4 lx = n.lox, hx = n.hix, ly = n.loy, hy = n.hiy, lz = n.loz, hz = n.hiz;
-            const int4 rf = n.ref;
-            float t0a, t0b, t0c, t0d;
-            float ka = slab(lx.x, ly.x, lz.x, hx.x, hy.x, hz.x, o, inv, t0a);
-            float kb = slab(lx.y, ly.y, lz.y, hx.y, hy.y, hz.y, o, inv, t0b);
-            float kc = slab(lx.z, ly.z, lz.z, hx.z, hy.z, hz.z, o, inv, t0c);
-            float kd = slab(lx.w, ly.w, lz.w, hx.w, hy.w, hz.w, o, inv, t0d);
-            const bool ha = rf.x != EMPTY4 && ka > 0.0f && !(t0a > best);
-            const bool hb = rf.y != EMPTY4 && kb > 0.0f && !(t0b > best);
-            const bool hc = rf.z != EMPTY4 && kc > 0.0f && !(t0c > best);
-            const bool hd = rf.w != EMPTY4 && kd > 0.0f && !(t0d > best);
-            const int c = int(ha) + int(hb) + int(hc) + int(hd);
-            if (c == 0) {
-                do_pop = true;
-            } else if (UNORDERED) {
+            Kids4 kid;
+            test_node4(sc.nodes4, ref, o, inv, rows, odd, best, kid);
+            const float none = __builtin_inff();
+            if (UNORDERED) {
                 // the first hit child next, the others pushed
-                if (sp + c - 1 > MAXD) { overflow = true; break; }
-                int first = EMPTY4;
-                if (ha) first = rf.x;
-                if (hb) { if (first == EMPTY4) first = rf.y; else stk.push(sp++, rf.y); }
-                if (hc) { if (first == EMPTY4) first = rf.z; else stk.push(sp++, rf.z); }
-                if (hd) { if (first == EMPTY4) first = rf.w; else stk.push(sp++, rf.w); }
-                ref = first;
+                const bool h0 = kid.k[0] < none, h1 = kid.k[1] < none, h2 = kid.k[2] < none, h3 = kid.k[3] < none;
+                const int4 rf = kid.ref;
+                if (!(h0 || h1 || h2 || h3)) {
+                    do_pop = true;
+                } else if (stk.room(top, 3)) {
+                    // all in LDS: every child after the first hit one is stored, a
+                    // missed one below the next (what lies above the new top is free)
+                    ref = h0 ? rf.x : h1 ? rf.y : h2 ? rf.z : rf.w;
+                    stk.put(top, rf.y);
+                    top += h0 && h1 ? stk.bs : 0;
+                    stk.put(top, rf.z);
+                    top += (h0 || h1) && h2 ? stk.bs : 0;
+                    stk.put(top, rf.w);
+                    top += (h0 || h1 || h2) && h3 ? stk.bs : 0;
+                } else {
+                    int sp = stk.depth(top);
+                    if (sp + int(h0) + int(h1) + int(h2) + int(h3) - 1 > MAXD) { overflow = true; break; }
+                    ref = h0 ? rf.x : h1 ? rf.y : h2 ? rf.z : rf.w;
+                    if (h0 && h1) stk.push(sp++, rf.y);
+                    if ((h0 || h1) && h2) stk.push(sp++, rf.z);
+                    if ((h0 || h1 || h2) && h3) stk.push(sp++, rf.w);
+                    top = stk.cursor(sp);
+                }
             } else {
-                const float big = __builtin_inff();
-                float q0 = ha ? ka : big, q1 = hb ? kb : big, q2 = hc ? kc : big, q3 = hd ? kd : big;
-                int r0 = rf.x, r1 = rf.y, r2 = rf.z, r3 = rf.w;
+                float q0 = kid.k[0], q1 = kid.k[1], q2 = kid.k[2], q3 = kid.k[3];
+                int r0 = kid.ref.x, r1 = kid.ref.y, r2 = kid.ref.z, r3 = kid.ref.w;
                 // sorting network on (key, ref); a pair swaps only on a strictly smaller key
 #define PT_CSWAP(qa, ra, qb, rb)                                      \
-    if (qb < qa) {                                                    \
-        const float tq = qa; qa = qb; qb = tq;                        \
-        const int tr = ra; ra = rb; rb = tr;                          \
+    {                                                                 \
+        const bool sw = qb < qa;                                      \
+        const float tq = sw ? qa : qb;                                \
+        qa = sw ? qb : qa; qb = tq;                                   \
+        const int tr = sw ? ra : rb;                                  \
+        ra = sw ? rb : ra; rb = tr;                                   \
     }
                 PT_CSWAP(q0, r0, q1, r1)
                 PT_CSWAP(q2, r2, q3, r3)
@@ -895,15 +994,31 @@ __device__ bool traverse(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& 
                 PT_CSWAP(q1, r1, q3, r3)
                 PT_CSWAP(q1, r1, q2, r2)
 #undef PT_CSWAP
-                if (sp + c - 1 > MAXD) { overflow = true; break; }
-                if (COUNT) {
-                    const int lo = sp > stk.S ? sp : stk.S, hi = sp + c - 1;
-                    if (hi > lo) cnt.spills += hi - lo;
+                const bool h1 = q1 < none, h2 = q2 < none, h3 = q3 < none;
+                const int more = int(h1) + int(h2) + int(h3);  // children to push
+                if (!(q0 < none)) {
+                    do_pop = true;
+                } else if (stk.room(top, 3)) {
+                    // all in LDS: three stores whatever the count (what lies above
+                    // the new top is free)
+                    stk.put(top, h3 ? r3 : (h2 ? r2 : r1));
+                    stk.put(top + stk.bs, h3 ? r2 : r1);
+                    stk.put(top + 2 * stk.bs, r1);
+                    top += more * stk.bs;
+                    ref = r0;
+                } else {
+                    int sp = stk.depth(top);
+                    if (sp + more > MAXD) { overflow = true; break; }
+                    if (COUNT) {
+                        const int lo = sp > stk.S ? sp : stk.S, hi = sp + more;
+                        if (hi > lo) cnt.spills += hi - lo;
+                    }
+                    if (h3) stk.push(sp++, r3);
+                    if (h2) stk.push(sp++, r2);
+                    if (h1) stk.push(sp++, r1);
+                    top = stk.cursor(sp);
+                    ref = r0;
                 }
-                if (c > 3) stk.push(sp++, r3);
-                if (c > 2) stk.push(sp++, r2);
-                if (c > 1) stk.push(sp++, r1);
-                ref = r0;
             }
         } else if (ref >= 0) {
             if (COUNT) cnt.nodes++;
@@ -916,9 +1031,15 @@ __device__ bool traverse(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& 
             if (hl && hr) {
                 int nearer = (!UNORDERED && kl > kr) ? n.d.y : n.d.x;
                 int farther = (!UNORDERED && kl > kr) ? n.d.x : n.d.y;
-                if (sp >= MAXD) { overflow = true; break; }
-                if (COUNT && sp >= stk.S) cnt.spills++;
-                stk.push(sp++, farther);
+                if (stk.room(top, 1)) {
+                    stk.put(top, farther);
+                } else {
+                    const int sp = stk.depth(top);
+                    if (sp >= MAXD) { overflow = true; break; }
+                    if (COUNT) cnt.spills++;
+                    stk.push(sp, farther);
+                }
+                top += stk.bs;
                 ref = nearer;
             } else if (hl) {
                 ref = n.d.x;
@@ -935,8 +1056,12 @@ __device__ bool traverse(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& 
             if (ANY && alpha) cur_mat = __float_as_int(I.f2.z);
             inst_to_object(I, O, D, o, d);
             inv = V(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-            blas_base = sp;
-            ref = __float_as_int(sc.nodes4 ? I.f2.w : I.f2.y);
+            if (WIDE) {
+                rows = near_rows(inv);
+                odd = sc.far_nodes4 || odd_ray(o, inv);
+            }
+            blas_base = top;
+            ref = __float_as_int(WIDE ? I.f2.w : I.f2.y);
         } else {
             const int code = -1 - ref;
             const int first = code >> 2, count = code & 3;
@@ -967,15 +1092,32 @@ __device__ bool traverse(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& 
             do_pop = true;
         }
         if (do_pop) {
-            if (blas_base >= 0 && sp == blas_base) {
+            if (top == blas_base) {
                 blas_base = -1;
                 o = O; d = D; inv = invD;
+                if (WIDE) {
+                    rows = near_rows(inv);
+                    odd = sc.far_nodes4 || odd_ray(o, inv);
+                }
             }
-            if (sp == 0) break;
-            ref = stk.pop(--sp);
+            if (stk.empty(top)) break;
+            top -= stk.bs;
+            ref = stk.room(top, 1) ? stk.lds[top] : stk.pop(stk.depth(top));
         }
     }
     return RESUME;
+}
+
+template <bool ANY, bool COUNT, bool RESUME = false, bool UNORDERED = false>
+__device__ bool traverse(const DevScene& sc, vec3 O, vec3 D, float tmax, Stack& stk, Hit& h, TravCount& cnt,
+                         bool& overflow, bool alpha = false, Rng* rng = nullptr, TravState* ts = nullptr,
+                         int budget = -1) {
+    static_assert(!(ANY && RESUME), "only closest-hit traversals are resumed");
+    static_assert(!UNORDERED || ANY, "only any-hit traversals ignore the visit order");
+    return sc.nodes4 ? traverse_form<true, ANY, COUNT, RESUME, UNORDERED>(sc, O, D, tmax, stk, h, cnt, overflow, alpha,
+                                                                         rng, ts, budget)
+                     : traverse_form<false, ANY, COUNT, RESUME, UNORDERED>(sc, O, D, tmax, stk, h, cnt, overflow, alpha,
+                                                                          rng, ts, budget);
 }
 
 // Light loop of ClosestHit (closest_hit.glsl:35-85): closest analytic light.

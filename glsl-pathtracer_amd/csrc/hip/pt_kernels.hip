@@ -14,6 +14,15 @@ namespace ptd {
 // ------------------------------------------------------------------ helpers
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// The thread's traversal stack: each wave has S * 64 entries of LDS of its own,
+// lane-interleaved, so an entry's address is a shift and an add.
+__device__ __forceinline__ Stack wave_stack(int* lds, int* spill, int S) {
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    return Stack{lds + wave * S * 64, spill, lane_id(), 64, S,
+                 blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
+                 static_cast<size_t>(gridDim.x) * blockDim.x};
+}
+
 // Work distribution of the persistent kernels. Every wave's first batch of 64
 // items is static (global wave index * 64); later batches are claimed in runs
 // of RUN batches with one atomic per wave on `counter`, offset past the
@@ -83,9 +92,7 @@ __global__ void __launch_bounds__(256) k_plain(DevScene sc, DevOpts op, float4* 
                                                int num_items, int* work, int S, int* spill,
                                                unsigned long long* counters, int* ovf_flag) {
     extern __shared__ int lds[];
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
-              static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     for (WorkCursor<RUN_TRAVERSE> wc; wc.base < num_items; wc.next(work)) {
@@ -255,9 +262,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
                                                 int budget, ContBuf cb, int* cont_count, int leave) {
     static_assert(!CAPPED || (!COUNT && !PRIMARY), "only uninstrumented later bounces are capped");
     extern __shared__ int lds[];
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
-              static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     int count = PRIMARY ? (BATCH ? bb.cur[3] : npaths) : *count_in;
@@ -331,9 +336,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
 k_extend_resume(DevScene sc, DevOpts op, PathBuf pb, ContBuf cb, const int* cont_count, int* hitq,
                 int* work, int S, int* spill, int* ovf_flag) {
     extern __shared__ int lds[];
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
-              static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     const int count = min(*cont_count, cb.cap);
@@ -378,9 +381,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene sc, DevOpts op0, PathBuf
                                                int* work, int compact, BatchBuf bb, int S, int* spill,
                                                unsigned long long* counters, int* ovf_flag) {
     extern __shared__ int lds[];
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
-              static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     const int count = *hit_count;
@@ -488,9 +489,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
                                                 int* work, int S, int* spill, unsigned long long* counters,
                                                 int* ovf_flag, unsigned* vis, int vshift) {
     extern __shared__ int lds[];
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
-              static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     const int count = *count_in;
@@ -556,8 +555,7 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
     const int* q = (b & 1) ? qb : qa;
     const int nw = static_cast<int>(gridDim.x);
     const int per = min(64, (count + nw - 1) / nw);
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), 64, FINISH_S,
-              blockIdx.x * static_cast<size_t>(64) + threadIdx.x, static_cast<size_t>(gridDim.x) * 64};
+    Stack stk = wave_stack(lds, spill, FINISH_S);
     bool ovf = false;
     for (int base = static_cast<int>(blockIdx.x) * per; base < count;) {
         const int l = lane_id(), i = base + l;
@@ -706,9 +704,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items, float4* __restrict__ accum,
               int* work, int S, int* spill, int* ovf_flag) {
     extern __shared__ int lds[];
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x,
-              static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     for (WorkCursor<RUN_TRAVERSE> wc; wc.base < items; wc.next(work)) {
@@ -1264,8 +1260,7 @@ __global__ void __launch_bounds__(256) k_query_closest(DevScene sc, DevOpts op, 
                                                        int* ovf_flag) {
     extern __shared__ int lds[];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              static_cast<size_t>(i), static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     if (i >= n) return;
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
@@ -1286,8 +1281,7 @@ __global__ void __launch_bounds__(256) k_query_any(DevScene sc, DevOpts op, cons
                                                    int n, int* occ, int S, int* spill, int* ovf_flag) {
     extern __shared__ int lds[];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    Stack stk{lds, spill, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x), S,
-              static_cast<size_t>(i), static_cast<size_t>(gridDim.x) * blockDim.x};
+    Stack stk = wave_stack(lds, spill, S);
     if (i >= n) return;
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;

@@ -246,6 +246,7 @@ struct pt_renderer_s {
     void select_bvh() {
         sc.nodes4 = (opts.bvh_width == 4 && nodes4.p) ? nodes4.p : nullptr;
         sc.root = sc.nodes4 ? root4_tlas : root2;
+        sc.far_nodes4 = nodes4.n >= (size_t{1} << 25) ? 1 : 0;
         sc.root_bin = (sc.nodes4 && any_blend) ? root2 : ptd::EMPTY4;
     }
     void set_tlas_roots(const Relayout& R) {

@@ -85,15 +85,28 @@ __host__ __device__ __forceinline__ int expand4(const GNode* n2, int off, int r,
     return k;
 }
 
+// A box of which one plane of an axis is NaN, as slab() takes it (the other
+// plane twice), for the four-wide test, which reads each plane by its side;
+// inverted planes the same way.
+__host__ __device__ __forceinline__ void tidy_box(float& lo, float& hi) {
+    if (!(lo <= hi)) {
+        const float a = lo, b = hi;
+        lo = fminf(a, b);
+        hi = fmaxf(a, b);
+    }
+}
+
 // GNode4 of up to four children; refs[] are the references written (internal
-// children already renumbered), EMPTY4 past count.
+// children already renumbered), EMPTY4 past count, with a box that no ray of
+// finite, non-zero direction enters.
 __host__ __device__ __forceinline__ GNode4 make_node4(const Child4 ch[4], int count, const int refs[4]) {
     float lo[3][4], hi[3][4];
     int rf[4];
     for (int k = 0; k < 4; ++k) {
         for (int a = 0; a < 3; ++a) {
-            lo[a][k] = k < count ? ch[k].lo[a] : 0.f;
-            hi[a][k] = k < count ? ch[k].hi[a] : 0.f;
+            lo[a][k] = k < count ? ch[k].lo[a] : __builtin_inff();
+            hi[a][k] = k < count ? ch[k].hi[a] : -__builtin_inff();
+            if (k < count) tidy_box(lo[a][k], hi[a][k]);
         }
         rf[k] = k < count ? refs[k] : EMPTY4;
     }

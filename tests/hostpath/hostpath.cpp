@@ -303,3 +303,47 @@ extern "C" int host_tlas4(const pt_scene_view* v, float* out, int cap, int* room
         return -1;
     }
 }
+
+// Node tests: n nodes of four children (boxes lo, hi [n*12], child count) and
+// n rays. For every child, test_node4's answer against slab() on the box as
+// given (the key where slab() hits and its entry is at most best, infinite
+// otherwise). Writes the children that differ, the hits and the rays that took
+// slab() itself.
+extern "C" int host_node4(int n, const float* lo, const float* hi, const int* count, const float* orig,
+                          const float* dir, const float* best, int* differ, int* hits, int* odds) {
+    int bad = 0, nh = 0, no = 0;
+    for (int i = 0; i < n; ++i) {
+        Child4 ch[4];
+        int refs[4];
+        for (int k = 0; k < 4; ++k) {
+            refs[k] = ch[k].ref = k;
+            for (int a = 0; a < 3; ++a) {
+                ch[k].lo[a] = lo[12 * i + 3 * k + a];
+                ch[k].hi[a] = hi[12 * i + 3 * k + a];
+            }
+        }
+        const GNode4 g = make_node4(ch, count[i], refs);
+        const vec3 o = V(orig[3 * i], orig[3 * i + 1], orig[3 * i + 2]);
+        const vec3 d = V(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]);
+        const vec3 inv = V(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+        const bool odd = odd_ray(o, inv);
+        no += odd;
+        Kids4 c;
+        test_node4(&g, 0, o, inv, near_rows(inv), odd, best[i], c);
+        for (int k = 0; k < 4; ++k) {
+            float want = HUGE_VALF;
+            if (k < count[i]) {
+                float t0;
+                const float key = slab(ch[k].lo[0], ch[k].lo[1], ch[k].lo[2], ch[k].hi[0], ch[k].hi[1], ch[k].hi[2], o,
+                                       inv, t0);
+                if (key > 0.0f && !(t0 > best[i])) want = fminf(key, 3.40282347e38f);
+            }
+            nh += want < HUGE_VALF;
+            if (memcmp(&want, &c.k[k], 4) != 0) bad++;
+        }
+    }
+    *differ = bad;
+    *hits = nh;
+    *odds = no;
+    return 0;
+}
