@@ -105,12 +105,17 @@ enum { KIND_PLAIN = 0, KIND_EXTEND = 1, KIND_SHADE = 2, KIND_SHADOW = 3, KIND_SH
 int persistent_blocks(int kind, int bs, int S, bool count, int num_cu, size_t extra_lds = 0);
 void launch_plain(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op, float4* accum,
                   int sample, int num_items, int* work, int S, int* spill, unsigned long long* counters, int* ovf,
-                  bool count);
+                  bool count, const int2* tiles);
+// Entries of the camera rays of every 8x8 tile (jobs: of every job, in item
+// order), read by the launches that take `tiles` (null: whole scene).
+void launch_tiles(hipStream_t s, const ptd::DevScene& sc, const ptd::DevOpts& op, const ptd::JobDev* jobs, int njobs,
+                  int ntiles, int2* out);
 void launch_extend(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op,
                    const ptd::PathBuf& pb, bool primary, const int* qin, const int* count_in, int npaths, int npix,
                    int first_sample, int* hitq, int* hit_count, int* work, int S, int* spill,
                    unsigned long long* counters, int* ovf, bool count, int budget = 0,
-                   const ptd::ContBuf* cb = nullptr, int* cont_count = nullptr, int leave = 0);
+                   const ptd::ContBuf* cb = nullptr, int* cont_count = nullptr, int leave = 0,
+                   const int2* tiles = nullptr);
 // leave: a later bounce that at most this many paths enter does nothing (launch_finish runs them).
 // A later bounce with budget > 0 (and not counting): traversals stop after
 // `budget` iterations into cb, each keeping a place in the hit queue;
@@ -127,7 +132,7 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const ptd::DevScene
 void launch_finish(hipStream_t s, int blocks, const ptd::DevScene& sc, const ptd::DevOpts& op,
                    const ptd::PathBuf& pb, const ptd::BatchBuf* bb, bool primary, bool inline_nee, const int* qa,
                    const int* qb, const int* cells, int nb, int limit, int D, int npaths, int npix, int first_sample,
-                   int* work, int* spill, int* ovf, unsigned* vis = nullptr, int vis_stride = 0);
+                   int* work, int* spill, int* ovf, const int2* tiles, unsigned* vis = nullptr, int vis_stride = 0);
 // Shade stage; bb: the batched form's pass state (null: one frame); inline_nee:
 // NEE visibility resolved in the stage (stochastic alpha, volume MIS), else
 // queued as shadow records. S and spill: the traversal stack (inline_nee).
@@ -153,13 +158,13 @@ void launch_pass_begin(hipStream_t s, const ptd::BatchBuf& bb, int* counters, in
 void launch_pass_end(hipStream_t s, const ptd::BatchBuf& bb);
 void launch_extend_batch(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op,
                          const ptd::PathBuf& pb, const ptd::BatchBuf& bb, int* hitq, int* hit_count, int* work, int S,
-                         int* spill, int* ovf);
+                         int* spill, int* ovf, const int2* tiles);
 void launch_accum_batch(hipStream_t s, int blocks, const ptd::PathBuf& pb, const ptd::BatchBuf& bb);
 // Batched render in one persistent launch of the plain form (jobs sorted by
 // item0, `items` = the sum of their npix).
 void launch_plain_batch(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op,
                         const ptd::JobDev* jobs, int njobs, int items, float4* accum, int* work, int S, int* spill,
-                        int* ovf);
+                        int* ovf, const int2* tiles);
 // Environment-map CDF and total luminance of an RGB32F image of n texels
 // (ok: one int of scratch; scratch: env_cdf_scratch_bytes(n) bytes, 8-byte aligned).
 // The parallel scan works in chunks of ENV_CDF_CHUNK texels (texels 1..n-1)

@@ -86,25 +86,94 @@ __device__ __forceinline__ void item_pixel(int i, int width, int& px, int& py) {
     py = (tile / tiles_x) * 8 + (l >> 3);
 }
 
+// Camera ray and initial state of a primary path (tile.glsl:41-69); the
+// bounce-0 stages recompute it instead of storing it.
+__device__ __forceinline__ void primary_path(const DevOpts& op, int px, int py, int sample, PathRegs& p) {
+    init_path(p);
+    p.rng = init_rng(static_cast<uint32_t>(px), static_cast<uint32_t>(py), static_cast<uint32_t>(sample + 2));
+    camera_ray(op, px, py, p.rng, p.ro, p.rd);
+}
+
+// Options of one job: shared switches, the job's camera, size and depth.
+__device__ __forceinline__ DevOpts job_opts(const DevOpts& op, const JobDev& J) {
+    DevOpts o = op;
+    o.width = J.width;
+    o.height = J.height;
+    o.max_depth = J.max_depth;
+    for (int i = 0; i < 3; ++i) {
+        o.cam_pos[i] = J.cam_pos[i];
+        o.cam_up[i] = J.cam_up[i];
+        o.cam_right[i] = J.cam_right[i];
+        o.cam_fwd[i] = J.cam_fwd[i];
+    }
+    o.cam_fov = J.cam_fov;
+    o.cam_focal = J.cam_focal;
+    o.cam_aperture = J.cam_aperture;
+    return o;
+}
+
+// ------------------------------------------------------------------ tile entries
+// One thread per 8x8 tile (of one camera, or of every job of a batch in item
+// order): where its camera rays begin (tile_entry). Read per wave, whose 64
+// paths are one tile's.
+__global__ void __launch_bounds__(64) k_tiles(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int ntiles,
+                                              int2* __restrict__ out) {
+    __shared__ int stack[CULL_STACK * 64];
+    const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= ntiles) return;
+    DevOpts op = op0;
+    int tile = t;
+    if (jobs) {
+        int lo = 0, hi = njobs - 1;  // the last job whose first item is <= the tile's
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (jobs[mid].item0 <= 64 * t) lo = mid;
+            else hi = mid - 1;
+        }
+        op = job_opts(op0, jobs[lo]);
+        tile = t - jobs[lo].item0 / 64;
+    }
+    Entry en{sc.root, true};
+    // a lens of positive radius has no single apex; a focal plane behind the
+    // camera turns the rays round
+    if (op.cam_aperture == 0.0f && op.cam_focal > 0.0f) en = tile_entry(sc, op, tile, stack + threadIdx.x, 64);
+    out[t] = make_int2(en.root, en.lights ? 1 : 0);
+}
+__device__ __forceinline__ Entry wave_entry(const DevScene& sc, const int2* tiles, int tile) {
+    if (!tiles) return whole_scene(sc);
+    const int2 t = tiles[__builtin_amdgcn_readfirstlane(tile)];
+    return Entry{__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y) != 0};
+}
+// The same for lanes of different tiles.
+__device__ __forceinline__ Entry lane_entry(const int2* tiles, int tile) {
+    const int2 t = tiles[tile];
+    return Entry{t.x, t.y != 0};
+}
+// Nothing in the tile's pyramid, and a miss that does not depend on the ray.
+__device__ __forceinline__ bool blank(const DevOpts& op, Entry en) {
+    return en.root == EMPTY4 && !en.lights && (!(op.flags & OPT_ENVMAP) || (op.flags & OPT_UNIFORM_LIGHT));
+}
+
 // ------------------------------------------------------------------ plain kernel
 template <bool COUNT>
 __global__ void __launch_bounds__(256) k_plain(DevScene sc, DevOpts op, float4* __restrict__ accum, int sample,
                                                int num_items, int* work, int S, int* spill,
-                                               unsigned long long* counters, int* ovf_flag) {
+                                               unsigned long long* counters, int* ovf_flag,
+                                               const int2* __restrict__ tiles) {
     extern __shared__ int lds[];
     Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     for (WorkCursor<RUN_TRAVERSE> wc; wc.base < num_items; wc.next(work)) {
         const int i = wc.base + lane_id();
+        const Entry en = wave_entry(sc, tiles, wc.base >> 6);
         int px, py;
         item_pixel(i, op.width, px, py);
         if (i < num_items && px < op.width && py < op.height) {
             PathRegs p;
-            init_path(p);
-            p.rng = init_rng(static_cast<uint32_t>(px), static_cast<uint32_t>(py), static_cast<uint32_t>(sample + 2));
-            camera_ray(op, px, py, p.rng, p.ro, p.rd);
-            float4 c = path_trace<COUNT>(sc, op, p, stk, cnt, ovf);
+            if (blank(op, en)) init_path(p);
+            else primary_path(op, px, py, sample, p);
+            float4 c = path_trace<COUNT>(sc, op, p, stk, cnt, ovf, en);
             float4* a = accum + static_cast<size_t>(py) * op.width + px;
             float4 acc = *a;
             acc.x += c.x; acc.y += c.y; acc.z += c.z; acc.w += c.w;
@@ -162,14 +231,6 @@ __device__ __forceinline__ void store_path(const PathBuf& pb, int slot, const Pa
 // meta.y flag of a path that ended in a bounce whose queue was not compacted.
 constexpr int PATH_DEAD = 1 << 18;
 
-// Camera ray and initial state of a primary path (tile.glsl:41-69); the
-// bounce-0 stages recompute it instead of storing it.
-__device__ __forceinline__ void primary_path(const DevOpts& op, int px, int py, int sample, PathRegs& p) {
-    init_path(p);
-    p.rng = init_rng(static_cast<uint32_t>(px), static_cast<uint32_t>(py), static_cast<uint32_t>(sample + 2));
-    camera_ray(op, px, py, p.rng, p.ro, p.rd);
-}
-
 // ---- batched render: slot -> (job, sample, pixel item) of the current pass
 __device__ __forceinline__ void batch_decode(const BatchBuf& bb, int slot, int& job, int& sample, int& item) {
     const int p0 = bb.cur[1], np = bb.cur[2];
@@ -183,24 +244,6 @@ __device__ __forceinline__ void batch_decode(const BatchBuf& bb, int slot, int& 
     job = pl.job;
     sample = pl.sample;
     item = slot - pl.slot0;
-}
-
-// Options of one job: shared switches, the job's camera, size and depth.
-__device__ __forceinline__ DevOpts job_opts(const DevOpts& op, const JobDev& J) {
-    DevOpts o = op;
-    o.width = J.width;
-    o.height = J.height;
-    o.max_depth = J.max_depth;
-    for (int i = 0; i < 3; ++i) {
-        o.cam_pos[i] = J.cam_pos[i];
-        o.cam_up[i] = J.cam_up[i];
-        o.cam_right[i] = J.cam_right[i];
-        o.cam_fwd[i] = J.cam_fwd[i];
-    }
-    o.cam_fov = J.cam_fov;
-    o.cam_focal = J.cam_focal;
-    o.cam_aperture = J.cam_aperture;
-    return o;
 }
 
 // End of a path's closest-hit step: a miss finishes the path here (environment
@@ -259,7 +302,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
                                                 const int* count_in, int npaths, int npix, int first_sample,
                                                 int* hitq, int* hit_count, int* work, int S, int* spill,
                                                 unsigned long long* counters, int* ovf_flag, BatchBuf bb,
-                                                int budget, ContBuf cb, int* cont_count, int leave) {
+                                                int budget, ContBuf cb, int* cont_count, int leave,
+                                                const int2* __restrict__ tiles) {
     static_assert(!CAPPED || (!COUNT && !PRIMARY), "only uninstrumented later bounces are capped");
     extern __shared__ int lds[];
     Stack stk = wave_stack(lds, spill, S);
@@ -274,20 +318,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
         PathRegs p;
         Hit h;
         TravState ts;
+        Entry en = whole_scene(sc);
         if (i < count) {
             slot = PRIMARY ? i : qin[i];
             valid = true;
             if (PRIMARY && BATCH) {
                 int job, smp, item, px, py;
                 batch_decode(bb, slot, job, smp, item);
-                const DevOpts oj = job_opts(op, bb.jobs[job]);
+                const JobDev& J = bb.jobs[job];
+                const DevOpts oj = job_opts(op, J);
+                en = wave_entry(sc, tiles, (J.item0 + item) >> 6);
                 item_pixel(item, oj.width, px, py);
                 valid = px < oj.width && py < oj.height;
-                if (valid) primary_path(oj, px, py, smp, p);
+                if (blank(op, en)) init_path(p);
+                else if (valid) primary_path(oj, px, py, smp, p);
             } else if (PRIMARY) {
                 int s, px, py;
                 valid = slot_pixel(op, slot, npix, s, px, py);
-                if (valid) primary_path(op, px, py, first_sample + s, p);
+                en = wave_entry(sc, tiles, (slot - s * npix) >> 6);
+                if (blank(op, en)) init_path(p);
+                else if (valid) primary_path(op, px, py, first_sample + s, p);
             } else {
                 const int2 mt = *reinterpret_cast<const int2*>(&pb.meta[slot]);
                 valid = !(mt.y & PATH_DEAD);  // ended path left in an uncompacted queue
@@ -301,7 +351,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
                 if (CAPPED) {
                     done = closest_begin(sc, op, p.ro, p.rd, p.depth, stk, ovf, h, ts, budget);
                 } else {
-                    h = closest<COUNT>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf);
+                    h = closest<COUNT>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
                     done = true;
                 }
             }
@@ -541,7 +591,7 @@ template <bool PRIMARY, bool BATCH, bool INLINE_NEE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, const int* cells, int nb, int limit,
          int D, int npaths, int npix, int first_sample, int* work, BatchBuf bb, int* spill, int* ovf_flag,
-         unsigned* vis, int vis_stride) {
+         unsigned* vis, int vis_stride, const int2* __restrict__ tiles) {
     extern __shared__ int lds[];
     int b = 0, count = 0;
     if (PRIMARY) {
@@ -563,6 +613,7 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
             const int slot = PRIMARY ? i : q[i];
             PathRegs p;
             DevOpts op = op0;
+            Entry en = whole_scene(sc);
             bool valid = true;
             if (BATCH) {
                 int job, smp, item;
@@ -573,17 +624,21 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
                     int px, py;
                     item_pixel(item, oj.width, px, py);
                     valid = px < oj.width && py < oj.height;
-                    if (valid) primary_path(oj, px, py, smp, p);
+                    if (tiles) en = lane_entry(tiles, (J->item0 + item) >> 6);
+                    if (blank(op0, en)) init_path(p);
+                    else if (valid) primary_path(oj, px, py, smp, p);
                 }
                 op.max_depth = J->max_depth;
             } else if (PRIMARY) {
                 int s, px, py;
                 valid = slot_pixel(op, slot, npix, s, px, py);
-                if (valid) primary_path(op, px, py, first_sample + s, p);
+                if (tiles) en = lane_entry(tiles, (slot - s * npix) >> 6);
+                if (blank(op, en)) init_path(p);
+                else if (valid) primary_path(op, px, py, first_sample + s, p);
             }
             if (!PRIMARY) load_path(pb, slot, p);
             if (valid) {
-                finish_path<INLINE_NEE>(sc, op, p, b, D, stk, ovf, [&](int bounce, int lit) {
+                finish_path<INLINE_NEE>(sc, op, p, b, D, stk, ovf, en, [&](int bounce, int lit) {
                     if (vis)
                         vis[static_cast<size_t>(bounce / VIS_BOUNCES_PER_WORD) * vis_stride + slot] |=
                             static_cast<unsigned>(lit) << (2 * (bounce % VIS_BOUNCES_PER_WORD));
@@ -702,7 +757,7 @@ __global__ void __launch_bounds__(256) k_replay_shade(DevScene sc, DevOpts op, P
 // takes 4 registers more than that allows.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items, float4* __restrict__ accum,
-              int* work, int S, int* spill, int* ovf_flag) {
+              int* work, int S, int* spill, int* ovf_flag, const int2* __restrict__ tiles) {
     extern __shared__ int lds[];
     Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
@@ -721,15 +776,17 @@ k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items
         item_pixel(item, width, px, py);
         if (item < Jp->npix && px < width && py < height) {
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+            const Entry en = wave_entry(sc, tiles, wc.base >> 6);
             for (int smp = 0; smp < spp; ++smp) {
                 // The camera is read again for each sample, after the previous
                 // trace (jobs is not restrict, so the trace's stores keep the
                 // loads here): only max_depth stays live through the trace.
                 PathRegs p;
-                primary_path(job_opts(op0, *Jp), px, py, smp, p);
+                if (blank(op0, en)) init_path(p);
+                else primary_path(job_opts(op0, *Jp), px, py, smp, p);
                 DevOpts op = op0;
                 op.max_depth = Jp->max_depth;
-                const float4 c = path_trace<false>(sc, op, p, stk, cnt, ovf);
+                const float4 c = path_trace<false>(sc, op, p, stk, cnt, ovf, en);
                 acc.x += c.x; acc.y += c.y; acc.z += c.z; acc.w += c.w;
             }
             accum[Jp->accum_off + static_cast<long long>(py) * width + px] = acc;
@@ -1378,25 +1435,31 @@ int persistent_blocks(int kind, int bs, int S, bool count, int num_cu, size_t ex
     return per_cu * num_cu;
 }
 
+void launch_tiles(hipStream_t s, const DevScene& sc, const DevOpts& op, const JobDev* jobs, int njobs, int ntiles,
+                  int2* out) {
+    hipLaunchKernelGGL(k_tiles, dim3((ntiles + 63) / 64), dim3(64), 0, s, sc, op, jobs, njobs, ntiles, out);
+}
+
 void launch_plain(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, float4* accum, int sample,
-                  int num_items, int* work, int S, int* spill, unsigned long long* counters, int* ovf, bool count) {
+                  int num_items, int* work, int S, int* spill, unsigned long long* counters, int* ovf, bool count,
+                  const int2* tiles) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
-    if (count) hipLaunchKernelGGL(k_plain<true>, dim3(blocks), dim3(bs), lds, s, sc, op, accum, sample, num_items, work, S, spill, counters, ovf);
-    else hipLaunchKernelGGL(k_plain<false>, dim3(blocks), dim3(bs), lds, s, sc, op, accum, sample, num_items, work, S, spill, counters, ovf);
+    if (count) hipLaunchKernelGGL(k_plain<true>, dim3(blocks), dim3(bs), lds, s, sc, op, accum, sample, num_items, work, S, spill, counters, ovf, tiles);
+    else hipLaunchKernelGGL(k_plain<false>, dim3(blocks), dim3(bs), lds, s, sc, op, accum, sample, num_items, work, S, spill, counters, ovf, tiles);
 }
 
 void launch_extend(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
                    bool primary, const int* qin, const int* count_in, int npaths, int npix, int first_sample,
                    int* hitq, int* hit_count, int* work, int S, int* spill, unsigned long long* counters, int* ovf,
-                   bool count, int budget, const ContBuf* cb, int* cont_count, int leave) {
+                   bool count, int budget, const ContBuf* cb, int* cont_count, int leave, const int2* tiles) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
     const BatchBuf nb{};
     const ContBuf nc{};
     if (budget > 0 && !primary && !count && cb && cont_count) {
-        hipLaunchKernelGGL((k_extend<false, false, false, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, budget, *cb, cont_count, leave);
+        hipLaunchKernelGGL((k_extend<false, false, false, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, budget, *cb, cont_count, leave, nullptr);
         return;
     }
-#define PT_EXT(C, P) hipLaunchKernelGGL((k_extend<C, P, false>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, 0, nc, nullptr, leave)
+#define PT_EXT(C, P) hipLaunchKernelGGL((k_extend<C, P, false>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, qin, count_in, npaths, npix, first_sample, hitq, hit_count, work, S, spill, counters, ovf, nb, 0, nc, nullptr, leave, tiles)
     if (count) { if (primary) PT_EXT(true, true); else PT_EXT(true, false); }
     else { if (primary) PT_EXT(false, true); else PT_EXT(false, false); }
 #undef PT_EXT
@@ -1412,10 +1475,10 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const DevScene& sc,
 void launch_finish(hipStream_t s, int blocks, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
                    const BatchBuf* bb, bool primary, bool inline_nee, const int* qa, const int* qb, const int* cells,
                    int nb, int limit, int D, int npaths, int npix, int first_sample, int* work, int* spill, int* ovf,
-                   unsigned* vis, int vis_stride) {
+                   const int2* tiles, unsigned* vis, int vis_stride) {
     const BatchBuf b = bb ? *bb : BatchBuf{};
     const size_t lds = FINISH_S * 64 * sizeof(int);
-#define PT_FIN(P, B, I) hipLaunchKernelGGL((k_finish<P, B, I>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, vis, vis_stride)
+#define PT_FIN(P, B, I) hipLaunchKernelGGL((k_finish<P, B, I>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, vis, vis_stride, tiles)
     if (bb) {
         if (inline_nee) { if (primary) PT_FIN(true, true, true); else PT_FIN(false, true, true); }
         else { if (primary) PT_FIN(true, true, false); else PT_FIN(false, true, false); }
@@ -1463,9 +1526,10 @@ void launch_pass_end(hipStream_t s, const BatchBuf& bb) {
 }
 
 void launch_extend_batch(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
-                         const BatchBuf& bb, int* hitq, int* hit_count, int* work, int S, int* spill, int* ovf) {
+                         const BatchBuf& bb, int* hitq, int* hit_count, int* work, int S, int* spill, int* ovf,
+                         const int2* tiles) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
-    hipLaunchKernelGGL((k_extend<false, true, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, nullptr, nullptr, 0, 0, 0, hitq, hit_count, work, S, spill, nullptr, ovf, bb, 0, ContBuf{}, nullptr, 0);
+    hipLaunchKernelGGL((k_extend<false, true, true>), dim3(blocks), dim3(bs), lds, s, sc, op, pb, nullptr, nullptr, 0, 0, 0, hitq, hit_count, work, S, spill, nullptr, ovf, bb, 0, ContBuf{}, nullptr, 0, tiles);
 }
 
 void launch_accum_batch(hipStream_t s, int blocks, const PathBuf& pb, const BatchBuf& bb) {
@@ -1473,10 +1537,11 @@ void launch_accum_batch(hipStream_t s, int blocks, const PathBuf& pb, const Batc
 }
 
 void launch_plain_batch(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const JobDev* jobs,
-                        int njobs, int items, float4* accum, int* work, int S, int* spill, int* ovf) {
+                        int njobs, int items, float4* accum, int* work, int S, int* spill, int* ovf,
+                        const int2* tiles) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
     hipLaunchKernelGGL(k_plain_batch, dim3(blocks), dim3(bs), lds, s, sc, op, jobs, njobs, items, accum, work, S, spill,
-                       ovf);
+                       ovf, tiles);
 }
 
 void launch_shadow(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,

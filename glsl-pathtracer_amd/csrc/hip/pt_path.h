@@ -63,14 +63,30 @@ __device__ __forceinline__ bool occluded(const DevScene& sc, const DevOpts& op, 
     return traverse<true, COUNT>(s, ro, rd, maxDist, stk, h, cnt, ovf, alpha, rng);
 }
 
+// Where the closest-hit query of a ray begins: the TLAS node to start at
+// (EMPTY4: no geometry) and whether an analytic light can be hit.
+struct Entry { int root; bool lights; };
+__device__ __forceinline__ Entry whole_scene(const DevScene& sc) { return Entry{sc.root, true}; }
+
+template <bool COUNT>
+__device__ __forceinline__ Hit closest(const DevScene& sc, const DevOpts& op, vec3 ro, vec3 rd, int depth, Stack& stk,
+                                       TravCount& cnt, bool& ovf, Entry en) {
+    Hit h;
+    h.t = INF; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1; h.light = -1;
+    if (en.lights && (op.flags & OPT_LIGHTS) && (!(op.flags & OPT_HIDE_EMITTERS) || depth > 0))
+        hit_lights<COUNT>(sc, ro, rd, h, cnt);
+    if (en.root != EMPTY4) {
+        DevScene s = sc;
+        s.root = en.root;
+        traverse<false, COUNT>(s, ro, rd, h.t, stk, h, cnt, ovf);
+    }
+    return h;
+}
+
 template <bool COUNT>
 __device__ __forceinline__ Hit closest(const DevScene& sc, const DevOpts& op, vec3 ro, vec3 rd, int depth, Stack& stk,
                                        TravCount& cnt, bool& ovf) {
-    Hit h;
-    h.t = INF; h.u = 0.f; h.v = 0.f; h.tri = -1; h.inst = -1; h.light = -1;
-    if ((op.flags & OPT_LIGHTS) && (!(op.flags & OPT_HIDE_EMITTERS) || depth > 0)) hit_lights<COUNT>(sc, ro, rd, h, cnt);
-    traverse<false, COUNT>(sc, ro, rd, h.t, stk, h, cnt, ovf);
-    return h;
+    return closest<COUNT>(sc, op, ro, rd, depth, stk, cnt, ovf, whole_scene(sc));
 }
 
 // closest() in pieces: the analytic lights, then at most `budget` traversal
@@ -429,11 +445,12 @@ __device__ __forceinline__ void nee_rays(const DevScene& sc, const DevOpts& op, 
 // called out of line it spills the path's registers to scratch.
 template <bool COUNT>
 __device__ __forceinline__ float4 path_trace(const DevScene& sc, const DevOpts& op, PathRegs& p, Stack& stk, TravCount& cnt,
-                             bool& ovf) {
+                             bool& ovf, Entry en) {
     SurfState st;
     init_surf(st);
     for (;; p.depth++) {
-        Hit h = closest<COUNT>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf);
+        Hit h = closest<COUNT>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
+        en = whole_scene(sc);
         if (h.t == INF) { on_miss(sc, op, p); break; }
         Material m;
         float eta;
@@ -453,6 +470,153 @@ __device__ __forceinline__ float4 path_trace(const DevScene& sc, const DevOpts& 
     return make_float4(p.rad.x, p.rad.y, p.rad.z, p.alpha);
 }
 
+template <bool COUNT>
+__device__ __forceinline__ float4 path_trace(const DevScene& sc, const DevOpts& op, PathRegs& p, Stack& stk, TravCount& cnt,
+                             bool& ovf) {
+    return path_trace<COUNT>(sc, op, p, stk, cnt, ovf, whole_scene(sc));
+}
+
+// What a tile's camera rays can hit. All rays of an 8x8 tile leave the camera
+// position (aperture 0) inside the pyramid of the tile's pixels and their one
+// pixel of jitter, so a box, rectangle or sphere outside one of its four side
+// planes is hit by none of them. The planes get a quarter pixel more and the
+// objects the rounding of the rays and of the slab test many times over
+// (1e-5 of the coordinates involved), so nothing a ray's own test accepts is
+// left out. The entry is the deepest TLAS node with every instance in the
+// pyramid below it: the subtrees left out hold no hit, and below the entry the
+// visit order is that of the whole traversal.
+struct Pyramid {
+    double px, py, pz;        // apex
+    double n[4][3];           // inward plane normals (zero: no plane)
+    double norm;              // largest apex coordinate
+};
+__device__ __forceinline__ void tile_pyramid(const DevOpts& op, int tile, Pyramid& P) {
+    const int tiles_x = (op.width + 7) >> 3;
+    const double x0 = (tile % tiles_x) * 8, y0 = (tile / tiles_x) * 8;
+    const double w = op.width, h = op.height;
+    const double scale = static_cast<double>(tanf(op.cam_fov * 0.5f)), sy = h / w * scale;
+    // pixel centres, one pixel of jitter, a quarter pixel more
+    const double dx[2] = {(2.0 * (x0 + 0.5 - 1.25) / w - 1.0) * scale, (2.0 * (x0 + 7.5 + 1.25) / w - 1.0) * scale};
+    const double dy[2] = {(2.0 * (y0 + 0.5 - 1.25) / h - 1.0) * sy, (2.0 * (y0 + 7.5 + 1.25) / h - 1.0) * sy};
+    double c[4][3], m[3];  // corner directions in order around the pyramid, and one inside
+    for (int a = 0; a < 3; ++a) {
+        const double r = op.cam_right[a], u = op.cam_up[a], f = op.cam_fwd[a];
+        c[0][a] = dx[0] * r + dy[0] * u + f;
+        c[1][a] = dx[1] * r + dy[0] * u + f;
+        c[2][a] = dx[1] * r + dy[1] * u + f;
+        c[3][a] = dx[0] * r + dy[1] * u + f;
+        m[a] = 0.5 * (dx[0] + dx[1]) * r + 0.5 * (dy[0] + dy[1]) * u + f;
+    }
+    for (int k = 0; k < 4; ++k) {
+        const double* a = c[k];
+        const double* b = c[(k + 1) & 3];
+        double n[3] = {a[1] * b[2] - a[2] * b[1], a[2] * b[0] - a[0] * b[2], a[0] * b[1] - a[1] * b[0]};
+        const double in = n[0] * m[0] + n[1] * m[1] + n[2] * m[2];
+        const double s = in > 0.0 ? 1.0 : (in < 0.0 ? -1.0 : 0.0);
+        for (int j = 0; j < 3; ++j) P.n[k][j] = s == 0.0 ? 0.0 : s * n[j];
+    }
+    P.px = op.cam_pos[0]; P.py = op.cam_pos[1]; P.pz = op.cam_pos[2];
+    P.norm = fmax(fabs(P.px), fmax(fabs(P.py), fabs(P.pz)));
+}
+// Whether the box is outside one plane of the pyramid (NaN: not).
+__device__ __forceinline__ bool outside(const Pyramid& P, double lx, double ly, double lz, double hx, double hy,
+                                        double hz) {
+    const double e = 1e-5 * (P.norm + fmax(fabs(lx), fmax(fabs(ly), fabs(lz))) + fmax(fabs(hx), fmax(fabs(hy), fabs(hz))));
+    for (int k = 0; k < 4; ++k) {
+        const double nx = P.n[k][0], ny = P.n[k][1], nz = P.n[k][2];
+        const double far = (nx > 0.0 ? nx * (hx + e - P.px) : nx * (lx - e - P.px)) +
+                           (ny > 0.0 ? ny * (hy + e - P.py) : ny * (ly - e - P.py)) +
+                           (nz > 0.0 ? nz * (hz + e - P.pz) : nz * (lz - e - P.pz));
+        if (far < 0.0) return true;
+    }
+    return false;
+}
+// Children of TLAS node r, in either form: references and boxes.
+struct Kid { int ref; float lo[3], hi[3]; };
+__device__ __forceinline__ int tlas_kids(const DevScene& sc, int r, Kid k[4]) {
+    if (sc.nodes4) {
+        const float* g = reinterpret_cast<const float*>(sc.nodes4 + r);
+        int n = 0;
+        for (int j = 0; j < 4; ++j) {
+            const int ref = reinterpret_cast<const int*>(g)[24 + j];
+            if (ref == EMPTY4) continue;
+            k[n++] = Kid{ref, {g[j], g[8 + j], g[16 + j]}, {g[4 + j], g[12 + j], g[20 + j]}};
+        }
+        return n;
+    }
+    const GNode g = sc.nodes[r];
+    k[0] = Kid{g.d.x, {g.a.x, g.a.y, g.a.z}, {g.a.w, g.b.x, g.b.y}};
+    k[1] = Kid{g.d.y, {g.b.z, g.b.w, g.c.x}, {g.c.y, g.c.z, g.c.w}};
+    return 2;
+}
+__device__ __forceinline__ bool outside(const Pyramid& P, const Kid& k) {
+    return outside(P, k.lo[0], k.lo[1], k.lo[2], k.hi[0], k.hi[1], k.hi[2]);
+}
+// Entry of a tile. stack: CULL_STACK entries at stride `step`; a TLAS deeper
+// than that is not searched further and counts as hit.
+constexpr int CULL_STACK = 48;
+__device__ __forceinline__ Entry tile_entry(const DevScene& sc, const DevOpts& op, int tile, int* stack, int step) {
+    Pyramid P;
+    tile_pyramid(op, tile, P);
+    Entry en{sc.root, false};
+    if ((op.flags & OPT_LIGHTS) && !(op.flags & OPT_HIDE_EMITTERS)) {
+        for (int i = 0; i < sc.num_lights && !en.lights; ++i) {
+            const GLight& L = sc.lights[i];
+            if (L.u.w == static_cast<float>(QUAD_LIGHT)) {
+                // RectIntersect accepts the points of the light's plane whose
+                // projections on u and v lie within them: the parallelogram with
+                // corners x, x.u = i u.u, x.v = j v.v (i, j in {0, 1}), which is
+                // the light's own where u and v are at right angles
+                const double u[3] = {L.u.x, L.u.y, L.u.z}, v[3] = {L.v.x, L.v.y, L.v.z};
+                const double uu = u[0] * u[0] + u[1] * u[1] + u[2] * u[2], vv = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+                const double uv = u[0] * v[0] + u[1] * v[1] + u[2] * v[2], det = uu * vv - uv * uv;
+                en.lights = true;
+                if (det > 1e-3 * uu * vv) {
+                    const float pos[3] = {L.p.x, L.p.y, L.p.z};
+                    double lo[3], hi[3];
+                    for (int a = 0; a < 3; ++a) {
+                        // corner (i, j) = i * (uu vv u - uu uv v) / det + j * (uu vv v - vv uv u) / det
+                        const double p = (uu * vv * u[a] - uu * uv * v[a]) / det, q = (uu * vv * v[a] - vv * uv * u[a]) / det;
+                        lo[a] = pos[a] + fmin(p, 0.0) + fmin(q, 0.0);
+                        hi[a] = pos[a] + fmax(p, 0.0) + fmax(q, 0.0);
+                    }
+                    en.lights = !outside(P, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]);
+                }
+            } else if (L.u.w == static_cast<float>(SPHERE_LIGHT)) {
+                const double r = fabs(static_cast<double>(L.p.w)) * 1.001;
+                en.lights = !outside(P, L.p.x - r, L.p.y - r, L.p.z - r, L.p.x + r, L.p.y + r, L.p.z + r);
+            }
+        }
+    }
+    while (en.root >= 0) {
+        Kid kids[4];
+        const int n = tlas_kids(sc, en.root, kids);
+        int seen = 0, only = EMPTY4;
+        for (int j = 0; j < n && seen < 2; ++j) {
+            if (outside(P, kids[j])) continue;
+            // does any instance below this child lie in the pyramid?
+            bool any = kids[j].ref < 0;
+            int sp = 0;
+            if (!any) { stack[0] = kids[j].ref; sp = 1; }
+            while (sp > 0 && !any) {
+                --sp;
+                Kid below[4];
+                const int m = tlas_kids(sc, stack[sp * step], below);
+                for (int i = 0; i < m && !any; ++i) {
+                    if (outside(P, below[i])) continue;
+                    if (below[i].ref < 0 || sp == CULL_STACK) any = true;
+                    else stack[sp++ * step] = below[i].ref;
+                }
+            }
+            if (any) { ++seen; only = kids[j].ref; }
+        }
+        if (seen == 0) { en.root = EMPTY4; break; }
+        if (seen > 1) break;
+        en.root = only;
+    }
+    return en;
+}
+
 // The rest of a path of the wavefront form, bounces b..D-1, in one go: the
 // same decisions, random draws and sums as the stage kernels make bounce by
 // bounce (the visible NEE contributions are added after the vertex's emission
@@ -460,10 +624,11 @@ __device__ __forceinline__ float4 path_trace(const DevScene& sc, const DevOpts& 
 // called for the visible NEE rays of bounce b (not with INLINE_NEE).
 template <bool INLINE_NEE, class Seen>
 __device__ __forceinline__ void finish_path(const DevScene& sc, const DevOpts& op, PathRegs& p, int b, int D,
-                                            Stack& stk, bool& ovf, Seen&& seen) {
+                                            Stack& stk, bool& ovf, Entry en, Seen&& seen) {
     TravCount cnt{0, 0, 0, 0, 0, 0};
     for (; b < D; ++b) {
-        const Hit h = closest<false>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf);
+        const Hit h = closest<false>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
+        en = whole_scene(sc);
         if (h.t == INF) { on_miss(sc, op, p); return; }
         SurfState st;
         init_surf(st);
