@@ -44,6 +44,17 @@ struct ShadowBuf {
     float4* c;  // [2n]   ray k: contribution without the throughput
 };
 
+// Counters of a pass lie CELL ints (a cache line) apart: atomics on one line
+// are served one after another.
+constexpr int CELL = 32;
+// Work counters (cells) of a persistent launch, one per share its items are
+// dealt out in.
+constexpr int SHARDS = 8;
+// Places of a queue for up to `items` items: appends in chunks leave at most an
+// eighth of the places read as empty ones, those of the stage before among
+// them (1/8 + 1/8^2 + ... = 1/7).
+inline size_t queue_room(size_t items) { return items + items / 7 + 64; }
+
 // LDS traversal-stack entries of k_finish (its blocks are one wave).
 constexpr int FINISH_S = 64;
 
@@ -186,6 +197,7 @@ inline LayoutSizes layout_sizes_here() {
                        sizeof(ptd::JobDev), sizeof(ptd::ContBuf)};
 }
 void launch_env_cdf(hipStream_t s, const float* img, int n, float* cdf, float* total, int* ok, void* scratch);
+void launch_zero_cells(hipStream_t s, int* cells, int n);  // cells 0..n-1, CELL ints apart
 void launch_fill(hipStream_t s, int* p, int n, int v);
 void launch_query_closest(hipStream_t s, const ptd::DevScene& sc, const ptd::DevOpts& op, const float* o,
                           const float* d, int n, float* t, int* inst, int* tri, int* light, float* uv, int S,

@@ -5,7 +5,10 @@
 // Reference behaviour (file:line in knightcrawler25/GLSL-PathTracer):
 //   bounce loop         src/shaders/common/pathtrace.glsl:285-476
 //   tonemap             src/shaders/tonemap.glsl:59-133
+#include <type_traits>
+
 #include "pt_kernels.h"
+
 #include "pt_path.h"
 #include "pt_replay.h"
 
@@ -23,48 +26,114 @@ __device__ __forceinline__ Stack wave_stack(int* lds, int* spill, int S) {
                  static_cast<size_t>(gridDim.x) * blockDim.x};
 }
 
-// Work distribution of the persistent kernels. Every wave's first batch of 64
-// items is static (global wave index * 64); later batches are claimed in runs
-// of RUN batches with one atomic per wave on `counter`, offset past the
-// static range. All waves of a grid share that one counter, and a wave waits
-// for the contended atomic's return before its next batch: claimed one batch
-// at a time by the camera-ray stage at 1080p it took half of the stage's time.
-// Runs trade that against the tail a long run left at the end of the queue
-// holds. Measured at 1080p (ms per frame): camera rays in runs of 4, 20.9 ->
-// 19.4 in the closest-hit stage against a static assignment (which gives a
-// wave tiles far apart); shade, whose items cost about the same, 8.2 -> 5.6
-// from runs of 1 to 16; shadow and later closest-hit bounces, whose items vary
-// with the traversal, best one batch at a time (shadow 6.5 -> 9.2 at 16).
-constexpr int RUN_CAMERA = 4, RUN_TRAVERSE = 1, RUN_SHADE = 16;
+// Work distribution of the persistent kernels. Batches of 64 items are dealt
+// out in runs to SHARES shares in turn (run r belongs to share r mod SHARES);
+// block b begins on share b mod SHARES. A wave's first run is static, later ones
+// are claimed with one atomic on the share's counter; a wave whose share is used
+// up goes on to the next ones. The chip serves one claim per 8.3 ns on one
+// counter: with a single one for the grid, 2.07M camera-ray batches at 1080p
+// took 31 ms claimed one by one, 19 in pairs and 13.9 four at a time, while
+// longer runs hold the tail of smaller launches (512x512x16 boxes: 10.3, 10.4,
+// 11.3 and, eight at a time, 13.1 ms), so runs grow with the batches a wave can
+// expect, up to MAX. Counters on lines of their own are served side by side:
+// with four, a batch of 16 Cornell jobs (cheap rays in every bounce) went from
+// 20.9 to 15.7 ms. Shares that do not help each other out leave a tail (1080p
+// shadow stage 4.1 -> 4.7 ms with two and more): the XCDs do not run equally fast.
 __device__ __forceinline__ int static_total() { return static_cast<int>(gridDim.x * (blockDim.x >> 6)) * 64; }
-__device__ __forceinline__ int first_batch() {
-    return static_cast<int>(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64;
-}
-template <int RUN>
+template <int MAX, int SHARES>
 struct WorkCursor {
-    int base, end;  // current batch; end of the claimed run
-    __device__ __forceinline__ WorkCursor() : base(first_batch()), end(first_batch() + 64) {}
-    __device__ __forceinline__ void next(int* counter) {
-        base += 64;
-        if (base < end) return;
-        int b = 0;
-        if (lane_id() == 0) b = atomicAdd(counter, 64 * RUN);
-        base = __builtin_amdgcn_readfirstlane(b) + static_total();
-        end = base + 64 * RUN;
+    static_assert(SHARES <= SHARDS, "one counter per share");
+    int base, end;    // current batch; end of the run
+    int share, left;  // share worked on, shares not used up
+    int run;          // items of a run
+    __device__ __forceinline__ int fixed() const {  // static runs of the share
+        return (static_cast<int>(gridDim.x) + SHARES - 1 - share) / SHARES * static_cast<int>(blockDim.x >> 6);
     }
+    __device__ __forceinline__ int start(int n) const { return (n * SHARES + share) * run; }
+    __device__ __forceinline__ explicit WorkCursor(int count)
+        : share(static_cast<int>(blockIdx.x) % SHARES), left(SHARES), run(64) {
+        if (MAX > 1) run = 64 * max(1, min(MAX, count / (32 * static_total())));
+        base = __builtin_amdgcn_readfirstlane(
+            start(static_cast<int>((blockIdx.x / SHARES) * (blockDim.x >> 6) + (threadIdx.x >> 6))));
+        end = base + run;
+    }
+    // The wave has a batch: its run's next one, or the first of a run claimed now.
+    __device__ __forceinline__ bool more(int* counters, int count) {
+        if (base < end && base < count) return true;
+        while (left > 0) {
+            int* c = counters + share * CELL;
+            int n = 0;
+            // another share's counter is read before it is claimed from
+            if (SHARES > 1 && left < SHARES)
+                n = __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (start(__builtin_amdgcn_readfirstlane(n) + fixed()) < count) {
+                if (lane_id() == 0) n = atomicAdd(c, 1);
+                base = __builtin_amdgcn_readfirstlane(start(__builtin_amdgcn_readfirstlane(n) + fixed()));
+                end = base + run;
+                if (base < count) return true;
+            }
+            --left;
+            share = share + 1 == SHARES ? 0 : share + 1;
+        }
+        return false;
+    }
+    __device__ __forceinline__ void step() { base += 64; }
 };
+using CameraCursor = WorkCursor<4, 8>;
+using ExtendCursor = WorkCursor<1, 4>;  // later bounces: an item's cost varies
+using ShadowCursor = WorkCursor<1, 4>;
+using ShadeCursor = WorkCursor<2, 8>;
+using PixelCursor = WorkCursor<1, 1>;  // whole paths of a pixel: few, long items
 
 // Wave-level stream compaction: one atomic per wave, lanes write at their
 // prefix position. Must be called by every lane of the wave.
+__device__ __forceinline__ int lanes_before(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
+                                     __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
+}
 __device__ __forceinline__ int wave_append(bool keep, int* counter) {
     const uint64_t mask = __ballot(keep);
     const int n = __popcll(mask);
-    const int prefix = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
-                                                 __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
     int base = 0;
     if (lane_id() == 0 && n > 0) base = atomicAdd(counter, n);
     base = __builtin_amdgcn_readfirstlane(base);
-    return keep ? base + prefix : -1;
+    return keep ? base + lanes_before(mask) : -1;
+}
+
+// The same with one atomic for many batches: a wave reserves `chunk` places of
+// the queue at a time and fills them batch by batch; the places left at its end
+// are marked empty (-1, which every reader of a queue skips). An append of its
+// own per batch costs 8.3 ns of the whole chip, as a claim does: the shade
+// stage made two per batch, 5.2 ms of its 5.8 at 1080p. The chunk follows the
+// batches a wave can expect (append_chunk), 0 where there are few: then every
+// batch appends for itself and the queue has no empty places.
+struct Append {
+    int at, end;  // reserved places not filled yet
+    __device__ __forceinline__ Append() : at(0), end(0) {}
+    __device__ __forceinline__ int take(bool keep, int* counter, int chunk) {
+        if (chunk == 0) return wave_append(keep, counter);
+        const uint64_t mask = __ballot(keep);
+        const int n = __popcll(mask), left = end - at;
+        int pos = at + lanes_before(mask);
+        if (n > left) {
+            int b = 0;
+            if (lane_id() == 0) b = atomicAdd(counter, chunk);
+            b = __builtin_amdgcn_readfirstlane(b);
+            if (pos >= end) pos = b + (pos - end);
+            at = b + (n - left);
+            end = b + chunk;
+        } else {
+            at += n;
+        }
+        return keep ? pos : -1;
+    }
+};
+// Places reserved at a time by a wave of a grid over `count` items: none below
+// eight batches per wave, else a sixteenth of them, 64 to 256 places (so at
+// most an eighth of the items' number of empty places).
+__device__ __forceinline__ int append_chunk(int count) {
+    const int per_wave = count / static_total();
+    return per_wave < 8 ? 0 : 64 * max(1, min(4, per_wave / 16));
 }
 
 template <bool COUNT>
@@ -164,7 +233,7 @@ __global__ void __launch_bounds__(256) k_plain(DevScene sc, DevOpts op, float4* 
     Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
-    for (WorkCursor<RUN_TRAVERSE> wc; wc.base < num_items; wc.next(work)) {
+    for (PixelCursor wc(num_items); wc.more(work, num_items); wc.step()) {
         const int i = wc.base + lane_id();
         const Entry en = wave_entry(sc, tiles, wc.base >> 6);
         int px, py;
@@ -311,7 +380,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
     bool ovf = false;
     int count = PRIMARY ? (BATCH ? bb.cur[3] : npaths) : *count_in;
     if (!PRIMARY && count <= leave) count = 0;  // few enough for k_finish
-    for (WorkCursor<PRIMARY ? RUN_CAMERA : RUN_TRAVERSE> wc; wc.base < count; wc.next(work)) {
+    const int chunk = COUNT ? 0 : append_chunk(count);  // instrumented: the hit count stays exact
+    Append hits, conts;
+    for (std::conditional_t<PRIMARY, CameraCursor, ExtendCursor> wc(count); wc.more(work, count); wc.step()) {
         const int i = wc.base + lane_id();
         bool keep = false, valid = false, done = false;
         int slot = -1;
@@ -322,7 +393,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
         if (i < count) {
             slot = PRIMARY ? i : qin[i];
             valid = true;
-            if (PRIMARY && BATCH) {
+            if (!PRIMARY && slot < 0) {  // empty place
+                valid = false;
+            } else if (PRIMARY && BATCH) {
                 int job, smp, item, px, py;
                 batch_decode(bb, slot, job, smp, item);
                 const JobDev& J = bb.jobs[job];
@@ -358,22 +431,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
         }
         if (CAPPED) {
             bool susp = valid && !done && ts.sp <= CONT_STACK;
-            const int r = wave_append(susp, cont_count);
+            const int r = conts.take(susp, cont_count, chunk);
             if (susp && r >= cb.cap) susp = false;  // no room: finish here
             if (!susp && valid && !done) {
                 traverse<false, false, true>(sc, p.ro, p.rd, h.t, stk, h, cnt, ovf, false, nullptr, &ts, -1);
                 done = true;
             }
             if (valid && done) keep = finish_extend<PRIMARY>(sc, op, pb, slot, p, h);
-            const int pos = wave_append(keep || susp, hit_count);
+            const int pos = hits.take(keep || susp, hit_count, chunk);
             if (keep) hitq[pos] = slot;
             if (susp) save_cont(cb, r, slot, ts, h, stk, pos);
         } else {
             if (valid && done) keep = finish_extend<PRIMARY>(sc, op, pb, slot, p, h);
-            const int pos = wave_append(keep, hit_count);
+            const int pos = hits.take(keep, hit_count, chunk);
             if (pos >= 0) hitq[pos] = slot;
         }
     }
+    for (int i = hits.at + lane_id(); i < hits.end; i += 64) hitq[i] = -1;
+    if (CAPPED)
+        for (int i = conts.at + lane_id(); i < min(conts.end, cb.cap); i += 64) cb.slot[i] = -1;
     flush_counts<COUNT>(cnt, counters);
     if (ovf) atomicOr(ovf_flag, 1);
 }
@@ -390,12 +466,12 @@ k_extend_resume(DevScene sc, DevOpts op, PathBuf pb, ContBuf cb, const int* cont
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     const int count = min(*cont_count, cb.cap);
-    for (WorkCursor<RUN_TRAVERSE> wc; wc.base < count; wc.next(work)) {
+    for (ExtendCursor wc(count); wc.more(work, count); wc.step()) {
         const int r = wc.base + lane_id();
         bool keep = false;
         int slot = -1;
-        if (r < count) {
-            slot = cb.slot[r];
+        if (r < count) slot = cb.slot[r];
+        if (slot >= 0) {  // -1: empty place
             const int4 st = cb.st[r];
             TravState ts{st.x, st.y, st.z, st.w};
             const float4 hf = cb.hf[r];
@@ -435,14 +511,16 @@ __global__ void __launch_bounds__(256) k_shade(DevScene sc, DevOpts op0, PathBuf
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     const int count = *hit_count;
-    for (WorkCursor<RUN_SHADE> wc; wc.base < count; wc.next(work)) {
+    const int chunk = append_chunk(count);
+    Append shadows, paths;
+    for (ShadeCursor wc(count); wc.more(work, count); wc.step()) {
         const int i = wc.base + lane_id();
         int slot = -1;
         bool keep = false;
         NeeRay nee[2];
         nee[0].valid = nee[1].valid = false;
         vec3 thr_nee = V1(0.f);
-        if (i < count) slot = hitq[i];  // -1: a place a resumed traversal left (a miss)
+        if (i < count) slot = hitq[i];  // -1: empty place, or one a resumed traversal left (a miss)
         if (slot >= 0) {
             PathRegs p;
             DevOpts op = op0;
@@ -504,7 +582,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene sc, DevOpts op0, PathBuf
             // contributions in DirectLight's order (no two threads update a
             // path's radiance).
             const int mask = (nee[0].valid ? 1 : 0) | (nee[1].valid ? 2 : 0);
-            const int pos = wave_append(mask != 0, shadow_count);
+            const int pos = shadows.take(mask != 0, shadow_count, chunk);
             if (pos >= 0) {
                 sb.idx[pos] = make_int2(slot, mask);
                 sb.o[pos] = F4(nee[(mask & 1) ? 0 : 1].o, 0.f);  // both rays start at the scatter point
@@ -517,10 +595,12 @@ __global__ void __launch_bounds__(256) k_shade(DevScene sc, DevOpts op0, PathBuf
             }
         }
         if (compact) {
-            const int pos = wave_append(keep, count_out);
+            const int pos = paths.take(keep, count_out, chunk);
             if (pos >= 0) qout[pos] = slot;
         }
     }
+    for (int i = shadows.at + lane_id(); i < shadows.end; i += 64) sb.idx[i] = make_int2(-1, 0);
+    for (int i = paths.at + lane_id(); i < paths.end; i += 64) qout[i] = -1;
     if (INLINE_NEE) {
         flush_counts<false>(cnt, counters);
         if (ovf) atomicOr(ovf_flag, 1);
@@ -543,10 +623,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
     const int count = *count_in;
-    for (WorkCursor<RUN_TRAVERSE> wc; wc.base < count; wc.next(work)) {
+    for (ShadowCursor wc(count); wc.more(work, count); wc.step()) {
         const int i = wc.base + lane_id();
         if (i < count) {
             const int2 id = sb.idx[i];
+            if (id.x < 0) continue;  // empty place
             const float4 o4 = sb.o[i];
             vec3 Ld = V1(0.0f);
             int lit = 0;
@@ -598,7 +679,7 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
         count = BATCH ? bb.cur[3] : npaths;
     } else {
         for (b = 1; b <= nb; ++b) {
-            const int c = cells[b];
+            const int c = cells[b * CELL];
             if (c > 0 && (c <= limit || b == nb)) { count = c; break; }
         }
     }
@@ -609,8 +690,8 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
     bool ovf = false;
     for (int base = static_cast<int>(blockIdx.x) * per; base < count;) {
         const int l = lane_id(), i = base + l;
-        if (l < per && i < count) {
-            const int slot = PRIMARY ? i : q[i];
+        const int slot = l < per && i < count ? (PRIMARY ? i : q[i]) : -1;  // -1: empty place too
+        if (slot >= 0) {
             PathRegs p;
             DevOpts op = op0;
             Entry en = whole_scene(sc);
@@ -674,12 +755,14 @@ __global__ void __launch_bounds__(256) k_replay_shade(DevScene sc, DevOpts op, P
         __syncthreads();
     }
     const int count = *hit_count;
-    for (WorkCursor<RUN_SHADE> wc; wc.base < count; wc.next(work)) {
+    const int chunk = append_chunk(count);
+    Append paths;
+    for (ShadeCursor wc(count); wc.more(work, count); wc.step()) {
         const int i = wc.base + lane_id();
         int slot = -1;
         bool keep = false;
-        if (i < count) {
-            slot = hitq[i];
+        if (i < count) slot = hitq[i];
+        if (slot >= 0) {  // -1: empty place
             int s, px, py;
             slot_pixel(op, slot, npix, s, px, py);
             PathRegs p;
@@ -736,10 +819,11 @@ __global__ void __launch_bounds__(256) k_replay_shade(DevScene sc, DevOpts op, P
             keep = rv.alive;
         }
         if (compact) {
-            const int pos = wave_append(keep, count_out);
+            const int pos = paths.take(keep, count_out, chunk);
             if (pos >= 0) qout[pos] = slot;
         }
     }
+    for (int i = paths.at + lane_id(); i < paths.end; i += 64) qout[i] = -1;
     if (rb.lds) {
         __syncthreads();
         for (int j = threadIdx.x; j < ng; j += blockDim.x)
@@ -762,7 +846,7 @@ k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items
     Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
     bool ovf = false;
-    for (WorkCursor<RUN_TRAVERSE> wc; wc.base < items; wc.next(work)) {
+    for (PixelCursor wc(items); wc.more(work, items); wc.step()) {
         int lo = 0, hi = njobs - 1;  // the last job whose first item is <= the batch's
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -815,7 +899,7 @@ __global__ void __launch_bounds__(256) k_accum(DevOpts op, PathBuf pb, float4* _
 // First node of a batched pass: make pass cur[0] current (copy its PassDev to
 // cur[1..8)) and zero the pass's queue and work counters.
 __global__ void __launch_bounds__(256) k_pass_begin(BatchBuf bb, int* counters, int ncounters) {
-    for (int i = threadIdx.x; i < ncounters; i += blockDim.x) counters[i] = 0;
+    for (int i = threadIdx.x; i < ncounters; i += blockDim.x) counters[i * CELL] = 0;
     if (threadIdx.x < 8) {
         const int* src = reinterpret_cast<const int*>(bb.passes + bb.cur[0]);
         bb.cur[1 + threadIdx.x] = threadIdx.x < 7 ? src[threadIdx.x] : 0;
@@ -1305,6 +1389,12 @@ __global__ void __launch_bounds__(ENV_SCAN_THREADS) k_env_scan(float* cdf, int n
     if (tid == 0) *total = n > 0 ? run : 0.0f;
 }
 
+// The counter cells of a pass.
+__global__ void k_zero_cells(int* cells, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) cells[i * CELL] = 0;
+}
+
 __global__ void k_fill_int(int* p, int n, int v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -1584,6 +1674,10 @@ void launch_env_cdf(hipStream_t s, const float* img, int n, float* cdf, float* t
         hipLaunchKernelGGL(k_env_chunk_write, dim3(nchunks), dim3(ZS_THREADS), ZL_WORDS * sizeof(int), s, cdf, n,
                            kguess, cstate, ok);
     hipLaunchKernelGGL(k_env_scan, dim3(1), dim3(ENV_SCAN_THREADS), 2 * ENV_CHUNK * sizeof(float), s, cdf, n, total, ok);
+}
+
+void launch_zero_cells(hipStream_t s, int* cells, int n) {
+    hipLaunchKernelGGL(k_zero_cells, dim3((n + 63) / 64), dim3(64), 0, s, cells, n);
 }
 
 void launch_fill(hipStream_t s, int* p, int n, int v) {

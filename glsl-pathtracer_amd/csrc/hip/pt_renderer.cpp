@@ -331,18 +331,27 @@ void check_ready(pt_renderer_s* h) {
     if (!h->has_cam) throw ArgError(PT_ERR_STATE, "no camera set (pt_set_camera)");
 }
 
-// Counter layout for one wavefront pass of D bounces (all zeroed per pass):
+// Counters of one wavefront pass of D bounces (all zeroed per pass), each on a
+// cache line of its own (ptd::CELL):
 //   [0, D+1)            paths entering extend at bounce b
 //   [D+1, 2D+2)         hits entering shade at bounce b
-//   [2D+2, 3D+3)        shadow rays of bounce b
-//   [3D+3, 6D+6)        work counters (extend, shade, shadow) of bounce b
-// Per pass: extend-queue counts [0, D], hit counts [D+1, 2D+1], shadow counts
-// [2D+2, 3D+2], three work counters per bounce [3D+3, 6D+3), then per bounce
-// the continuation count and the resume stage's work counter [6D+6, 8D+6).
-// Then the work counter of k_finish.
-int counter_cells(int D) { return 8 * D + 7; }
-int* cont_cells(int* cnt, int D, int b) { return cnt + 6 * D + 6 + 2 * b; }
-int* finish_cell(int* cnt, int D) { return cnt + 8 * D + 6; }
+//   [2D+2, 3D+3)        shadow records of bounce b
+//   [3D+3, 4D+3)        stopped traversals of bounce b
+//   4D+3                the work counter of k_finish
+//   from 4D+4           work counters (ptd::SHARDS each) of the extend, shade,
+//                       shadow and resume stages of bounce b
+int counter_cells(int D) { return 4 * D + 4 + 4 * D * ptd::SHARDS; }
+struct Cells {
+    int* base;
+    int D;
+    int* at(int i) const { return base + static_cast<size_t>(i) * ptd::CELL; }
+    int* paths(int b) const { return at(b); }
+    int* hits(int b) const { return at(D + 1 + b); }
+    int* shadows(int b) const { return at(2 * (D + 1) + b); }
+    int* conts(int b) const { return at(3 * (D + 1) + b); }
+    int* finish() const { return at(4 * D + 3); }
+    int* work(int b, int stage) const { return at(4 * D + 4 + (4 * b + stage) * ptd::SHARDS); }
+};
 
 // k_finish takes a pass over from the stages at the first later bounce whose
 // paths fill its grid at most once, and after FINISH_BOUNCES bounces at the
@@ -375,12 +384,14 @@ void ensure_paths(pt_renderer_s* h, size_t max_paths) {
     h->p_rng.ensure(max_paths); h->p_meta.ensure(max_paths); h->p_aux.ensure(max_paths);
     if (h->any_medium) h->p_med.ensure(max_paths);
     h->p_hit.ensure(max_paths); h->p_hit2.ensure(max_paths);
-    h->qa.ensure(max_paths); h->qb.ensure(max_paths); h->hq.ensure(max_paths);
+    const size_t room = ptd::queue_room(max_paths);
+    h->qa.ensure(room); h->qb.ensure(room); h->hq.ensure(room);
 }
 
 void ensure_shadow(pt_renderer_s* h, size_t max_paths) {
-    h->s_idx.ensure(max_paths); h->s_o.ensure(max_paths); h->s_t.ensure(max_paths);
-    h->s_d.ensure(2 * max_paths); h->s_c.ensure(2 * max_paths);
+    const size_t room = ptd::queue_room(max_paths);
+    h->s_idx.ensure(room); h->s_o.ensure(room); h->s_t.ensure(room);
+    h->s_d.ensure(2 * room); h->s_c.ensure(2 * room);
 }
 
 ptd::ShadowBuf shadow_buf(pt_renderer_s* h) { return ptd::ShadowBuf{h->s_idx.p, h->s_o.p, h->s_t.p, h->s_d.p, h->s_c.p}; }
@@ -462,7 +473,7 @@ Wavefront wavefront_setup(pt_renderer_s* h, const DevOpts& op, int num_samples, 
     if (staged && !w.inline_nee) ensure_shadow(h, max_paths);
     // Bounce iterations: maxDepth + 1 closest hits; alpha pass-through repeats a depth.
     w.D = op.max_depth + 1 + ((op.flags & ptd::OPT_ALPHA_TEST) ? 64 : 0);
-    h->counters.ensure(counter_cells(w.D));
+    h->counters.ensure(static_cast<size_t>(counter_cells(w.D)) * ptd::CELL);
     h->ensure_misc();
     w.bs = h->block_size();
     w.S = h->stack_S();
@@ -485,19 +496,19 @@ Wavefront wavefront_setup(pt_renderer_s* h, const DevOpts& op, int num_samples, 
 // words of the pass, ceil(D / 16) arrays of max_paths words.
 void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const ptd::PathBuf& pb,
                  const ptd::ShadowBuf& sb, int npaths, int fs, unsigned* vis) {
-    int* cnt = h->counters.p;
     hipStream_t s = h->stream;
     const int D = w.D;
+    const Cells cells{h->counters.p, D};
     hipEvent_t ev;
-    ptk::launch_fill(s, cnt, counter_cells(D), 0);
+    ptk::launch_zero_cells(s, cells.base, counter_cells(D));
     int* qin = h->qa.p;
     int* qout = h->qb.p;
-    int* c_ext = cnt;  // count of the current extend queue
+    int* c_ext = cells.paths(0);  // count of the current extend queue
     const int cadence = std::max(1, h->opts.compact_every);
     auto finish = [&](bool primary, int nb) {
         h->stage_begin(PT_STAGE_PLAIN, ev);
-        ptk::launch_finish(s, w.fin.blocks, h->sc, op, pb, nullptr, primary, w.inline_nee, h->qa.p, h->qb.p, cnt, nb,
-                           w.fin.leave, D, npaths, w.npix, fs, finish_cell(cnt, D), h->spill.p, h->ovf.p, w.tiles, vis,
+        ptk::launch_finish(s, w.fin.blocks, h->sc, op, pb, nullptr, primary, w.inline_nee, h->qa.p, h->qb.p, cells.base, nb,
+                           w.fin.leave, D, npaths, w.npix, fs, cells.finish(), h->spill.p, h->ovf.p, w.tiles, vis,
                            static_cast<int>(w.max_paths));
         h->stage_end(PT_STAGE_PLAIN, ev);
     };
@@ -507,33 +518,31 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
     }
     const int nb = w.fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
     for (int b = 0; b < nb; ++b) {
-        int* c_hit = cnt + (D + 1) + b;
-        int* c_sh = cnt + 2 * (D + 1) + b;
-        int* wk = cnt + 3 * (D + 1) + 3 * b;
+        int* c_hit = cells.hits(b);
+        int* c_sh = cells.shadows(b);
         const bool primary = b == 0;
         // bounce 0 always compacts (its input is the implicit slot range);
         // later bounces compact every `cadence`-th time, otherwise the next
         // extend re-reads this queue and skips ended paths.
         const bool compact = primary || (b % cadence) == 0;
-        int* c_next = compact ? cnt + b + 1 : c_ext;
-        int* c_cont = cont_cells(cnt, D, b);
+        int* c_next = compact ? cells.paths(b + 1) : c_ext;
         const bool capped = w.cap > 0 && !primary;
         h->stage_begin(PT_STAGE_EXTEND, ev);
         ptk::launch_extend(s, w.b_ext, w.bs, h->sc, op, pb, primary, qin, c_ext, npaths, w.npix, fs, h->hq.p, c_hit,
-                           wk + 0, w.S, h->spill.p, h->work_counts.p, h->ovf.p, w.cw, capped ? w.cap : 0, &w.cb,
-                           c_cont, w.fin.leave, w.tiles);
+                           cells.work(b, 0), w.S, h->spill.p, h->work_counts.p, h->ovf.p, w.cw, capped ? w.cap : 0, &w.cb,
+                           cells.conts(b), w.fin.leave, w.tiles);
         if (capped)
-            ptk::launch_extend_resume(s, w.b_ext, w.bs, h->sc, op, pb, w.cb, c_cont, h->hq.p, c_cont + 1, w.S,
+            ptk::launch_extend_resume(s, w.b_ext, w.bs, h->sc, op, pb, w.cb, cells.conts(b), h->hq.p, cells.work(b, 3), w.S,
                                       h->spill.p, h->ovf.p);
         h->stage_end(PT_STAGE_EXTEND, ev);
         h->stage_begin(PT_STAGE_SHADE, ev);
         ptk::launch_shade(s, w.b_sha, w.bs, h->sc, op, pb, sb, nullptr, primary, w.inline_nee, h->hq.p, c_hit, w.npix,
-                          fs, qout, c_next, c_sh, wk + 1, compact, w.S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
+                          fs, qout, c_next, c_sh, cells.work(b, 1), compact, w.S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
         h->stage_end(PT_STAGE_SHADE, ev);
         if (!w.inline_nee) {
             unsigned* vb = vis ? vis + static_cast<size_t>(b / ptd::VIS_BOUNCES_PER_WORD) * w.max_paths : nullptr;
             h->stage_begin(PT_STAGE_SHADOW, ev);
-            ptk::launch_shadow(s, w.b_sdw, w.bs, h->sc, op, pb, sb, c_sh, wk + 2, w.S, h->spill.p,
+            ptk::launch_shadow(s, w.b_sdw, w.bs, h->sc, op, pb, sb, c_sh, cells.work(b, 2), w.S, h->spill.p,
                                h->work_counts.p + 8, h->ovf.p, w.cw, vb, 2 * (b % ptd::VIS_BOUNCES_PER_WORD));
             h->stage_end(PT_STAGE_SHADOW, ev);
         }
@@ -560,8 +569,9 @@ void render_wavefront(pt_renderer_s* h, int first_sample, int num_samples) {
         HIPCHK(hipGetLastError());
         if (w.cw) {  // instrumented runs: hits per bounce of this pass (the counters are reused per pass)
             std::vector<int> hits(w.D);
-            HIPCHK(hipMemcpyAsync(hits.data(), h->counters.p + (w.D + 1), w.D * sizeof(int), hipMemcpyDeviceToHost,
-                                  h->stream));
+            const Cells cells{h->counters.p, w.D};
+            HIPCHK(hipMemcpy2DAsync(hits.data(), sizeof(int), cells.hits(0), ptd::CELL * sizeof(int), sizeof(int), w.D,
+                                    hipMemcpyDeviceToHost, h->stream));
             HIPCHK(hipStreamSynchronize(h->stream));
             for (int b = 0; b < w.D; ++b) h->stats.bounce_hits[std::min(b, 15)] += hits[b];
         }
@@ -607,8 +617,8 @@ void adjoint_wavefront(pt_renderer_s* h, int first_sample, int num_samples, floa
     rb.num_mats = h->num_materials;
     rb.lds = lds ? 1 : 0;
     hipStream_t s = h->stream;
-    int* cnt = h->counters.p;
     const int D = w.D;
+    const Cells cells{h->counters.p, D};
     const int cadence = std::max(1, h->opts.compact_every);
     for (int s0 = 0; s0 < num_samples; s0 += w.spp_pass) {
         const int ns = std::min(w.spp_pass, num_samples - s0);
@@ -616,26 +626,25 @@ void adjoint_wavefront(pt_renderer_s* h, int first_sample, int num_samples, floa
         ptk::launch_fill(s, reinterpret_cast<int*>(h->a_vis.p), static_cast<int>(vis_words), 0);
         run_bounces(h, op, w, pb, sb, npaths, fs, h->a_vis.p);
         // replay: the extend stage of the forward renderer, then the replay stage
-        ptk::launch_fill(s, cnt, counter_cells(D), 0);
+        ptk::launch_zero_cells(s, cells.base, counter_cells(D));
         int* qin = h->qa.p;
         int* qout = h->qb.p;
-        int* c_ext = cnt;
+        int* c_ext = cells.paths(0);
         hipEvent_t ev;
         for (int b = 0; b < D; ++b) {
-            int* c_hit = cnt + (D + 1) + b;
-            int* wk = cnt + 3 * (D + 1) + 3 * b;
+            int* c_hit = cells.hits(b);
             const bool primary = b == 0;
             const bool compact = primary || (b % cadence) == 0;
-            int* c_next = compact ? cnt + b + 1 : c_ext;
+            int* c_next = compact ? cells.paths(b + 1) : c_ext;
             h->stage_begin(PT_STAGE_EXTEND, ev);
             ptk::launch_extend(s, w.b_ext, w.bs, h->sc, op, pb2, primary, qin, c_ext, npaths, w.npix, fs, h->hq.p,
-                               c_hit, wk + 0, w.S, h->spill.p, h->work_counts.p, h->ovf.p, false, 0, nullptr, nullptr, 0,
+                               c_hit, cells.work(b, 0), w.S, h->spill.p, h->work_counts.p, h->ovf.p, false, 0, nullptr, nullptr, 0,
                                w.tiles);
             h->stage_end(PT_STAGE_EXTEND, ev);
             rb.vis = h->a_vis.p + static_cast<size_t>(b / ptd::VIS_BOUNCES_PER_WORD) * w.max_paths;
             h->stage_begin(PT_STAGE_ADJOINT, ev);
             ptk::launch_replay_shade(s, b_rep, w.bs, h->sc, op, pb2, primary, h->hq.p, c_hit, w.npix, fs, qout, c_next,
-                                     wk + 1, compact, rb, 2 * (b % ptd::VIS_BOUNCES_PER_WORD));
+                                     cells.work(b, 1), compact, rb, 2 * (b % ptd::VIS_BOUNCES_PER_WORD));
             h->stage_end(PT_STAGE_ADJOINT, ev);
             if (compact) {
                 std::swap(qin, qout);
@@ -747,12 +756,12 @@ void batch_render_plain(pt_renderer_s* h, const pt_job* jobs, int n) {
     hipStream_t s = h->stream;
     h->b_jobs.upload(P.jobs.data(), P.jobs.size(), s);
     h->b_accum.ensure(P.pixels);
-    h->counters.ensure(std::max<size_t>(h->counters.n, 8));
+    h->counters.ensure(ptd::SHARDS * ptd::CELL);
     h->ensure_misc();
     const int bs = h->block_size(), S = h->stack_S();
     const int blocks = ptk::persistent_blocks(ptk::KIND_PLAIN_BATCH, bs, S, false, h->num_cu);
     h->ensure_spill(static_cast<size_t>(blocks) * bs);
-    ptk::launch_fill(s, h->counters.p, 1, 0);
+    ptk::launch_zero_cells(s, h->counters.p, ptd::SHARDS);
     const int2* tiles = tile_entries(h, op, h->b_jobs.p, n, static_cast<int>(P.items / 64), P.max_side, P.samples);
     hipEvent_t ev;
     h->stage_begin(PT_STAGE_BATCH, ev);
@@ -787,7 +796,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     if (!whole && !inl) ensure_shadow(h, max_paths);
     const int D = P.max_depth + 1 + ((op.flags & ptd::OPT_ALPHA_TEST) ? 64 : 0);
     const int ncells = counter_cells(D);
-    h->counters.ensure(ncells);
+    h->counters.ensure(static_cast<size_t>(ncells) * ptd::CELL);
     h->ensure_misc();
     const int bs = h->block_size(), S = h->stack_S();
     const int b_ext = ptk::persistent_blocks(ptk::KIND_EXTEND, bs, S, false, h->num_cu);
@@ -811,7 +820,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     const ptd::PathBuf pb = path_buf(h);
     const ptd::ShadowBuf sb = shadow_buf(h);
     const int2* tiles = tile_entries(h, op, h->b_jobs.p, n, static_cast<int>(P.items / 64), P.max_side, P.samples);
-    int* cnt = h->counters.p;
+    const Cells cells{h->counters.p, D};
     const int cadence = std::max(1, h->opts.compact_every);
     const bool graph = h->opts.use_graph != 0;
 
@@ -824,45 +833,43 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
             launch();
             if (timed) h->stage_end(id, ev);
         };
-        ptk::launch_pass_begin(s, bb, cnt, ncells);
+        ptk::launch_pass_begin(s, bb, cells.base, ncells);
         int* qin = h->qa.p;
         int* qout = h->qb.p;
-        int* c_ext = cnt;
+        int* c_ext = cells.paths(0);
         auto finish = [&](bool primary, int nb) {
             stage(PT_STAGE_PLAIN, [&] {
-                ptk::launch_finish(s, fin.blocks, h->sc, op, pb, &bb, primary, inl, h->qa.p, h->qb.p, cnt, nb, fin.leave,
-                                   D, 0, 0, 0, finish_cell(cnt, D), h->spill.p, h->ovf.p, tiles);
+                ptk::launch_finish(s, fin.blocks, h->sc, op, pb, &bb, primary, inl, h->qa.p, h->qb.p, cells.base, nb, fin.leave,
+                                   D, 0, 0, 0, cells.finish(), h->spill.p, h->ovf.p, tiles);
             });
         };
         const int nb = whole ? 0 : fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
         if (whole) finish(true, 0);
         for (int b = 0; b < nb; ++b) {
-            int* c_hit = cnt + (D + 1) + b;
-            int* c_sh = cnt + 2 * (D + 1) + b;
-            int* wk = cnt + 3 * (D + 1) + 3 * b;
+            int* c_hit = cells.hits(b);
+            int* c_sh = cells.shadows(b);
             const bool primary = b == 0;
             const bool compact = primary || (b % cadence) == 0;
-            int* c_next = compact ? cnt + b + 1 : c_ext;
-            int* c_cont = cont_cells(cnt, D, b);
+            int* c_next = compact ? cells.paths(b + 1) : c_ext;
             stage(PT_STAGE_EXTEND, [&] {
                 if (primary) {
-                    ptk::launch_extend_batch(s, b_ext, bs, h->sc, op, pb, bb, h->hq.p, c_hit, wk, S, h->spill.p, h->ovf.p,
+                    ptk::launch_extend_batch(s, b_ext, bs, h->sc, op, pb, bb, h->hq.p, c_hit, cells.work(b, 0), S, h->spill.p, h->ovf.p,
                                              tiles);
                 } else {
-                    ptk::launch_extend(s, b_ext, bs, h->sc, op, pb, false, qin, c_ext, 0, 0, 0, h->hq.p, c_hit, wk, S,
-                                       h->spill.p, h->work_counts.p, h->ovf.p, false, cap, &cb, c_cont, fin.leave);
+                    ptk::launch_extend(s, b_ext, bs, h->sc, op, pb, false, qin, c_ext, 0, 0, 0, h->hq.p, c_hit, cells.work(b, 0), S,
+                                       h->spill.p, h->work_counts.p, h->ovf.p, false, cap, &cb, cells.conts(b), fin.leave);
                     if (cap > 0)
-                        ptk::launch_extend_resume(s, b_ext, bs, h->sc, op, pb, cb, c_cont, h->hq.p, c_cont + 1,
+                        ptk::launch_extend_resume(s, b_ext, bs, h->sc, op, pb, cb, cells.conts(b), h->hq.p, cells.work(b, 3),
                                                   S, h->spill.p, h->ovf.p);
                 }
             });
             stage(PT_STAGE_SHADE, [&] {
                 ptk::launch_shade(s, b_sha, bs, h->sc, op, pb, sb, &bb, primary, inl, h->hq.p, c_hit, 0, 0, qout,
-                                  c_next, c_sh, wk + 1, compact, S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
+                                  c_next, c_sh, cells.work(b, 1), compact, S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
             });
             if (!inl)
                 stage(PT_STAGE_SHADOW, [&] {
-                    ptk::launch_shadow(s, b_sdw, bs, h->sc, op, pb, sb, c_sh, wk + 2, S, h->spill.p,
+                    ptk::launch_shadow(s, b_sdw, bs, h->sc, op, pb, sb, c_sh, cells.work(b, 2), S, h->spill.p,
                                        h->work_counts.p + 8, h->ovf.p, false);
                 });
             if (compact) {
@@ -914,7 +921,7 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
     const DevOpts op = h->dev_opts();
     const int W = op.width, H = op.height;
     const int items = ((W + 7) / 8) * ((H + 7) / 8) * 64;
-    h->counters.ensure(std::max<size_t>(h->counters.n, 8));
+    h->counters.ensure(ptd::SHARDS * ptd::CELL);
     h->ensure_misc();
     const int bs = h->block_size(), S = h->stack_S();
     const bool cw = h->opts.count_work != 0;
@@ -923,7 +930,7 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
     const int2* tiles = tile_entries(h, op, nullptr, 0, items / 64, std::max(W, H), static_cast<long long>(items) * num_samples);
     for (int smp = first_sample; smp < first_sample + num_samples; ++smp) {
         hipEvent_t ev;
-        ptk::launch_fill(h->stream, h->counters.p, 1, 0);
+        ptk::launch_zero_cells(h->stream, h->counters.p, ptd::SHARDS);
         h->stage_begin(PT_STAGE_PLAIN, ev);
         ptk::launch_plain(h->stream, blocks, bs, h->sc, op, h->accum.p, smp, items, h->counters.p, S, h->spill.p,
                           h->work_counts.p, h->ovf.p, cw, tiles);
