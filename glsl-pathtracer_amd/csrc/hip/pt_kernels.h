@@ -109,14 +109,14 @@ struct BatchBuf {
 namespace ptk {
 enum { KIND_PLAIN = 0, KIND_EXTEND = 1, KIND_SHADE = 2, KIND_SHADOW = 3, KIND_SHADE_BATCH = 4,
        KIND_SHADE_INLINE = 5, KIND_SHADE_BATCH_INLINE = 6, KIND_REPLAY = 7, KIND_PLAIN_BATCH = 8,
-       KIND_FINISH = 9, KIND_FINISH_INLINE = 10 };
+       KIND_FINISH = 9, KIND_FINISH_INLINE = 10, KIND_PLAIN_INLINE = 11, KIND_PLAIN_BATCH_INLINE = 12 };
 
 // Resident blocks for a persistent launch (occupancy x CUs); extra_lds is the
 // replay stage's per-block gradient table.
 int persistent_blocks(int kind, int bs, int S, bool count, int num_cu, size_t extra_lds = 0);
 void launch_plain(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op, float4* accum,
                   int sample, int num_items, int* work, int S, int* spill, unsigned long long* counters, int* ovf,
-                  bool count, const int2* tiles);
+                  bool count, bool inline_nee, const int2* tiles);
 // Entries of the camera rays of every 8x8 tile (jobs: of every job, in item
 // order), read by the launches that take `tiles` (null: whole scene).
 void launch_tiles(hipStream_t s, const ptd::DevScene& sc, const ptd::DevOpts& op, const ptd::JobDev* jobs, int njobs,
@@ -175,7 +175,7 @@ void launch_accum_batch(hipStream_t s, int blocks, const ptd::PathBuf& pb, const
 // item0, `items` = the sum of their npix).
 void launch_plain_batch(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op,
                         const ptd::JobDev* jobs, int njobs, int items, float4* accum, int* work, int S, int* spill,
-                        int* ovf, const int2* tiles);
+                        int* ovf, bool inline_nee, const int2* tiles);
 // Environment-map CDF and total luminance of an RGB32F image of n texels
 // (ok: one int of scratch; scratch: env_cdf_scratch_bytes(n) bytes, 8-byte aligned).
 // The parallel scan works in chunks of ENV_CDF_CHUNK texels (texels 1..n-1)

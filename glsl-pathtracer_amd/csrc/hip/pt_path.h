@@ -622,11 +622,11 @@ __device__ __forceinline__ Entry tile_entry(const DevScene& sc, const DevOpts& o
 // bounce (the visible NEE contributions are added after the vertex's emission
 // and only when one is visible, as the shadow stage does). `seen(b, mask)` is
 // called for the visible NEE rays of bounce b (not with INLINE_NEE).
-template <bool INLINE_NEE, class Seen>
+template <bool INLINE_NEE, bool PLAIN, class Seen>
 __device__ __forceinline__ void finish_path(const DevScene& sc, const DevOpts& op, PathRegs& p, int b, int D,
                                             Stack& stk, bool& ovf, Entry en, Seen&& seen) {
     TravCount cnt{0, 0, 0, 0, 0, 0};
-    for (; b < D; ++b) {
+    for (; PLAIN || b < D; ++b) {
         const Hit h = closest<false>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
         en = whole_scene(sc);
         if (h.t == INF) { on_miss(sc, op, p); return; }
@@ -656,7 +656,7 @@ __device__ __forceinline__ void finish_path(const DevScene& sc, const DevOpts& o
                     Ld = Ld + r.contrib;
                     lit |= 1 << kind;
                 }
-                if (lit) {
+                if (PLAIN || lit) {
                     p.rad = p.rad + Ld * p.thr;
                     seen(b, lit);
                 }

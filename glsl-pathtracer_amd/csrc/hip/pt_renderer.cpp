@@ -759,14 +759,16 @@ void batch_render_plain(pt_renderer_s* h, const pt_job* jobs, int n) {
     h->counters.ensure(ptd::SHARDS * ptd::CELL);
     h->ensure_misc();
     const int bs = h->block_size(), S = h->stack_S();
-    const int blocks = ptk::persistent_blocks(ptk::KIND_PLAIN_BATCH, bs, S, false, h->num_cu);
+    const bool inl = needs_inline_nee(h, op);
+    const int blocks =
+        ptk::persistent_blocks(inl ? ptk::KIND_PLAIN_BATCH_INLINE : ptk::KIND_PLAIN_BATCH, bs, S, false, h->num_cu);
     h->ensure_spill(static_cast<size_t>(blocks) * bs);
     ptk::launch_zero_cells(s, h->counters.p, ptd::SHARDS);
     const int2* tiles = tile_entries(h, op, h->b_jobs.p, n, static_cast<int>(P.items / 64), P.max_side, P.samples);
     hipEvent_t ev;
     h->stage_begin(PT_STAGE_BATCH, ev);
     ptk::launch_plain_batch(s, blocks, bs, h->sc, op, h->b_jobs.p, n, static_cast<int>(P.items), h->b_accum.p,
-                            h->counters.p, S, h->spill.p, h->ovf.p, tiles);
+                            h->counters.p, S, h->spill.p, h->ovf.p, inl, tiles);
     h->stage_end(PT_STAGE_BATCH, ev);
     HIPCHK(hipGetLastError());
     for (int j = 0; j < n; ++j) {
@@ -925,7 +927,9 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
     h->ensure_misc();
     const int bs = h->block_size(), S = h->stack_S();
     const bool cw = h->opts.count_work != 0;
-    const int blocks = ptk::persistent_blocks(ptk::KIND_PLAIN, bs, S, cw, h->num_cu);
+    const bool inl = needs_inline_nee(h, op);
+    const int blocks =
+        ptk::persistent_blocks(inl && !cw ? ptk::KIND_PLAIN_INLINE : ptk::KIND_PLAIN, bs, S, cw, h->num_cu);
     h->ensure_spill(static_cast<size_t>(blocks) * bs);
     const int2* tiles = tile_entries(h, op, nullptr, 0, items / 64, std::max(W, H), static_cast<long long>(items) * num_samples);
     for (int smp = first_sample; smp < first_sample + num_samples; ++smp) {
@@ -933,7 +937,7 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
         ptk::launch_zero_cells(h->stream, h->counters.p, ptd::SHARDS);
         h->stage_begin(PT_STAGE_PLAIN, ev);
         ptk::launch_plain(h->stream, blocks, bs, h->sc, op, h->accum.p, smp, items, h->counters.p, S, h->spill.p,
-                          h->work_counts.p, h->ovf.p, cw, tiles);
+                          h->work_counts.p, h->ovf.p, cw, inl, tiles);
         h->stage_end(PT_STAGE_PLAIN, ev);
         HIPCHK(hipGetLastError());
     }
