@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(256) k_plain(DevScene sc, DevOpts op, float4* 
         }
     }
     flush_counts<COUNT>(cnt, counters);
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // ------------------------------------------------------------------ wavefront
@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
     if (CAPPED)
         for (int i = conts.at + lane_id(); i < min(conts.end, cb.cap); i += 64) cb.slot[i] = -1;
     flush_counts<COUNT>(cnt, counters);
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // The traversals a capped extend stage stopped, packed densely: each record's
@@ -501,7 +501,7 @@ k_extend_resume(DevScene sc, DevOpts op, PathBuf pb, ContBuf cb, const int* cont
             hitq[hi.w] = keep ? slot : -1;
         }
     }
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // Shade: one bounce of every path that hit something. The NEE rays of the
@@ -616,7 +616,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene sc, DevOpts op0, PathBuf
     for (int i = paths.at + lane_id(); i < paths.end; i += 64) qout[i] = -1;
     if (INLINE_NEE) {
         flush_counts<false>(cnt, counters);
-        if (ovf) atomicOr(ovf_flag, 1);
+        if (ovf) *ovf_flag = 1;
     }
 }
 
@@ -659,7 +659,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
         }
     }
     flush_counts<COUNT>(cnt, counters);
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // The rest of a pass's paths in one launch, once few are left (or, PRIMARY,
@@ -744,7 +744,7 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
         if (l == 0) next = atomicAdd(work, per);
         base = __builtin_amdgcn_readfirstlane(next) + nw * per;
     }
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // Replay stage of the path-replay adjoint: one bounce of every path that hit
@@ -890,7 +890,7 @@ k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items
             accum[Jp->accum_off + static_cast<long long>(py) * width + px] = acc;
         }
     }
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // Accumulate: accum[pixel] += radiance of samples s = 0..nsamp-1 in order.
@@ -1434,7 +1434,7 @@ __global__ void __launch_bounds__(256) k_query_closest(DevScene sc, DevOpts op, 
     light[i] = h.light;
     uv[2 * i] = h.tri >= 0 ? h.u : 0.f;
     uv[2 * i + 1] = h.tri >= 0 ? h.v : 0.f;
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 __global__ void __launch_bounds__(256) k_query_any(DevScene sc, DevOpts op, const float* __restrict__ orig,
@@ -1449,7 +1449,7 @@ __global__ void __launch_bounds__(256) k_query_any(DevScene sc, DevOpts op, cons
     vec3 o = V(orig[3 * i], orig[3 * i + 1], orig[3 * i + 2]);
     vec3 d = V(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]);
     occ[i] = occluded<false, true>(sc, op, o, d, maxd[i], stk, cnt, ovf) ? 1 : 0;
-    if (ovf) atomicOr(ovf_flag, 1);
+    if (ovf) *ovf_flag = 1;
 }
 
 // ------------------------------------------------------------------ tonemap (tonemap.glsl:59-133)
