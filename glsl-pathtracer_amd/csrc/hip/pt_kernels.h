@@ -78,6 +78,20 @@ struct ReplayBuf {
     int lds;              // 1: accumulate per block in LDS (grad, then mgrad)
 };
 
+// What the adjoint's primal pass leaves for its replay: the closest hits of
+// bounces 0..bounces-1 (hit and hit2 by slot, q the slots in any order, rows of
+// `row` and `qrow` entries per bounce; counts[b * CELL] of them) and the
+// visibility words (arrays of `row` words).
+struct Record {
+    float4* hit;
+    int2* hit2;
+    int* q;
+    int* counts;
+    size_t row, qrow;
+    int bounces;
+    unsigned* vis;
+};
+
 // ---- batched render of many jobs (one scene, own camera / size / depth each)
 // One job of a batch.
 struct JobDev {
@@ -138,12 +152,12 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const ptd::DevScene
 // Every path left after the stages of bounces [0, nb), run to its end (primary:
 // every path of the pass from its camera ray): the queue of the first bounce
 // whose entry count cells[b] is at most `limit`, or of bounce nb. qa, qb: the
-// queues of even and odd bounces; D: bounces of the pass in all; vis: the
-// adjoint's visibility words (arrays of vis_stride words), else null.
+// queues of even and odd bounces; D: bounces of the pass in all; rec: the
+// adjoint's record (one frame, inline_nee off), else null.
 void launch_finish(hipStream_t s, int blocks, const ptd::DevScene& sc, const ptd::DevOpts& op,
                    const ptd::PathBuf& pb, const ptd::BatchBuf* bb, bool primary, bool inline_nee, const int* qa,
                    const int* qb, const int* cells, int nb, int limit, int D, int npaths, int npix, int first_sample,
-                   int* work, int* spill, int* ovf, const int2* tiles, unsigned* vis = nullptr, int vis_stride = 0);
+                   int* work, int* spill, int* ovf, const int2* tiles, const ptd::Record* rec = nullptr);
 // Shade stage; bb: the batched form's pass state (null: one frame); inline_nee:
 // NEE visibility resolved in the stage (stochastic alpha, volume MIS), else
 // queued as shadow records. S and spill: the traversal stack (inline_nee).

@@ -233,7 +233,7 @@ template <bool COUNT, bool INLINE_NEE>
 __device__ __forceinline__ float4 plain_sample(const DevScene& sc, const DevOpts& op, PathRegs& p, Stack& stk,
                                                TravCount& cnt, bool& ovf, Entry en) {
     if (COUNT || INLINE_NEE) return path_trace<COUNT>(sc, op, p, stk, cnt, ovf, en);
-    finish_path<false, true>(sc, op, p, 0, 0, stk, ovf, en, [](int, int) {});
+    finish_path<false, true>(sc, op, p, 0, 0, stk, ovf, en, [](int, const Hit&) {}, [](int, int) {});
     return make_float4(p.rad.x, p.rad.y, p.rad.z, p.alpha);
 }
 
@@ -328,6 +328,11 @@ __device__ __forceinline__ void batch_decode(const BatchBuf& bb, int slot, int& 
     item = slot - pl.slot0;
 }
 
+__device__ __forceinline__ void store_hit(float4* hit, int2* hit2, int slot, const Hit& h) {
+    hit[slot] = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
+    hit2[slot] = make_int2(h.inst, h.light);
+}
+
 // End of a path's closest-hit step: a miss finishes the path here (environment
 // or uniform light), a hit is recorded for the shade stage (returns true).
 template <bool PRIMARY>
@@ -344,8 +349,7 @@ __device__ __forceinline__ bool finish_extend(const DevScene& sc, const DevOpts&
         if (!PRIMARY) pb.meta[slot].y = PATH_DEAD;
         return false;
     }
-    pb.hit[slot] = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
-    pb.hit2[slot] = make_int2(h.inst, h.light);
+    store_hit(pb.hit, pb.hit2, slot, h);
     return true;
 }
 
@@ -680,12 +684,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
 // has the room), so deep traversals do not go to the backing store.
 // The queue is that of the first bounce b in [1, nb] which the stages left
 // (count in cells[b] at most `limit`) or, at b == nb, could not start.
-// vis: visibility words as in k_shadow (array w at vis + w * vis_stride).
-template <bool PRIMARY, bool BATCH, bool INLINE_NEE>
+// RECORD: the paths' hits and visible NEE rays go to `rec`. All lanes of a wave
+// are at the same bounce (they began at one), so a wave appends its hits of a
+// bounce with one atomic.
+template <bool PRIMARY, bool BATCH, bool INLINE_NEE, bool RECORD>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, const int* cells, int nb, int limit,
          int D, int npaths, int npix, int first_sample, int* work, BatchBuf bb, int* spill, int* ovf_flag,
-         unsigned* vis, int vis_stride, const int2* __restrict__ tiles) {
+         Record rec, const int2* __restrict__ tiles) {
     extern __shared__ int lds[];
     int b = 0, count = 0;
     if (PRIMARY) {
@@ -732,11 +738,24 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
             }
             if (!PRIMARY) load_path(pb, slot, p);
             if (valid) {
-                finish_path<INLINE_NEE, false>(sc, op, p, b, D, stk, ovf, en, [&](int bounce, int lit) {
-                    if (vis)
-                        vis[static_cast<size_t>(bounce / VIS_BOUNCES_PER_WORD) * vis_stride + slot] |=
+                finish_path<INLINE_NEE, false>(
+                    sc, op, p, b, D, stk, ovf, en,
+                    [&](int bounce, const Hit& h) {
+                        if (!RECORD) return;
+                        const int at = __builtin_amdgcn_readfirstlane(bounce);
+                        if (at >= rec.bounces) return;
+                        const unsigned long long hits = __ballot(1);
+                        int first = 0;
+                        if (l == __ffsll(hits) - 1) first = atomicAdd(rec.counts + at * CELL, __popcll(hits));
+                        first = __builtin_amdgcn_readfirstlane(first);  // of the lane that added, the first one
+                        rec.q[at * rec.qrow + first + __popcll(hits & ((1ull << l) - 1))] = slot;
+                        store_hit(rec.hit + at * rec.row, rec.hit2 + at * rec.row, slot, h);
+                    },
+                    [&](int bounce, int lit) {
+                        if (!RECORD) return;
+                        rec.vis[static_cast<size_t>(bounce / VIS_BOUNCES_PER_WORD) * rec.row + slot] |=
                             static_cast<unsigned>(lit) << (2 * (bounce % VIS_BOUNCES_PER_WORD));
-                });
+                    });
                 pb.rad[slot] = F4(p.rad, p.alpha);
             }
         }
@@ -1533,8 +1552,8 @@ int persistent_blocks(int kind, int bs, int S, bool count, int num_cu, size_t ex
         case KIND_SHADE_BATCH: per_cu = max_blocks(k_shade<false, true, false>, bs, 0); break;
         case KIND_SHADE_INLINE: per_cu = max_blocks(k_shade<false, false, true>, bs, lds); break;
         case KIND_SHADE_BATCH_INLINE: per_cu = max_blocks(k_shade<false, true, true>, bs, lds); break;
-        case KIND_FINISH: per_cu = max_blocks(k_finish<false, false, false>, 64, FINISH_S * 64 * sizeof(int)); break;
-        case KIND_FINISH_INLINE: per_cu = max_blocks(k_finish<false, false, true>, 64, FINISH_S * 64 * sizeof(int)); break;
+        case KIND_FINISH: per_cu = max_blocks(k_finish<false, false, false, false>, 64, FINISH_S * 64 * sizeof(int)); break;
+        case KIND_FINISH_INLINE: per_cu = max_blocks(k_finish<false, false, true, false>, 64, FINISH_S * 64 * sizeof(int)); break;
         case KIND_REPLAY: per_cu = max_blocks(k_replay_shade<false>, bs, extra_lds); break;
         default: break;
     }
@@ -1584,16 +1603,19 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const DevScene& sc,
 void launch_finish(hipStream_t s, int blocks, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
                    const BatchBuf* bb, bool primary, bool inline_nee, const int* qa, const int* qb, const int* cells,
                    int nb, int limit, int D, int npaths, int npix, int first_sample, int* work, int* spill, int* ovf,
-                   const int2* tiles, unsigned* vis, int vis_stride) {
+                   const int2* tiles, const Record* rec) {
     const BatchBuf b = bb ? *bb : BatchBuf{};
+    const Record r = rec ? *rec : Record{};
     const size_t lds = FINISH_S * 64 * sizeof(int);
-#define PT_FIN(P, B, I) hipLaunchKernelGGL((k_finish<P, B, I>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, vis, vis_stride, tiles)
+#define PT_FIN(P, B, I, R) hipLaunchKernelGGL((k_finish<P, B, I, R>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, r, tiles)
     if (bb) {
-        if (inline_nee) { if (primary) PT_FIN(true, true, true); else PT_FIN(false, true, true); }
-        else { if (primary) PT_FIN(true, true, false); else PT_FIN(false, true, false); }
+        if (inline_nee) { if (primary) PT_FIN(true, true, true, false); else PT_FIN(false, true, true, false); }
+        else { if (primary) PT_FIN(true, true, false, false); else PT_FIN(false, true, false, false); }
+    } else if (rec) {
+        if (primary) PT_FIN(true, false, false, true); else PT_FIN(false, false, false, true);
     } else {
-        if (inline_nee) { if (primary) PT_FIN(true, false, true); else PT_FIN(false, false, true); }
-        else { if (primary) PT_FIN(true, false, false); else PT_FIN(false, false, false); }
+        if (inline_nee) { if (primary) PT_FIN(true, false, true, false); else PT_FIN(false, false, true, false); }
+        else { if (primary) PT_FIN(true, false, false, false); else PT_FIN(false, false, false, false); }
     }
 #undef PT_FIN
 }

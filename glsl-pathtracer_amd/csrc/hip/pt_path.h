@@ -620,16 +620,18 @@ __device__ __forceinline__ Entry tile_entry(const DevScene& sc, const DevOpts& o
 // The rest of a path of the wavefront form, bounces b..D-1, in one go: the
 // same decisions, random draws and sums as the stage kernels make bounce by
 // bounce (the visible NEE contributions are added after the vertex's emission
-// and only when one is visible, as the shadow stage does). `seen(b, mask)` is
-// called for the visible NEE rays of bounce b (not with INLINE_NEE).
-template <bool INLINE_NEE, bool PLAIN, class Seen>
+// and only when one is visible, as the shadow stage does). `found(b, h)` is
+// called for the closest hit of bounce b, `seen(b, mask)` for its visible NEE
+// rays (not with INLINE_NEE).
+template <bool INLINE_NEE, bool PLAIN, class Found, class Seen>
 __device__ __forceinline__ void finish_path(const DevScene& sc, const DevOpts& op, PathRegs& p, int b, int D,
-                                            Stack& stk, bool& ovf, Entry en, Seen&& seen) {
+                                            Stack& stk, bool& ovf, Entry en, Found&& found, Seen&& seen) {
     TravCount cnt{0, 0, 0, 0, 0, 0};
     for (; PLAIN || b < D; ++b) {
         const Hit h = closest<false>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
         en = whole_scene(sc);
         if (h.t == INF) { on_miss(sc, op, p); return; }
+        found(b, h);
         SurfState st;
         init_surf(st);
         Material m;
