@@ -129,8 +129,8 @@ enum { KIND_PLAIN = 0, KIND_EXTEND = 1, KIND_SHADE = 2, KIND_SHADOW = 3, KIND_SH
 // replay stage's per-block gradient table.
 int persistent_blocks(int kind, int bs, int S, bool count, int num_cu, size_t extra_lds = 0);
 void launch_plain(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op, float4* accum,
-                  int sample, int num_items, int* work, int S, int* spill, unsigned long long* counters, int* ovf,
-                  bool count, bool inline_nee, const int2* tiles);
+                  int sample, int spp, int refill, int num_items, int* work, int S, int* spill,
+                  unsigned long long* counters, int* ovf, bool count, bool inline_nee, const int2* tiles);
 // Entries of the camera rays of every 8x8 tile (jobs: of every job, in item
 // order), read by the launches that take `tiles` (null: whole scene).
 void launch_tiles(hipStream_t s, const ptd::DevScene& sc, const ptd::DevOpts& op, const ptd::JobDev* jobs, int njobs,
@@ -157,7 +157,7 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const ptd::DevScene
 void launch_finish(hipStream_t s, int blocks, const ptd::DevScene& sc, const ptd::DevOpts& op,
                    const ptd::PathBuf& pb, const ptd::BatchBuf* bb, bool primary, bool inline_nee, const int* qa,
                    const int* qb, const int* cells, int nb, int limit, int D, int npaths, int npix, int first_sample,
-                   int* work, int* spill, int* ovf, const int2* tiles, const ptd::Record* rec = nullptr);
+                   int* work, int* spill, int* ovf, const int2* tiles, int refill, const ptd::Record* rec = nullptr);
 // Shade stage; bb: the batched form's pass state (null: one frame); inline_nee:
 // NEE visibility resolved in the stage (stochastic alpha, volume MIS), else
 // queued as shadow records. S and spill: the traversal stack (inline_nee).
@@ -188,8 +188,8 @@ void launch_accum_batch(hipStream_t s, int blocks, const ptd::PathBuf& pb, const
 // Batched render in one persistent launch of the plain form (jobs sorted by
 // item0, `items` = the sum of their npix).
 void launch_plain_batch(hipStream_t s, int blocks, int bs, const ptd::DevScene& sc, const ptd::DevOpts& op,
-                        const ptd::JobDev* jobs, int njobs, int items, float4* accum, int* work, int S, int* spill,
-                        int* ovf, bool inline_nee, const int2* tiles);
+                        const ptd::JobDev* jobs, int njobs, int items, int refill, float4* accum, int* work, int S,
+                        int* spill, int* ovf, bool inline_nee, const int2* tiles);
 // Environment-map CDF and total luminance of an RGB32F image of n texels
 // (ok: one int of scratch; scratch: env_cdf_scratch_bytes(n) bytes, 8-byte aligned).
 // The parallel scan works in chunks of ENV_CDF_CHUNK texels (texels 1..n-1)

@@ -224,22 +224,46 @@ __device__ __forceinline__ bool blank(const DevOpts& op, Entry en) {
 }
 
 // ------------------------------------------------------------------ plain kernel
-// One sample of a pixel, the path kept in registers. INLINE_NEE as in k_shade:
-// without it (no stochastic alpha, no volume MIS) the any-hit queries need not
-// keep the reference's visit order and the transmittance code is not in the
-// kernel (1024x1024, four samples: Cornell box 6.99 -> 6.56 ms, spheres 3.88 ->
-// 3.67, boxes 10.2 -> 9.8; batch of 16 Cornell jobs 13.5 -> 12.9).
-template <bool COUNT, bool INLINE_NEE>
-__device__ __forceinline__ float4 plain_sample(const DevScene& sc, const DevOpts& op, PathRegs& p, Stack& stk,
-                                               TravCount& cnt, bool& ovf, Entry en) {
-    if (COUNT || INLINE_NEE) return path_trace<COUNT>(sc, op, p, stk, cnt, ovf, en);
-    finish_path<false, true>(sc, op, p, 0, 0, stk, ovf, en, [](int, const Hit&) {}, [](int, int) {});
-    return make_float4(p.rad.x, p.rad.y, p.rad.z, p.alpha);
+// A pixel's samples 0..spp-1 added to acc in order, the path kept in registers;
+// begin(sample, path) sets up a camera ray, `first` is its entry. INLINE_NEE as in
+// k_shade: without it (no stochastic alpha, no volume MIS) the any-hit queries
+// need not keep the reference's visit order and the transmittance code is not in
+// the kernel (1024x1024, four samples: Cornell box 6.99 -> 6.56 ms, spheres 3.88
+// -> 3.67, boxes 10.2 -> 9.8; batch of 16 Cornell jobs 13.5 -> 12.9).
+// A lane whose path has ended waits until `refill` lanes of its wave do (64: all),
+// then they begin their next samples while the others go on. In scenes of few
+// triangles that fills the wave: three batches of 4 and 16 Cornell jobs 12.9 ->
+// 12.8 ms, 6.3 -> 5.4, 7.9 -> 6.7 at 8 lanes (2 lanes: 14.5, 5.9; 32: 13.1, 5.6),
+// as setting up rays for a few lanes costs the wave as much as for all. In larger
+// scenes the camera rays' short, alike traversals then wait for those of later
+// bounces; refill_lanes() has the rule.
+template <bool INLINE_NEE, class Begin>
+__device__ __forceinline__ void pixel_samples(const DevScene& sc, const DevOpts& op, Stack& stk, bool& ovf, Entry first,
+                                              int spp, int refill, float4& acc, Begin&& begin) {
+    PathRegs p;
+    bool alive = false, fresh = false;
+    for (int smp = 0;;) {
+        const unsigned long long live = __ballot(alive), wait = __ballot(!alive && smp < spp);
+        if (!(live | wait)) break;
+        if (!alive && smp < spp && (!live || __popcll(wait) >= refill)) {
+            begin(smp, p);
+            alive = fresh = true;
+        }
+        if (alive) {
+            const Entry en = fresh ? first : whole_scene(sc);
+            alive = path_bounce<INLINE_NEE, true>(sc, op, p, 0, stk, ovf, en, [](int, const Hit&) {}, [](int, int) {});
+            fresh = false;
+            if (!alive) {
+                acc.x += p.rad.x; acc.y += p.rad.y; acc.z += p.rad.z; acc.w += p.alpha;
+                ++smp;
+            }
+        }
+    }
 }
 
 template <bool COUNT, bool INLINE_NEE>
 __global__ void __launch_bounds__(256) k_plain(DevScene sc, DevOpts op, float4* __restrict__ accum, int sample,
-                                               int num_items, int* work, int S, int* spill,
+                                               int spp, int refill, int num_items, int* work, int S, int* spill,
                                                unsigned long long* counters, int* ovf_flag,
                                                const int2* __restrict__ tiles) {
     extern __shared__ int lds[];
@@ -252,13 +276,23 @@ __global__ void __launch_bounds__(256) k_plain(DevScene sc, DevOpts op, float4* 
         int px, py;
         item_pixel(i, op.width, px, py);
         if (i < num_items && px < op.width && py < op.height) {
-            PathRegs p;
-            if (blank(op, en)) init_path(p);
-            else primary_path(op, px, py, sample, p);
-            float4 c = plain_sample<COUNT, INLINE_NEE>(sc, op, p, stk, cnt, ovf, en);
+            const bool empty = blank(op, en);
             float4* a = accum + static_cast<size_t>(py) * op.width + px;
             float4 acc = *a;
-            acc.x += c.x; acc.y += c.y; acc.z += c.z; acc.w += c.w;
+            auto begin = [&](int k, PathRegs& p) {
+                if (empty) init_path(p);
+                else primary_path(op, px, py, sample + k, p);
+            };
+            if (COUNT) {
+                for (int k = 0; k < spp; ++k) {
+                    PathRegs p;
+                    begin(k, p);
+                    const float4 c = path_trace<COUNT>(sc, op, p, stk, cnt, ovf, en);
+                    acc.x += c.x; acc.y += c.y; acc.z += c.z; acc.w += c.w;
+                }
+            } else {
+                pixel_samples<INLINE_NEE>(sc, op, stk, ovf, en, spp, refill, acc, begin);
+            }
             *a = acc;
         }
     }
@@ -668,7 +702,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
 
 // The rest of a pass's paths in one launch, once few are left (or, PRIMARY,
 // every path of a small pass from its camera ray on): each lane runs its path
-// to the end in registers (finish_path) and writes its radiance. What the
+// to the end in registers and writes its radiance. What the
 // stages buy is full waves of paths at the same step; they pay with a launch
 // per stage and, per launch, the wait for its slowest ray. Once the paths left
 // fit the chip at once there is nothing to buy: a bounce's stage launches last
@@ -684,14 +718,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
 // has the room), so deep traversals do not go to the backing store.
 // The queue is that of the first bounce b in [1, nb] which the stages left
 // (count in cells[b] at most `limit`) or, at b == nb, could not start.
-// RECORD: the paths' hits and visible NEE rays go to `rec`. All lanes of a wave
-// are at the same bounce (they began at one), so a wave appends its hits of a
-// bounce with one atomic.
+// RECORD: the paths' hits and visible NEE rays go to `rec`.
+// A lane whose path has ended waits until `refill` lanes of its wave do (64: all)
+// and they take the next paths, as in pixel_samples: two samples of a 1024x800
+// Cornell box 3.25 -> 2.39 ms (at 16 lanes 2.44, 32: 2.64), but 1280x720 spheres
+// 0.94 -> 1.07. A wave takes its next paths up to 64 at a time, fewer towards the
+// end of the work (640x360 boxes 1.57 -> 1.42 ms), but with INLINE_NEE, where
+// the vertices' work keeps the SIMDs busy, never fewer (1001x563x2 volume MIS 2.26
+// ms against 2.37).
 template <bool PRIMARY, bool BATCH, bool INLINE_NEE, bool RECORD>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, const int* cells, int nb, int limit,
          int D, int npaths, int npix, int first_sample, int* work, BatchBuf bb, int* spill, int* ovf_flag,
-         Record rec, const int2* __restrict__ tiles) {
+         Record rec, const int2* __restrict__ tiles, int refill) {
     extern __shared__ int lds[];
     int b = 0, count = 0;
     if (PRIMARY) {
@@ -703,65 +742,97 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
         }
     }
     const int* q = (b & 1) ? qb : qa;
-    const int nw = static_cast<int>(gridDim.x);
+    const int first_bounce = b, nw = static_cast<int>(gridDim.x), l = lane_id();
     const int per = min(64, (count + nw - 1) / nw);
     Stack stk = wave_stack(lds, spill, FINISH_S);
-    bool ovf = false;
-    for (int base = static_cast<int>(blockIdx.x) * per; base < count;) {
-        const int l = lane_id(), i = base + l;
-        const int slot = l < per && i < count ? (PRIMARY ? i : q[i]) : -1;  // -1: empty place too
-        if (slot >= 0) {
-            PathRegs p;
-            DevOpts op = op0;
-            Entry en = whole_scene(sc);
-            bool valid = true;
-            if (BATCH) {
-                int job, smp, item;
-                batch_decode(bb, slot, job, smp, item);
-                const JobDev* J = bb.jobs + job;
-                if (PRIMARY) {
-                    const DevOpts oj = job_opts(op0, *J);
-                    int px, py;
-                    item_pixel(item, oj.width, px, py);
-                    valid = px < oj.width && py < oj.height;
-                    if (tiles) en = lane_entry(tiles, (J->item0 + item) >> 6);
-                    if (blank(op0, en)) init_path(p);
-                    else if (valid) primary_path(oj, px, py, smp, p);
-                }
-                op.max_depth = J->max_depth;
-            } else if (PRIMARY) {
-                int s, px, py;
-                valid = slot_pixel(op, slot, npix, s, px, py);
-                if (tiles) en = lane_entry(tiles, (slot - s * npix) >> 6);
-                if (blank(op, en)) init_path(p);
-                else if (valid) primary_path(op, px, py, first_sample + s, p);
+    bool ovf = false, alive = false;
+    int at = static_cast<int>(blockIdx.x) * per, end = min(at + per, count);  // the wave's items
+    bool more = nw * per < count;
+    int slot = -1, max_depth = op0.max_depth;
+    int tile = -1;  // of a camera ray that has an entry
+    PathRegs p;
+    for (;;) {
+        unsigned long long live = __ballot(alive);
+        const int idle = 64 - __popcll(live);
+        if (!live || idle >= refill) {
+            if (at >= end && more) {
+                const int part = INLINE_NEE ? 64 : max(8, min(64, (count - end) / (2 * nw)));
+                int next = 0;
+                if (l == 0) next = atomicAdd(work, part);
+                at = __builtin_amdgcn_readfirstlane(next) + nw * per;
+                end = min(at + part, count);
+                more = at + part < count;
             }
-            if (!PRIMARY) load_path(pb, slot, p);
-            if (valid) {
-                finish_path<INLINE_NEE, false>(
-                    sc, op, p, b, D, stk, ovf, en,
-                    [&](int bounce, const Hit& h) {
-                        if (!RECORD) return;
-                        const int at = __builtin_amdgcn_readfirstlane(bounce);
-                        if (at >= rec.bounces) return;
-                        const unsigned long long hits = __ballot(1);
-                        int first = 0;
-                        if (l == __ffsll(hits) - 1) first = atomicAdd(rec.counts + at * CELL, __popcll(hits));
-                        first = __builtin_amdgcn_readfirstlane(first);  // of the lane that added, the first one
-                        rec.q[at * rec.qrow + first + __popcll(hits & ((1ull << l) - 1))] = slot;
-                        store_hit(rec.hit + at * rec.row, rec.hit2 + at * rec.row, slot, h);
-                    },
-                    [&](int bounce, int lit) {
-                        if (!RECORD) return;
-                        rec.vis[static_cast<size_t>(bounce / VIS_BOUNCES_PER_WORD) * rec.row + slot] |=
-                            static_cast<unsigned>(lit) << (2 * (bounce % VIS_BOUNCES_PER_WORD));
-                    });
-                pb.rad[slot] = F4(p.rad, p.alpha);
+            if (at < end) {
+                const int i = at + __popcll(~live & ((1ull << l) - 1));
+                at += idle;
+                if (!alive && i < end) {
+                    slot = PRIMARY ? i : q[i];  // -1: empty place
+                    alive = slot >= 0 && first_bounce < D;
+                    b = first_bounce;
+                    if (BATCH && alive) {
+                        int job, smp, item;
+                        batch_decode(bb, slot, job, smp, item);
+                        const JobDev* J = bb.jobs + job;
+                        if (PRIMARY) {
+                            const DevOpts oj = job_opts(op0, *J);
+                            int px, py;
+                            item_pixel(item, oj.width, px, py);
+                            alive = px < oj.width && py < oj.height;
+                            if (tiles) tile = (J->item0 + item) >> 6;
+                            if (tiles && blank(op0, lane_entry(tiles, tile))) init_path(p);
+                            else if (alive) primary_path(oj, px, py, smp, p);
+                        }
+                        max_depth = J->max_depth;
+                    } else if (PRIMARY) {
+                        int s, px, py;
+                        alive = slot_pixel(op0, slot, npix, s, px, py);
+                        if (tiles) tile = (slot - s * npix) >> 6;
+                        if (tiles && blank(op0, lane_entry(tiles, tile))) init_path(p);
+                        else if (alive) primary_path(op0, px, py, first_sample + s, p);
+                    }
+                    if (!PRIMARY && alive) load_path(pb, slot, p);
+                }
+            }
+            live = __ballot(alive);
+            if (!live) {
+                if (at >= end && !more) break;
+                continue;
             }
         }
-        int next = 0;
-        if (l == 0) next = atomicAdd(work, per);
-        base = __builtin_amdgcn_readfirstlane(next) + nw * per;
+        if (alive) {
+            DevOpts op = op0;
+            if (BATCH) op.max_depth = max_depth;
+            Entry en = whole_scene(sc);
+            if (PRIMARY && tile >= 0) en = lane_entry(tiles, tile);
+            alive = path_bounce<INLINE_NEE, false>(
+                sc, op, p, b, stk, ovf, en,
+                [&](int bounce, const Hit& h) {
+                    if (!RECORD || bounce >= rec.bounces) return;
+                    int place = 0;
+                    for (bool todo = true; todo;) {  // the lanes' bounces one after another
+                        const int at_b = __builtin_amdgcn_readfirstlane(bounce);
+                        const unsigned long long mine = __ballot(bounce == at_b);
+                        if (bounce == at_b) {
+                            int base = 0;
+                            if (l == __ffsll(mine) - 1) base = atomicAdd(rec.counts + at_b * CELL, __popcll(mine));
+                            base = __builtin_amdgcn_readfirstlane(base);  // of the lane that added, the first one
+                            place = base + __popcll(mine & ((1ull << l) - 1));
+                            todo = false;
+                        }
+                    }
+                    rec.q[bounce * rec.qrow + place] = slot;
+                    store_hit(rec.hit + bounce * rec.row, rec.hit2 + bounce * rec.row, slot, h);
+                },
+                [&](int bounce, int lit) {
+                    if (!RECORD) return;
+                    rec.vis[static_cast<size_t>(bounce / VIS_BOUNCES_PER_WORD) * rec.row + slot] |=
+                        static_cast<unsigned>(lit) << (2 * (bounce % VIS_BOUNCES_PER_WORD));
+                });
+            tile = -1;
+            if (++b >= D) alive = false;
+            if (!alive) pb.rad[slot] = F4(p.rad, p.alpha);
+        }
     }
     if (ovf) *ovf_flag = 1;
 }
@@ -873,8 +944,8 @@ __global__ void __launch_bounds__(256) k_replay_shade(DevScene sc, DevOpts op, P
 // takes 4 registers more than that allows.
 template <bool INLINE_NEE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items, float4* __restrict__ accum,
-              int* work, int S, int* spill, int* ovf_flag, const int2* __restrict__ tiles) {
+k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items, int refill,
+              float4* __restrict__ accum, int* work, int S, int* spill, int* ovf_flag, const int2* __restrict__ tiles) {
     extern __shared__ int lds[];
     Stack stk = wave_stack(lds, spill, S);
     TravCount cnt{0, 0, 0, 0, 0, 0};
@@ -894,18 +965,16 @@ k_plain_batch(DevScene sc, DevOpts op0, const JobDev* jobs, int njobs, int items
         if (item < Jp->npix && px < width && py < height) {
             float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
             const Entry en = wave_entry(sc, tiles, wc.base >> 6);
-            for (int smp = 0; smp < spp; ++smp) {
-                // The camera is read again for each sample, after the previous
-                // trace (jobs is not restrict, so the trace's stores keep the
-                // loads here): only max_depth stays live through the trace.
-                PathRegs p;
-                if (blank(op0, en)) init_path(p);
+            const bool empty = blank(op0, en);
+            DevOpts op = op0;
+            op.max_depth = Jp->max_depth;
+            // The camera is read again for each sample, after the previous trace
+            // (jobs is not restrict, so the trace's stores keep the loads here):
+            // only max_depth stays live through the trace.
+            pixel_samples<INLINE_NEE>(sc, op, stk, ovf, en, spp, refill, acc, [&](int smp, PathRegs& p) {
+                if (empty) init_path(p);
                 else primary_path(job_opts(op0, *Jp), px, py, smp, p);
-                DevOpts op = op0;
-                op.max_depth = Jp->max_depth;
-                const float4 c = plain_sample<false, INLINE_NEE>(sc, op, p, stk, cnt, ovf, en);
-                acc.x += c.x; acc.y += c.y; acc.z += c.z; acc.w += c.w;
-            }
+            });
             accum[Jp->accum_off + static_cast<long long>(py) * width + px] = acc;
         }
     }
@@ -1566,10 +1635,10 @@ void launch_tiles(hipStream_t s, const DevScene& sc, const DevOpts& op, const Jo
 }
 
 void launch_plain(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, float4* accum, int sample,
-                  int num_items, int* work, int S, int* spill, unsigned long long* counters, int* ovf, bool count,
-                  bool inline_nee, const int2* tiles) {
+                  int spp, int refill, int num_items, int* work, int S, int* spill, unsigned long long* counters,
+                  int* ovf, bool count, bool inline_nee, const int2* tiles) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
-#define PT_PLAIN(C, I) hipLaunchKernelGGL((k_plain<C, I>), dim3(blocks), dim3(bs), lds, s, sc, op, accum, sample, num_items, work, S, spill, counters, ovf, tiles)
+#define PT_PLAIN(C, I) hipLaunchKernelGGL((k_plain<C, I>), dim3(blocks), dim3(bs), lds, s, sc, op, accum, sample, spp, refill, num_items, work, S, spill, counters, ovf, tiles)
     if (count) PT_PLAIN(true, true);
     else if (inline_nee) PT_PLAIN(false, true);
     else PT_PLAIN(false, false);
@@ -1603,11 +1672,11 @@ void launch_extend_resume(hipStream_t s, int blocks, int bs, const DevScene& sc,
 void launch_finish(hipStream_t s, int blocks, const DevScene& sc, const DevOpts& op, const PathBuf& pb,
                    const BatchBuf* bb, bool primary, bool inline_nee, const int* qa, const int* qb, const int* cells,
                    int nb, int limit, int D, int npaths, int npix, int first_sample, int* work, int* spill, int* ovf,
-                   const int2* tiles, const Record* rec) {
+                   const int2* tiles, int refill, const Record* rec) {
     const BatchBuf b = bb ? *bb : BatchBuf{};
     const Record r = rec ? *rec : Record{};
     const size_t lds = FINISH_S * 64 * sizeof(int);
-#define PT_FIN(P, B, I, R) hipLaunchKernelGGL((k_finish<P, B, I, R>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, r, tiles)
+#define PT_FIN(P, B, I, R) hipLaunchKernelGGL((k_finish<P, B, I, R>), dim3(blocks), dim3(64), lds, s, sc, op, pb, qa, qb, cells, nb, limit, D, npaths, npix, first_sample, work, b, spill, ovf, r, tiles, refill)
     if (bb) {
         if (inline_nee) { if (primary) PT_FIN(true, true, true, false); else PT_FIN(false, true, true, false); }
         else { if (primary) PT_FIN(true, true, false, false); else PT_FIN(false, true, false, false); }
@@ -1668,13 +1737,13 @@ void launch_accum_batch(hipStream_t s, int blocks, const PathBuf& pb, const Batc
 }
 
 void launch_plain_batch(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const JobDev* jobs,
-                        int njobs, int items, float4* accum, int* work, int S, int* spill, int* ovf,
+                        int njobs, int items, int refill, float4* accum, int* work, int S, int* spill, int* ovf,
                         bool inline_nee, const int2* tiles) {
     const size_t lds = static_cast<size_t>(S) * bs * sizeof(int);
     if (inline_nee)
-        hipLaunchKernelGGL(k_plain_batch<true>, dim3(blocks), dim3(bs), lds, s, sc, op, jobs, njobs, items, accum, work, S, spill, ovf, tiles);
+        hipLaunchKernelGGL(k_plain_batch<true>, dim3(blocks), dim3(bs), lds, s, sc, op, jobs, njobs, items, refill, accum, work, S, spill, ovf, tiles);
     else
-        hipLaunchKernelGGL(k_plain_batch<false>, dim3(blocks), dim3(bs), lds, s, sc, op, jobs, njobs, items, accum, work, S, spill, ovf, tiles);
+        hipLaunchKernelGGL(k_plain_batch<false>, dim3(blocks), dim3(bs), lds, s, sc, op, jobs, njobs, items, refill, accum, work, S, spill, ovf, tiles);
 }
 
 void launch_shadow(hipStream_t s, int blocks, int bs, const DevScene& sc, const DevOpts& op, const PathBuf& pb,

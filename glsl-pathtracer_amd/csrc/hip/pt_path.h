@@ -617,56 +617,52 @@ __device__ __forceinline__ Entry tile_entry(const DevScene& sc, const DevOpts& o
     return en;
 }
 
-// The rest of a path of the wavefront form, bounces b..D-1, in one go: the
-// same decisions, random draws and sums as the stage kernels make bounce by
-// bounce (the visible NEE contributions are added after the vertex's emission
-// and only when one is visible, as the shadow stage does). `found(b, h)` is
-// called for the closest hit of bounce b, `seen(b, mask)` for its visible NEE
-// rays (not with INLINE_NEE).
+// Bounce b of a path kept in registers, from its closest hit to the next ray;
+// false where the path ends. The same decisions, random draws and sums as the
+// stage kernels make (the visible NEE contributions are added after the vertex's
+// emission and only when one is visible, as the shadow stage does; PLAIN: always,
+// as path_trace does). `found(b, h)` is called for the closest hit, `seen(b,
+// mask)` for the visible NEE rays (not with INLINE_NEE).
 template <bool INLINE_NEE, bool PLAIN, class Found, class Seen>
-__device__ __forceinline__ void finish_path(const DevScene& sc, const DevOpts& op, PathRegs& p, int b, int D,
-                                            Stack& stk, bool& ovf, Entry en, Found&& found, Seen&& seen) {
+__device__ __forceinline__ bool path_bounce(const DevScene& sc, const DevOpts& op, PathRegs& p, int b, Stack& stk,
+                                            bool& ovf, Entry en, Found&& found, Seen&& seen) {
     TravCount cnt{0, 0, 0, 0, 0, 0};
-    for (; PLAIN || b < D; ++b) {
-        const Hit h = closest<false>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
-        en = whole_scene(sc);
-        if (h.t == INF) { on_miss(sc, op, p); return; }
-        found(b, h);
-        SurfState st;
-        init_surf(st);
-        Material m;
-        float eta;
-        const int ev = bounce_pre(sc, op, h, p, st, m, eta);
-        if (ev == EV_END) return;
-        if (ev != EV_PASS) {
-            if (INLINE_NEE) {
-                vec3 Ld;
-                if ((op.flags & OPT_MEDIUM) && (op.flags & OPT_VOL_MIS))
-                    Ld = direct_light_volmis<false>(sc, op, p.rd, st, m, eta, p.med, ev == EV_SURFACE, p.rng, stk, cnt,
-                                                    ovf);
-                else
-                    Ld = direct_light<false>(sc, op, p.rd, st, m, eta, p.rng, stk, cnt, ovf);
+    const Hit h = closest<false>(sc, op, p.ro, p.rd, p.depth, stk, cnt, ovf, en);
+    if (h.t == INF) { on_miss(sc, op, p); return false; }
+    found(b, h);
+    SurfState st;
+    init_surf(st);
+    Material m;
+    float eta;
+    const int ev = bounce_pre(sc, op, h, p, st, m, eta);
+    if (ev == EV_END) return false;
+    if (ev != EV_PASS) {
+        if (INLINE_NEE) {
+            vec3 Ld;
+            if ((op.flags & OPT_MEDIUM) && (op.flags & OPT_VOL_MIS))
+                Ld = direct_light_volmis<false>(sc, op, p.rd, st, m, eta, p.med, ev == EV_SURFACE, p.rng, stk, cnt, ovf);
+            else
+                Ld = direct_light<false>(sc, op, p.rd, st, m, eta, p.rng, stk, cnt, ovf);
+            p.rad = p.rad + Ld * p.thr;
+        } else {
+            vec3 Ld = V1(0.0f);
+            int lit = 0;
+            for (int kind = 0; kind < 2; ++kind) {
+                if (kind == 0 && !((op.flags & OPT_ENVMAP) && !(op.flags & OPT_UNIFORM_LIGHT))) continue;
+                if (kind == 1 && !(op.flags & OPT_LIGHTS)) continue;
+                const NeeRay r = nee_setup(sc, op, kind, p.rd, st, m, eta, p.rng);
+                if (!r.valid || occluded<false, true>(sc, op, r.o, r.d, r.maxd, stk, cnt, ovf)) continue;
+                Ld = Ld + r.contrib;
+                lit |= 1 << kind;
+            }
+            if (PLAIN || lit) {
                 p.rad = p.rad + Ld * p.thr;
-            } else {
-                vec3 Ld = V1(0.0f);
-                int lit = 0;
-                for (int kind = 0; kind < 2; ++kind) {
-                    if (kind == 0 && !((op.flags & OPT_ENVMAP) && !(op.flags & OPT_UNIFORM_LIGHT))) continue;
-                    if (kind == 1 && !(op.flags & OPT_LIGHTS)) continue;
-                    const NeeRay r = nee_setup(sc, op, kind, p.rd, st, m, eta, p.rng);
-                    if (!r.valid || occluded<false, true>(sc, op, r.o, r.d, r.maxd, stk, cnt, ovf)) continue;
-                    Ld = Ld + r.contrib;
-                    lit |= 1 << kind;
-                }
-                if (PLAIN || lit) {
-                    p.rad = p.rad + Ld * p.thr;
-                    seen(b, lit);
-                }
+                seen(b, lit);
             }
         }
-        if (!bounce_post(op, p, st, m, eta, ev)) return;
-        p.depth++;
     }
+    if (!bounce_post(op, p, st, m, eta, ev)) return false;
+    p.depth++;
+    return true;
 }
-
 }  // namespace ptd

@@ -413,6 +413,7 @@ struct Cells {
 // half, one, two and four fills 415, 412, 410, 412 and 421 ms (stages to the
 // end: 440); after 16, 30 and 40 bounces at the latest 461, 412 and 409.
 constexpr int FINISH_BOUNCES = 40;
+constexpr long long FEW_TRIS = 16384;  // over all instances
 
 // NEE visibility is resolved inside the shade stage (shadow records are not
 // used) when AnyHit draws from the path's random numbers between NEE sampling
@@ -461,6 +462,16 @@ ptd::ShadowBuf shadow_buf(pt_renderer_s* h) { return ptd::ShadowBuf{h->s_idx.p, 
 //   21M triangles with foliage: 0.23M 19.1 / 20.3; 0.5M 30 / 26; 1M 48 / 39.
 struct Finish { int blocks, leave, whole; };
 
+// How many lanes of a wave wait before they begin new paths (64: all), in k_finish
+// and the plain form; paths: of the launch. Scenes of few triangles: 8
+// (pixel_samples has the figures, k_finish those of a larger scene). inl
+// (visibility inside the vertices): only from 16 paths per lane of the two waves
+// per SIMD on (900x700x8 volume MIS 7.1 -> 6.3 ms, blended alpha 7.1 -> 6.6;
+// 1001x563x2 volume MIS 2.26 -> 2.35, 1640x900 2.42 -> 2.41).
+int refill_lanes(const pt_renderer_s* h, bool inl, long long paths) {
+    return h->traced_tris <= FEW_TRIS && (!inl || paths >= 16LL * 512 * h->num_cu) ? 8 : 64;
+}
+
 Finish finish_setup(pt_renderer_s* h, bool inl) {
     Finish f{0, 0, 0};
     // uncompacted queues and instrumented runs keep the stages throughout
@@ -469,7 +480,7 @@ Finish finish_setup(pt_renderer_s* h, bool inl) {
                                       h->num_cu);
     h->spill.ensure(static_cast<size_t>(f.blocks) * 64 * (ptd::MAXD - ptd::FINISH_S + 1));
     f.leave = f.blocks * 64;
-    const long long fills = h->traced_tris <= 16384 ? 64 : h->traced_tris <= 4000000 ? 16 : 2;
+    const long long fills = h->traced_tris <= FEW_TRIS ? 64 : h->traced_tris <= 4000000 ? 16 : 2;
     f.whole = static_cast<int>(std::min<long long>(fills * f.leave, INT32_MAX / 2));
     return f;
 }
@@ -575,7 +586,8 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
     auto finish = [&](bool primary, int nb) {
         h->stage_begin(PT_STAGE_PLAIN, ev);
         ptk::launch_finish(s, w.fin.blocks, h->sc, op, pb0, nullptr, primary, w.inline_nee, h->qa.p, h->qb.p, cells.base, nb,
-                           w.fin.leave, D, npaths, w.npix, fs, cells.finish(), h->spill.p, h->ovf.p, w.tiles, rec);
+                           w.fin.leave, D, npaths, w.npix, fs, cells.finish(), h->spill.p, h->ovf.p, w.tiles,
+                           refill_lanes(h, w.inline_nee, npaths), rec);
         h->stage_end(PT_STAGE_PLAIN, ev);
     };
     if (w.fin.whole > 0 && w.max_paths <= static_cast<size_t>(w.fin.whole)) {
@@ -920,8 +932,8 @@ void batch_render_plain(pt_renderer_s* h, const pt_job* jobs, int n) {
     const int2* tiles = tile_entries(h, op, h->b_jobs.p, n, static_cast<int>(P.items / 64), P.max_side, P.samples);
     hipEvent_t ev;
     h->stage_begin(PT_STAGE_BATCH, ev);
-    ptk::launch_plain_batch(s, blocks, bs, h->sc, op, h->b_jobs.p, n, static_cast<int>(P.items), h->b_accum.p,
-                            h->counters.p, S, h->spill.p, h->ovf.p, inl, tiles);
+    ptk::launch_plain_batch(s, blocks, bs, h->sc, op, h->b_jobs.p, n, static_cast<int>(P.items), refill_lanes(h, inl, P.samples),
+                            h->b_accum.p, h->counters.p, S, h->spill.p, h->ovf.p, inl, tiles);
     h->stage_end(PT_STAGE_BATCH, ev);
     HIPCHK(hipGetLastError());
     batch_images(h, jobs, P);
@@ -991,7 +1003,8 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
         auto finish = [&](bool primary, int nb) {
             stage(PT_STAGE_PLAIN, [&] {
                 ptk::launch_finish(s, fin.blocks, h->sc, op, pb, &bb, primary, inl, h->qa.p, h->qb.p, cells.base, nb, fin.leave,
-                                   D, 0, 0, 0, cells.finish(), h->spill.p, h->ovf.p, tiles);
+                                   D, 0, 0, 0, cells.finish(), h->spill.p, h->ovf.p, tiles,
+                                   refill_lanes(h, inl, P.max_paths));
             });
         };
         const int nb = whole ? 0 : fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
@@ -1065,6 +1078,9 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     batch_images(h, jobs, P);
 }
 
+// Samples of a launch of the plain form.
+constexpr int PLAIN_SPP = 16;
+
 void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
     const DevOpts op = h->dev_opts();
     const int W = op.width, H = op.height;
@@ -1078,11 +1094,13 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
         ptk::persistent_blocks(inl && !cw ? ptk::KIND_PLAIN_INLINE : ptk::KIND_PLAIN, bs, S, cw, h->num_cu);
     h->ensure_spill(static_cast<size_t>(blocks) * bs);
     const int2* tiles = tile_entries(h, op, nullptr, 0, items / 64, std::max(W, H), static_cast<long long>(items) * num_samples);
-    for (int smp = first_sample; smp < first_sample + num_samples; ++smp) {
+    for (int k = 0; k < num_samples; k += PLAIN_SPP) {
+        const int spp = std::min(PLAIN_SPP, num_samples - k);
         hipEvent_t ev;
         ptk::launch_zero_cells(h->stream, h->counters.p, ptd::SHARDS);
         h->stage_begin(PT_STAGE_PLAIN, ev);
-        ptk::launch_plain(h->stream, blocks, bs, h->sc, op, h->accum.p, smp, items, h->counters.p, S, h->spill.p,
+        ptk::launch_plain(h->stream, blocks, bs, h->sc, op, h->accum.p, first_sample + k, spp,
+                          refill_lanes(h, inl, static_cast<long long>(items) * spp), items, h->counters.p, S, h->spill.p,
                           h->work_counts.p, h->ovf.p, cw, inl, tiles);
         h->stage_end(PT_STAGE_PLAIN, ev);
         HIPCHK(hipGetLastError());
