@@ -24,14 +24,16 @@
 
 namespace ptx {
 
-constexpr size_t LANE_PINNED = size_t{4} << 20;  // pinned bytes of a lane
+constexpr size_t LANE_PINNED = size_t{4} << 20;  // pinned bytes of a lane,
+constexpr size_t LANE_SMALL = size_t{64} << 10;  // or these (4 MB take 0.1 ms to pin, 0.1 to give back)
 constexpr int LANES_PER_CALL = 8;
 constexpr size_t POOL_LANES = 16;
 
 struct Lane {
     int device = 0;
     hipStream_t stream = nullptr;
-    char* pinned = nullptr;  // LANE_PINNED bytes
+    char* pinned = nullptr;
+    size_t pinned_n = 0;
     int* spill = nullptr;    // device: the query's traversal-stack backing store
     size_t spill_n = 0;
 
@@ -45,8 +47,16 @@ struct Lane {
     }
     hipError_t open(int dev) {
         device = dev;
-        hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&pinned), LANE_PINNED, hipHostMallocDefault);
+        return hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+    }
+    hipError_t ensure_pinned(size_t bytes) {  // bytes <= LANE_PINNED
+        if (pinned_n >= bytes) return hipSuccess;
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+        pinned_n = 0;
+        const size_t n = bytes <= LANE_SMALL ? LANE_SMALL : LANE_PINNED;
+        const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&pinned), n, hipHostMallocDefault);
+        if (e == hipSuccess) pinned_n = n;
         return e;
     }
     hipError_t ensure_spill(size_t ints) {
@@ -78,19 +88,21 @@ public:
         }
         for (Lane* l : gone) discard(l);
     }
-    // An idle lane of the device or a new one; null where none can be made.
-    Lane* take(int device) {
+    // An idle lane of the device or a new one, with `bytes` of pinned memory; null
+    // where that cannot be had.
+    Lane* take(int device, size_t bytes) {
+        Lane* l = nullptr;
         {
             std::lock_guard<std::mutex> g(m_);
-            for (size_t i = idle_.size(); i-- > 0;)
+            for (size_t i = idle_.size(); i-- > 0 && !l;)
                 if (idle_[i]->device == device) {
-                    Lane* l = idle_[i];
+                    l = idle_[i];
                     idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(i));
-                    return l;
                 }
         }
-        Lane* l = new (std::nothrow) Lane;
-        if (l && l->open(device) != hipSuccess) {
+        const bool made = !l;
+        if (made) l = new (std::nothrow) Lane;
+        if (l && ((made && l->open(device) != hipSuccess) || l->ensure_pinned(bytes) != hipSuccess)) {
             (void)hipGetLastError();
             delete l;
             l = nullptr;
@@ -121,12 +133,12 @@ private:
     int users_ = 0;
 };
 
-// Lanes lent to one call.
+// Lanes lent to one call, each with `bytes` of pinned memory.
 class Lanes {
 public:
-    Lanes(int device, int want) {
+    Lanes(int device, int want, size_t bytes) {
         for (int i = 0; i < std::min(want, LANES_PER_CALL); ++i) {
-            Lane* l = Pool::get().take(device);
+            Lane* l = Pool::get().take(device, bytes);
             if (!l) break;
             l_.push_back(l);
         }

@@ -341,7 +341,7 @@ static_assert(IMAGE_PART <= ptx::LANE_PINNED, "an image part fits a lane's pinne
 void copy_out(pt_renderer_s* h, void* dst, const void* src, size_t bytes) {
     const size_t part = IMAGE_PART;
     const int parts = static_cast<int>((bytes + part - 1) / part);
-    ptx::Lanes lanes(h->device, parts);
+    ptx::Lanes lanes(h->device, parts, std::min(bytes, part));
     if (lanes.size() == 0) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
@@ -899,7 +899,7 @@ void batch_images(pt_renderer_s* h, const pt_job* jobs, const BatchPlan& P) {
     std::sort(by_dst.begin(), by_dst.end(), [](const Part& a, const Part& b) { return a.dst < b.dst; });
     bool shared = false;
     for (size_t j = 1; j < by_dst.size(); ++j) shared |= by_dst[j].dst < by_dst[j - 1].dst + by_dst[j - 1].n;
-    ptx::Lanes lanes(h->device, shared ? 1 : static_cast<int>(std::min<size_t>(parts.size(), 64)));
+    ptx::Lanes lanes(h->device, shared ? 1 : static_cast<int>(std::min<size_t>(parts.size(), 64)), IMAGE_PART);
     if (lanes.size() == 0) {
         for (const Part& p : parts) HIPCHK(hipMemcpyAsync(p.dst, p.src, p.n, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
@@ -1123,7 +1123,7 @@ template <class Launch, class Done>
 int query(pt_handle h, const float* origins, const float* dirs, const float* reach, int n,
           Launch&& launch, Done&& done) {
     constexpr int RAYS = 65536, FEW = 32768;
-    static_assert(64 + size_t{RAYS} * 4 * (6 + 6) <= ptx::LANE_PINNED, "a part fits a lane's pinned memory");
+    static_assert(64 + size_t{RAYS} * 4 * (7 + 6) <= ptx::LANE_PINNED, "a part fits a lane's pinned memory");
     HIPCHK(hipSetDevice(h->device));
     HIPCHK(hipStreamSynchronize(h->stream));  // an edit or clear under way
     h->resolve_events();
@@ -1132,9 +1132,9 @@ int query(pt_handle h, const float* origins, const float* dirs, const float* rea
     const int least = (n - 1) / RAYS + 1, four = std::min(4, (n - 1) / FEW + 1);
     const int per = ((n - 1) / std::max(least, four) / 256 + 1) * 256;
     const int parts = (n - 1) / per + 1;
-    ptx::Lanes lanes(h->device, parts);
+    const size_t in_words = reach ? 7 : 6, out_words = 6;
+    ptx::Lanes lanes(h->device, parts, 64 + static_cast<size_t>(std::min(n, per)) * 4 * (in_words + out_words));
     if (lanes.size() == 0) return Fail(h, PT_ERR_HIP, "no pinned memory for a ray query");
-    const size_t in_words = reach ? 7 : 6;
     std::atomic<int> over{0};
     lanes.each(parts, [&](ptx::Lane& l, int k) {
         const int m = std::min(n - k * per, per);
