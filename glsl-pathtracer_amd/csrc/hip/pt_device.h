@@ -908,6 +908,13 @@ __device__ __forceinline__ void test_node4(const GNode4* __restrict__ nodes, int
 // hit does not depend on the order; what would is a stochastic alpha test,
 // whose draws follow the visit order, so callers that pass an RNG keep the
 // reference's order.
+// An iteration has the bodies one after another, instance entry, node, leaf, and
+// a lane goes through as many as its traversal comes to in that order (entry and
+// root node, node and the leaf it found): a wave of rays at different kinds of
+// body executes all of them in every iteration anyway, and so needs fewer
+// iterations than with one body per lane and iteration. Closest-hit stages of
+// the 4K foliage frame 305 -> 269 ms, 1080p spheres 13.9 -> 12.8, 512x512 boxes
+// 6.3 -> 5.9; preview of 995 moved instances 18.5 -> 16.0.
 // WIDE: the four-wide form (one loop per form: in a common one the other
 // form's node test costs registers and moves in every iteration).
 template <bool WIDE, bool ANY, bool COUNT, bool RESUME, bool UNORDERED>
@@ -943,6 +950,21 @@ __device__ __forceinline__ bool traverse_form(const DevScene& sc, vec3 O, vec3 D
             return false;
         }
         bool do_pop = false;
+        if (ref < 0 && blas_base < 0) {
+            // TLAS leaf: enter the instance's BLAS with the ray in object space.
+            if (COUNT) cnt.insts++;
+            cur_inst = -1 - ref;
+            const GInst I = sc.inst[cur_inst];
+            if (ANY && alpha) cur_mat = __float_as_int(I.f2.z);
+            inst_to_object(I, O, D, o, d);
+            inv = V(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+            if (WIDE) {
+                rows = near_rows(inv);
+                odd = sc.far_nodes4 || odd_ray(o, inv);
+            }
+            blas_base = top;
+            ref = __float_as_int(WIDE ? I.f2.w : I.f2.y);
+        }
         if (ref >= 0 && WIDE) {
             // Four-wide node (TLAS or BLAS): the hit children in order of the
             // reference's key (nearest first; equal keys in child order), the
@@ -1048,21 +1070,8 @@ __device__ __forceinline__ bool traverse_form(const DevScene& sc, vec3 O, vec3 D
             } else {
                 do_pop = true;
             }
-        } else if (blas_base < 0) {
-            // TLAS leaf: enter the instance's BLAS with the ray in object space.
-            if (COUNT) cnt.insts++;
-            cur_inst = -1 - ref;
-            const GInst I = sc.inst[cur_inst];
-            if (ANY && alpha) cur_mat = __float_as_int(I.f2.z);
-            inst_to_object(I, O, D, o, d);
-            inv = V(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-            if (WIDE) {
-                rows = near_rows(inv);
-                odd = sc.far_nodes4 || odd_ray(o, inv);
-            }
-            blas_base = top;
-            ref = __float_as_int(WIDE ? I.f2.w : I.f2.y);
-        } else {
+        }
+        if (!do_pop && ref < 0 && blas_base >= 0) {
             const int code = -1 - ref;
             const int first = code >> 2, count = code & 3;
             for (int i = 0; i < count; ++i) {
