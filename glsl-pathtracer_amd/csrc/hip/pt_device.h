@@ -914,7 +914,11 @@ __device__ __forceinline__ void test_node4(const GNode4* __restrict__ nodes, int
 // body executes all of them in every iteration anyway, and so needs fewer
 // iterations than with one body per lane and iteration. Closest-hit stages of
 // the 4K foliage frame 305 -> 269 ms, 1080p spheres 13.9 -> 12.8, 512x512 boxes
-// 6.3 -> 5.9; preview of 995 moved instances 18.5 -> 16.0.
+// 6.3 -> 5.9; preview of 995 moved instances 18.5 -> 16.0. A leaf is tested one
+// triangle per iteration: a loop over its triangles kept the wave's other rays
+// waiting (1080p closest hits 12.8 -> 12.5, any hits 3.9 -> 3.6, boxes 5.9 -> 5.5
+// and 2.7 -> 2.5; the foliage's any hits 19.2 -> 18.3, its closest hits, of which
+// the iteration limit then stops more, 270 -> 273).
 // WIDE: the four-wide form (one loop per form: in a common one the other
 // form's node test costs registers and moves in every iteration).
 template <bool WIDE, bool ANY, bool COUNT, bool RESUME, bool UNORDERED>
@@ -1074,9 +1078,9 @@ __device__ __forceinline__ bool traverse_form(const DevScene& sc, vec3 O, vec3 D
         if (!do_pop && ref < 0 && blas_base >= 0) {
             const int code = -1 - ref;
             const int first = code >> 2, count = code & 3;
-            for (int i = 0; i < count; ++i) {
+            if (count > 0) {
                 if (COUNT) cnt.tris++;
-                const GTri T = sc.tris[first + i];
+                const GTri T = sc.tris[first];
                 vec3 v0 = xyz(T.v0), e0 = xyz(T.e0), e1 = xyz(T.e1);
                 vec3 pv = cross(d, e1);
                 float det = dot(e0, pv);
@@ -1092,13 +1096,15 @@ __device__ __forceinline__ bool traverse_form(const DevScene& sc, vec3 O, vec3 D
                 float tt = dot(e1, qv) * rdet;
                 float ww = 1.0f - uu - vv;
                 if (uu >= 0.0f && vv >= 0.0f && tt >= 0.0f && ww >= 0.0f && tt < best) {
-                    if (ANY && !(alpha && alpha_transparent(sc, first + i, cur_mat, uu, vv, ww, rng))) return true;
-                    if (ANY) continue;
-                    best = tt;
-                    h.t = tt; h.u = uu; h.v = vv; h.tri = first + i; h.inst = cur_inst; h.light = -1;
+                    if (ANY && !(alpha && alpha_transparent(sc, first, cur_mat, uu, vv, ww, rng))) return true;
+                    if (!ANY) {
+                        best = tt;
+                        h.t = tt; h.u = uu; h.v = vv; h.tri = first; h.inst = cur_inst; h.light = -1;
+                    }
                 }
             }
-            do_pop = true;
+            if (count > 1) ref -= 3;  // the leaf without its first triangle
+            else do_pop = true;
         }
         if (do_pop) {
             if (top == blas_base) {
