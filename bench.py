@@ -590,7 +590,7 @@ def main():
     extend_ms = st_w["ms_stage"]["extend"]
     extend_launches = max(1, st_w["launches_stage"]["extend"])
     if not args.no_count:
-        cspp = min(args.spp, 4)
+        cspp = min(args.spp, 16)  # as many as make camera rays start at their tiles' entries, as in the timed frames
         cw = count_work(r, sc, rs, cspp, opts_kw)
         scale = args.spp * args.steps / cspp
         bytes_total = scale * (B_NODE * cw["nodes_visited"] + B_TRI * cw["tris_tested"] +

@@ -324,8 +324,8 @@ int pt_batch_render(pt_handle h, const pt_job* jobs, int32_t num_jobs);
  * Sampling, MIS weights and Russian roulette are detached: the estimate is
  * unbiased for the gradient of the expected image. Runs the wavefront form
  * whatever pt_options.mode says: a primal pass (the forward render, which
- * also records which NEE rays were visible) and a replay pass that re-traces
- * the same paths and accumulates the gradients. Returns PT_ERR_UNSUPPORTED
+ * also records the closest hits and which NEE rays were visible) and a replay pass over
+ * the same paths that accumulates the gradients. Returns PT_ERR_UNSUPPORTED
  * with roughness mollification, stochastic (blend) alpha in shadow rays or
  * volume MIS enabled; PT_ERR_STATE if a path vertex names a material outside
  * the table. Vertices whose gradient has a non-finite term are left out and
