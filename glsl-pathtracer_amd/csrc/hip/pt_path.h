@@ -480,9 +480,10 @@ __device__ __forceinline__ float4 path_trace(const DevScene& sc, const DevOpts& 
 // position (aperture 0) inside the pyramid of the tile's pixels and their one
 // pixel of jitter, so a box, rectangle or sphere outside one of its four side
 // planes is hit by none of them. The planes get a quarter pixel more and the
-// objects the rounding of the rays and of the slab test many times over
-// (1e-5 of the coordinates involved), so nothing a ray's own test accepts is
-// left out. The entry is the deepest TLAS node with every instance in the
+// objects the rounding of the rays and of the slab and rectangle tests many
+// times over (1e-5 of the coordinates involved); a sphere's own test is far
+// less exact where it is small and distant, so a sphere gets that test's error
+// (below). Nothing a ray's own test accepts is left out. The entry is the deepest TLAS node with every instance in the
 // pyramid below it: the subtrees left out hold no hit, and below the entry the
 // visit order is that of the whole traversal.
 struct Pyramid {
@@ -583,7 +584,14 @@ __device__ __forceinline__ Entry tile_entry(const DevScene& sc, const DevOpts& o
                     en.lights = !outside(P, lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]);
                 }
             } else if (L.u.w == static_cast<float>(SPHERE_LIGHT)) {
-                const double r = fabs(static_cast<double>(L.p.w)) * 1.001;
+                // SphereIntersect compares b * b - d * d + r * r with 0 in floats (d
+                // the distance of the centre, b its component along the ray). With
+                // the ray's direction of unit length to 4 roundings, b * b is off
+                // by at most 14 of them (2^-24 d * d each), d * d by 5 and the
+                // difference by one: 1.2e-6 d * d, more than r * r where the sphere
+                // is smaller than a thousandth of its distance.
+                const double x = L.p.x - P.px, y = L.p.y - P.py, z = L.p.z - P.pz, rad = L.p.w;
+                const double r = sqrt(1.002 * rad * rad + 2e-6 * (x * x + y * y + z * z));
                 en.lights = !outside(P, L.p.x - r, L.p.y - r, L.p.z - r, L.p.x + r, L.p.y + r, L.p.z + r);
             }
         }

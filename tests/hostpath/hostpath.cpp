@@ -347,3 +347,51 @@ extern "C" int host_node4(int n, const float* lo, const float* hi, const int* co
     *odds = no;
     return 0;
 }
+
+// Camera rays of the 8x8 tiles [tx0, tx1) x [ty0, ty1), samples [0, n): the
+// closest hit from the tile's entry (tile_entry) against the one from the whole
+// scene. Writes the rays whose hits differ in any bit, the rays that hit
+// something, and the tiles whose entry leaves out lights or part of the TLAS.
+extern "C" int host_tile_hits(const pt_scene_view* v, const pt_options* o, const pt_camera* cam, int tx0, int ty0,
+                              int tx1, int ty1, int n, int* differ, int* hits, int* culled) {
+    try {
+        HostScene H(v, o, cam);
+        const DevScene& sc = H.sc;
+        const DevOpts op = H.op;
+        const int tiles_x = (op.width + 7) / 8;
+        int bad = 0, nh = 0, nc = 0;
+#pragma omp parallel reduction(+ : bad, nh, nc)
+        {
+            std::vector<int> lds(MAXD + 1), spill(MAXD + 1), walk(CULL_STACK);
+            Stack stk{lds.data(), spill.data(), 0, 1, MAXD, 0, 1};
+            TravCount cnt{0, 0, 0, 0, 0, 0};
+            bool ovf = false;
+#pragma omp for schedule(dynamic, 1)
+            for (int ty = ty0; ty < ty1; ++ty)
+                for (int tx = tx0; tx < tx1; ++tx) {
+                    const Entry en = tile_entry(sc, op, ty * tiles_x + tx, walk.data(), 1);
+                    nc += en.root != sc.root || !en.lights;
+                    for (int i = 0; i < 64 * n; ++i) {
+                        const int px = 8 * tx + (i & 7), py = 8 * ty + ((i >> 3) & 7);
+                        if (px >= op.width || py >= op.height) continue;
+                        PathRegs p;
+                        p.rng = init_rng((uint32_t)px, (uint32_t)py, (uint32_t)((i >> 6) + 2));
+                        camera_ray(op, px, py, p.rng, p.ro, p.rd);
+                        const Hit a = closest<false>(sc, op, p.ro, p.rd, 0, stk, cnt, ovf);
+                        const Hit b = closest<false>(sc, op, p.ro, p.rd, 0, stk, cnt, ovf, en);
+                        nh += a.t != INF;
+                        bad += !(memcmp(&a.t, &b.t, 4) == 0 && memcmp(&a.u, &b.u, 4) == 0 &&
+                                 memcmp(&a.v, &b.v, 4) == 0 && a.tri == b.tri && a.inst == b.inst &&
+                                 a.light == b.light);
+                    }
+                }
+        }
+        *differ = bad;
+        *hits = nh;
+        *culled = nc;
+        return 0;
+    } catch (const std::exception& e) {
+        fprintf(stderr, "host_tile_hits: %s\n", e.what());
+        return -1;
+    }
+}
