@@ -483,9 +483,10 @@ __device__ __forceinline__ float4 path_trace(const DevScene& sc, const DevOpts& 
 // objects the rounding of the rays and of the slab and rectangle tests many
 // times over (1e-5 of the coordinates involved); a sphere's own test is far
 // less exact where it is small and distant, so a sphere gets that test's error
-// (below). Nothing a ray's own test accepts is left out. The entry is the deepest TLAS node with every instance in the
-// pyramid below it: the subtrees left out hold no hit, and below the entry the
-// visit order is that of the whole traversal.
+// (below). Nothing a ray's own test accepts is left out. The entry is the
+// deepest inner TLAS node with every instance in the pyramid below it: the
+// subtrees left out hold no hit, and below the entry the visit order is that of
+// the whole traversal.
 struct Pyramid {
     double px, py, pz;        // apex
     double n[4][3];           // inward plane normals (zero: no plane)
@@ -619,7 +620,9 @@ __device__ __forceinline__ Entry tile_entry(const DevScene& sc, const DevOpts& o
             if (any) { ++seen; only = kids[j].ref; }
         }
         if (seen == 0) { en.root = EMPTY4; break; }
-        if (seen > 1) break;
+        // an instance is entered from its parent, which tests its box: at a
+        // silhouette the rounded box decides, and a BLAS that is one leaf has none
+        if (seen > 1 || only < 0) break;
         en.root = only;
     }
     return en;

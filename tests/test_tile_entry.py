@@ -75,3 +75,29 @@ def test_lights_are_still_left_out():
     sc, rs, cam, at = lights_in_view(np.random.default_rng(8), 1, 640, 360, 40.0, 0.02)
     differ, _, culled = tile_hits(sc, rs, cam, (0, 0, 80, 45), 1)
     assert differ == 0 and culled > 80 * 45 * 0.9
+
+
+@pytest.mark.parametrize("width4", [2, 4])
+@pytest.mark.parametrize("far", [0.0, 1e3, 1e5])
+@pytest.mark.parametrize("freq", [0, 2])
+def test_instance_boxes_are_tested(freq, far, width4):
+    """Instances far from the origin, where the rounding of boxes and rays is
+    seen at silhouettes: a tile that sees one instance alone tests its box all
+    the same. freq 0: single quads, whose BLAS has no box of its own."""
+    rng = np.random.default_rng(11)
+    sc = scenes.Scene()
+    if freq:
+        mesh = sc.AddMesh(*scenes.displaced_icosphere(freq, 0.1, 3), name="sphere")
+    else:
+        mesh = sc.AddMesh(*scenes._uv_quad((-0.5, -0.5, 0), (1, 0, 0), (0, 1, 0)), name="quad")
+    mat = sc.AddMaterial(baseColor=(0.7, 0.7, 0.7))
+    for k in range(40):
+        t = rng.uniform(-12, 12, 3) + np.array([far, -far, far])
+        rot = scenes.random_rotation(rng) if k % 4 else np.eye(4)
+        sc.AddMeshInstance(mesh, scenes.mat4(translate=t, scale=(rng.uniform(0.5, 3),) * 3, rot=rot), mat)
+    sc.AddCamera((far, -far, far + 36), (far, -far, far), 45.0)
+    sc.ProcessScene()
+    rs = scenes.RenderSettings(400, 300, 16, 1)
+    differ, hits, culled = tile_hits(sc, rs, sc.camera(), (0, 0, 50, 38), 16, bvh_width=width4)
+    print(f"{differ} of {hits} hits differ, {culled} tiles culled")
+    assert differ == 0 and hits > 1000 and culled > 100
