@@ -83,7 +83,8 @@ struct DevScene {
     const float* __restrict__ env_img;  // RGB32F
     const float* __restrict__ env_cdf;
     int root;                           // TLAS root reference (in nodes4 when that is set)
-    int far_nodes4;                     // 1: nodes4 holds 2^25 entries or more (beyond 32-bit byte offsets)
+    int far_nodes4;                     // 1: nodes4 holds 2^25 entries or more (beyond 32-bit byte offsets), or
+                                        // a box plane so far out that a key may be infinite (ptl::FAR_PLANE)
     int root_bin;                       // EMPTY4, or the BVH2 TLAS root that any-hit traversals drawing
                                         // random numbers walk (nodes4 set and a material blends)
     int num_lights;
@@ -859,7 +860,8 @@ __device__ __forceinline__ void test_node4(const GNode4* __restrict__ nodes, int
                                            bool odd, float best, Kids4& c) {
     const float none = __builtin_inff();
     // 32-bit byte offsets: arrays of 2^25 nodes and more go through `odd` (the
-    // wrapped offset still lies in the array)
+    // wrapped offset still lies in the array), as do scenes whose planes could
+    // make a hit child's key infinite (a clamp here is four instructions per node)
     const char* base = reinterpret_cast<const char*>(nodes);
     const uint32_t at = static_cast<uint32_t>(ref) << 7;
     const uint32_t ax = at | rows.x, ay = at | rows.y, az = at | rows.z;

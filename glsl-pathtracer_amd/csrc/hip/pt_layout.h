@@ -109,6 +109,36 @@ inline int collapse4_tlas(const GNode* n2, int off, int root2, int base, size_t 
     return root4;
 }
 
+// Whether a box plane lies beyond FAR_PLANE: its distance times a reciprocal
+// direction of up to 1e18 (ptd::odd_ray) can then pass the float range, and the
+// four-wide node test takes an infinite key for a miss (DevScene::far_nodes4).
+constexpr float FAR_PLANE = 1e18f;
+inline bool far_plane(float a, float b, float c) {
+    return std::fabs(a) > FAR_PLANE || std::fabs(b) > FAR_PLANE || std::fabs(c) > FAR_PLANE;
+}
+inline bool far_node(const GNode& g) {
+    return far_plane(g.a.x, g.a.y, g.a.z) || far_plane(g.a.w, g.b.x, g.b.y) || far_plane(g.b.z, g.b.w, g.c.x) ||
+           far_plane(g.c.y, g.c.z, g.c.w);
+}
+// The largest coordinate of the instances' local boxes.
+inline float local_reach(const std::vector<float>& local) {
+    float m = 0.f;
+    for (float f : local) m = std::max(m, std::fabs(f));
+    return m;
+}
+// Whether a box of these instances may have a far plane (not finite: yes).
+inline bool far_instances(const float* xf, int n, float reach) {
+    for (int i = 0; i < n; ++i) {
+        const float* m = xf + 16 * static_cast<size_t>(i);
+        for (int r = 0; r < 3; ++r) {
+            const double a = std::fabs(static_cast<double>(m[r])) + std::fabs(static_cast<double>(m[4 + r])) +
+                             std::fabs(static_cast<double>(m[8 + r]));
+            if (!(a * reach + std::fabs(static_cast<double>(m[12 + r])) <= FAR_PLANE)) return true;
+        }
+    }
+    return false;
+}
+
 // Re-layout of the reference's flat node array (bvh_translator.cpp:32-137)
 // into BVH2 nodes. Only nodes reachable from the TLAS root are converted;
 // GNode order follows the flat (preorder) order, so subtrees stay contiguous.
@@ -123,6 +153,8 @@ struct Relayout {
     int tlas4_base = 0;                     // first four-wide TLAS entry in wide.nodes (at least max(n - 1, 1) follow)
     int root4 = 0;                          // four-wide TLAS root reference
     long long traced_tris = 0;              // triangles over all instances (an estimate)
+    float local_max = 0.f;                  // local_reach of inst_local
+    bool far = false;                       // a TLAS box or a BLAS root's box has a far plane
     // The TLAS as the device rebuild writes it: one instance per leaf, every
     // instance once, internal nodes numbered in preorder from tlas_base to the
     // end of the node array.
@@ -244,6 +276,16 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
         auto tris_of = [&](int ref) { return ref < 0 ? (-1 - ref) & 3 : below[ref]; };
         for (int i = n - 1; i >= 0; --i) below[i] = tris_of(R.nodes[i].d.x) + tris_of(R.nodes[i].d.y);
         for (int i = 0; i < num_instances; ++i) R.traced_tris += tris_of(R.inst_blas_ref[i]);
+    }
+    R.local_max = local_reach(R.inst_local);
+    R.far = R.local_max > FAR_PLANE;
+    for (st.assign(1, R.root); !st.empty() && !R.far;) {  // the inner TLAS nodes
+        const int r = st.back();
+        st.pop_back();
+        if (r < 0) continue;
+        R.far = far_node(R.nodes[r]);
+        st.push_back(R.nodes[r].d.x);
+        st.push_back(R.nodes[r].d.y);
     }
     R.inst_blas4_ref.assign(num_instances, 0);
     for (int i = 0; i < num_instances; ++i) {

@@ -93,6 +93,8 @@ struct pt_renderer_s {
     std::unordered_map<int, int> root4;    // BLAS root: BVH2 reference -> four-wide reference
     int root2 = 0, root4_tlas = 0;         // TLAS root in the BVH2 and in the four-wide form
     int t4_base = 0, t4_room = 0;          // four-wide TLAS entries [t4_base, t4_base + t4_room) of nodes4
+    float local_max = 0.f;                 // largest coordinate of the instances' local boxes
+    bool far_boxes = false;                // a box plane may lie beyond ptl::FAR_PLANE
     DevBuf<GTri> tris;
     DevBuf<int4> vidx;
     DevBuf<float4> verts, norms, mats;
@@ -258,7 +260,7 @@ struct pt_renderer_s {
     void select_bvh() {
         sc.nodes4 = (opts.bvh_width == 4 && nodes4.p) ? nodes4.p : nullptr;
         sc.root = sc.nodes4 ? root4_tlas : root2;
-        sc.far_nodes4 = nodes4.n >= (size_t{1} << 25) ? 1 : 0;
+        sc.far_nodes4 = nodes4.n >= (size_t{1} << 25) || far_boxes ? 1 : 0;
         sc.root_bin = (sc.nodes4 && any_blend) ? root2 : ptd::EMPTY4;
     }
     void set_tlas_roots(const Relayout& R) {
@@ -267,6 +269,8 @@ struct pt_renderer_s {
         t4_base = R.tlas4_base;
         t4_room = static_cast<int>(R.wide.nodes.size()) - R.tlas4_base;
         traced_tris = R.traced_tris;
+        local_max = R.local_max;
+        far_boxes = R.far;
     }
     // Four-wide BLAS roots of BVH2 BLAS root references.
     std::vector<int> blas4_of(const std::vector<int>& blas2) const {
@@ -1437,6 +1441,9 @@ int pt_update_instances(pt_handle h, const float* transforms, int32_t num_instan
             h->inst_blas4 = blas4;
             h->inst_mat = T.mat;
             h->tlas_on_device = false;
+            h->local_max = ptl::local_reach(local);
+            h->far_boxes = h->local_max > ptl::FAR_PLANE || std::any_of(T.nodes.begin(), T.nodes.end(), ptl::far_node);
+            h->select_bvh();
         } else if (nodes) {
             // Everything is checked before any state changes.
             std::vector<pt_bvh_node> flat = h->flat;
@@ -1546,6 +1553,8 @@ int pt_rebuild_instances(pt_handle h, const float* transforms, int32_t num_insta
         }
         HIPCHK(hipStreamSynchronize(s));
         h->tlas_on_device = true;
+        h->far_boxes = h->local_max > ptl::FAR_PLANE || ptl::far_instances(transforms, n, h->local_max);
+        h->select_bvh();
         return PT_OK;
     });
 }

@@ -50,6 +50,7 @@ struct HostScene {
         sc.env_img = has_env ? v->env_img : nullptr;
         sc.env_cdf = has_env ? v->env_cdf : nullptr;
         sc.root = sc.nodes4 ? R.root4 : R.root;
+        sc.far_nodes4 = R.far;
         bool any_blend = false;
         for (int i = 0; i < v->num_materials; ++i)
             if ((int)v->materials[i].alphaMode == ALPHA_MODE_BLEND) any_blend = true;
@@ -392,6 +393,33 @@ extern "C" int host_tile_hits(const pt_scene_view* v, const pt_options* o, const
         return 0;
     } catch (const std::exception& e) {
         fprintf(stderr, "host_tile_hits: %s\n", e.what());
+        return -1;
+    }
+}
+
+// Closest hits of n rays.
+extern "C" int host_closest(const pt_scene_view* v, const pt_options* o, const pt_camera* cam, int n, const float* orig,
+                            const float* dir, float* t, int* tri, int* inst) {
+    try {
+        HostScene H(v, o, cam);
+#pragma omp parallel
+        {
+            std::vector<int> lds(MAXD + 1), spill(MAXD + 1);
+            Stack stk{lds.data(), spill.data(), 0, 1, MAXD, 0, 1};
+            TravCount cnt{0, 0, 0, 0, 0, 0};
+            bool ovf = false;
+#pragma omp for schedule(dynamic, 256)
+            for (int i = 0; i < n; ++i) {
+                const Hit h = closest<false>(H.sc, H.op, V(orig[3 * i], orig[3 * i + 1], orig[3 * i + 2]),
+                                             V(dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]), 1, stk, cnt, ovf);
+                t[i] = h.t;
+                tri[i] = h.tri;
+                inst[i] = h.inst;
+            }
+        }
+        return 0;
+    } catch (const std::exception& e) {
+        fprintf(stderr, "host_closest: %s\n", e.what());
         return -1;
     }
 }
