@@ -162,10 +162,10 @@ struct pt_renderer_s {
     DevBuf<float4> c_hf;
     DevBuf<int> spill;
     DevBuf<unsigned long long> work_counts;  // [0,6) closest-hit work, [8,14) shadow work: nodes, tris, insts, lights, spills, rays
-    // Stack-overflow flag in pinned memory: the host clears it before a render
-    // (none is under way then) and reads it after, with no copy of its own; a
-    // kernel stores 1.
-    struct { int* p = nullptr; } ovf;  // made by the first render
+    // Stack-overflow flag, in pinned memory where that can be had: the host clears
+    // it before a render (none is under way then) and reads it after, with no copy
+    // of its own; a kernel stores 1.
+    struct { int* p = nullptr; bool pinned = false; } ovf;  // made by the first render
     bool lane_user = false;
     DevBuf<uchar4> ldr;
 
@@ -195,7 +195,7 @@ struct pt_renderer_s {
         t_xf.free(); t_local.free(); t_box.free(); t_cen.free(); t_blas.free(); t_blas4.free(); t_mat.free(); t_ord.free();
         t_pre.free(); t_pos.free(); t_pseg.free(); t_seg.free(); t_keys.free();
         r_hit.free(); r_hit2.free(); r_q.free();
-        if (ovf.p) (void)hipHostFree(ovf.p);
+        if (ovf.p) (void)(ovf.pinned ? hipHostFree(ovf.p) : hipFree(ovf.p));
         if (stream) (void)hipStreamDestroy(stream);
         if (lane_user) ptx::Pool::get().drop_user();
     }
@@ -253,7 +253,12 @@ struct pt_renderer_s {
             stats.rays_shadow = static_cast<int64_t>(c[13]);
             stats.stack_spills = static_cast<int64_t>(c[4] + c[12]);
         }
-        if (ovf.p) stats.stack_overflow = *static_cast<volatile int*>(ovf.p);
+        if (ovf.p) {
+            int f = 0;
+            if (ovf.pinned) f = *static_cast<volatile int*>(ovf.p);
+            else HIPCHK(hipMemcpy(&f, ovf.p, sizeof(int), hipMemcpyDeviceToHost));
+            stats.stack_overflow = f;
+        }
     }
 
     // The BLAS form the kernels traverse follows pt_options.bvh_width.
@@ -295,7 +300,17 @@ struct pt_renderer_s {
     }
     void ensure_misc() {
         work_counts.ensure(16);
-        if (!ovf.p) HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&ovf.p), sizeof(int), hipHostMallocDefault));
+        if (ovf.p) return;
+        ovf.pinned = hipHostMalloc(reinterpret_cast<void**>(&ovf.p), sizeof(int), hipHostMallocDefault) == hipSuccess;
+        if (!ovf.pinned) {
+            (void)hipGetLastError();
+            ovf.p = nullptr;
+            HIPCHK(hipMalloc(reinterpret_cast<void**>(&ovf.p), sizeof(int)));
+        }
+    }
+    void clear_ovf() {
+        if (ovf.pinned) *ovf.p = 0;
+        else HIPCHK(hipMemsetAsync(ovf.p, 0, sizeof(int), stream));
     }
     // Continuation buffer for passes of up to max_paths paths: room for a
     // quarter of them (later bounces hold only the paths still alive, and of
@@ -1113,7 +1128,7 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
 
 // A ray query over the caller's arrays in parts of up to RAYS rays, each through
 // the pinned memory of a lane, which the kernel reads and writes itself over the
-// bus: launch(lane, n, in, out, S, flag) queues the query of n rays whose inputs
+// bus: launch(stream, spill, n, in, out, S, flag) queues the query of n rays whose inputs
 // lie at `in` (origins, directions, and reaches where given, one after another)
 // and whose answers, up to six words a ray, go to `out`; done(first, n, out) takes
 // them. Copies of the parts to device memory and back instead cost as much as
@@ -1138,7 +1153,37 @@ int query(pt_handle h, const float* origins, const float* dirs, const float* rea
     const int parts = (n - 1) / per + 1;
     const size_t in_words = reach ? 7 : 6, out_words = 6;
     ptx::Lanes lanes(h->device, parts, 64 + static_cast<size_t>(std::min(n, per)) * 4 * (in_words + out_words));
-    if (lanes.size() == 0) return Fail(h, PT_ERR_HIP, "no pinned memory for a ray query");
+    if (lanes.size() == 0) {  // no pinned memory to be had: through device memory, part by part
+        struct Buffers {
+            DevBuf<float> in, out;
+            DevBuf<int> spill, flag;
+            ~Buffers() { in.free(); out.free(); spill.free(); flag.free(); }
+        } b;
+        std::vector<float> answers(static_cast<size_t>(std::min(n, per)) * out_words);
+        int over = 0;
+        for (int k = 0; k < parts; ++k) {
+            const int m = std::min(n - k * per, per);
+            const size_t first = static_cast<size_t>(k) * per, um = static_cast<size_t>(m);
+            b.in.ensure(um * in_words);
+            b.out.ensure(um * out_words);
+            b.spill.ensure((um + 255) / 256 * 256 * static_cast<size_t>(ptd::MAXD - S + 1));
+            b.flag.ensure(1);
+            HIPCHK(hipMemsetAsync(b.flag.p, 0, sizeof(int), h->stream));
+            HIPCHK(hipMemcpyAsync(b.in.p, origins + 3 * first, 12 * um, hipMemcpyHostToDevice, h->stream));
+            HIPCHK(hipMemcpyAsync(b.in.p + 3 * um, dirs + 3 * first, 12 * um, hipMemcpyHostToDevice, h->stream));
+            if (reach)
+                HIPCHK(hipMemcpyAsync(b.in.p + 6 * um, reach + first, 4 * um, hipMemcpyHostToDevice, h->stream));
+            launch(h->stream, b.spill.p, m, b.in.p, b.out.p, S, b.flag.p);
+            HIPCHK(hipGetLastError());
+            int f = 0;
+            HIPCHK(hipMemcpyAsync(answers.data(), b.out.p, 4 * um * out_words, hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(hipMemcpyAsync(&f, b.flag.p, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(hipStreamSynchronize(h->stream));
+            done(first, m, answers.data());
+            over |= f;
+        }
+        return over ? Fail(h, PT_ERR_OVERFLOW, "BVH traversal exceeded the maximum stack depth") : PT_OK;
+    }
     std::atomic<int> over{0};
     lanes.each(parts, [&](ptx::Lane& l, int k) {
         const int m = std::min(n - k * per, per);
@@ -1151,7 +1196,7 @@ int query(pt_handle h, const float* origins, const float* dirs, const float* rea
         std::memcpy(in, origins + 3 * first, 12 * um);
         std::memcpy(in + 3 * um, dirs + 3 * first, 12 * um);
         if (reach) std::memcpy(in + 6 * um, reach + first, 4 * um);
-        launch(l, m, in, out, S, flag);
+        launch(l.stream, l.spill, m, in, out, S, flag);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(l.stream));
         done(first, m, out);
@@ -1684,7 +1729,7 @@ int pt_render(pt_handle h, int32_t first_sample, int32_t num_samples) {
             HIPCHK(hipMemsetAsync(h->work_counts.p, 0, 16 * sizeof(unsigned long long), h->stream));
         }
         h->ensure_misc();
-        *h->ovf.p = 0;
+        h->clear_ovf();
         HIPCHK(hipEventRecord(h->ev_r0, h->stream));
         if (h->opts.mode == PT_MODE_PLAIN) render_plain(h, first_sample, num_samples);
         else render_wavefront(h, first_sample, num_samples);
@@ -1778,11 +1823,11 @@ int pt_closest_hit(pt_handle h, const float* origins, const float* dirs, int32_t
         const DevOpts op = query_opts(h);
         return query(
             h, origins, dirs, nullptr, n,
-            [&](ptx::Lane& l, int m, float* in, float* out, int S, int* flag) {
+            [&](hipStream_t s, int* spill, int m, float* in, float* out, int S, int* flag) {
                 int* ids = reinterpret_cast<int*>(out);
-                ptk::launch_query_closest(l.stream, h->sc, op, in, in + 3 * static_cast<size_t>(m), m, out, ids + m,
+                ptk::launch_query_closest(s, h->sc, op, in, in + 3 * static_cast<size_t>(m), m, out, ids + m,
                                           ids + 2 * static_cast<size_t>(m), ids + 3 * static_cast<size_t>(m),
-                                          out + 4 * static_cast<size_t>(m), S, l.spill, flag);
+                                          out + 4 * static_cast<size_t>(m), S, spill, flag);
             },
             [&](size_t first, int m, const float* out) {
                 const size_t um = static_cast<size_t>(m);
@@ -1812,10 +1857,10 @@ int pt_any_hit(pt_handle h, const float* origins, const float* dirs, const float
         const DevOpts op = query_opts(h);
         return query(
             h, origins, dirs, max_dist, n,
-            [&](ptx::Lane& l, int m, float* in, float* out, int S, int* flag) {
+            [&](hipStream_t s, int* spill, int m, float* in, float* out, int S, int* flag) {
                 const size_t um = static_cast<size_t>(m);
-                ptk::launch_query_any(l.stream, h->sc, op, in, in + 3 * um, in + 6 * um, m, reinterpret_cast<int*>(out),
-                                      S, l.spill, flag);
+                ptk::launch_query_any(s, h->sc, op, in, in + 3 * um, in + 6 * um, m, reinterpret_cast<int*>(out),
+                                      S, spill, flag);
             },
             [&](size_t first, int m, const float* out) { std::memcpy(occluded + first, out, 4 * static_cast<size_t>(m)); });
     });
@@ -1830,7 +1875,7 @@ int pt_batch_render(pt_handle h, const pt_job* jobs, int32_t num_jobs) {
         HIPCHK(hipSetDevice(h->device));
         h->resolve_events();
         h->ensure_misc();
-        *h->ovf.p = 0;
+        h->clear_ovf();
         HIPCHK(hipEventRecord(h->ev_r0, h->stream));
         batch_render(h, jobs, num_jobs);
         HIPCHK(hipEventRecord(h->ev_r1, h->stream));
@@ -1861,7 +1906,7 @@ static int adjoint_call(pt_handle h, int32_t first_sample, int32_t num_samples, 
         ptk::launch_fill(h->stream, reinterpret_cast<int*>(h->a_grad.p), static_cast<int>(ng), 0);
         ptk::launch_fill(h->stream, h->a_flags.p, 2, 0);
         h->ensure_misc();
-        *h->ovf.p = 0;
+        h->clear_ovf();
         HIPCHK(hipEventRecord(h->ev_r0, h->stream));
         adjoint_wavefront(h, first_sample, num_samples, 1.0f / static_cast<float>(num_samples), d_medium != nullptr);
         HIPCHK(hipEventRecord(h->ev_r1, h->stream));
