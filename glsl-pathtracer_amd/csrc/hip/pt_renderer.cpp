@@ -47,6 +47,12 @@ struct HipError : std::exception {
     explicit HipError(std::string m) : msg(std::move(m)) {}
     const char* what() const noexcept override { return msg.c_str(); }
 };
+// Device memory that could not be had. Every call asks for its memory before it
+// changes what a repetition of the call would count again (accumulated samples,
+// gradients), so Guard() may run it a second time.
+struct MemError : HipError {
+    using HipError::HipError;
+};
 #define HIPCHK(x)                                                                           \
     do {                                                                                    \
         hipError_t e_ = (x);                                                                \
@@ -66,7 +72,11 @@ struct DevBuf {
         if (count <= n && p) return;
         free();
         if (count == 0) return;
-        HIPCHK(hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T)));
+        const hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T));
+        if (e != hipSuccess) {
+            p = nullptr;
+            throw MemError("device memory of " + std::to_string(count * sizeof(T)) + " bytes: " + hipGetErrorString(e));
+        }
         n = count;
     }
     void upload(const T* src, size_t count, hipStream_t s) {
@@ -198,6 +208,13 @@ struct pt_renderer_s {
         if (ovf.p) (void)(ovf.pinned ? hipHostFree(ovf.p) : hipFree(ovf.p));
         if (stream) (void)hipStreamDestroy(stream);
         if (lane_user) ptx::Pool::get().drop_user();
+    }
+
+    // Gives the adjoint's record of hits back; whether there was one.
+    bool drop_record() {
+        const bool any = r_hit.p || r_hit2.p || r_q.p;
+        r_hit.free(); r_hit2.free(); r_q.free();
+        return any;
     }
 
     hipEvent_t get_event() {
@@ -335,6 +352,12 @@ template <class F>
 int Guard(pt_handle h, F&& f) {
     if (!h) return PT_ERR_INVALID_ARG;
     try {
+        try {
+            return f();
+        } catch (const MemError&) {  // again, without the record that earlier adjoints left
+            (void)hipGetLastError();
+            if (!h->drop_record()) throw;
+        }
         return f();
     } catch (const HipError& e) {
         return Fail(h, PT_ERR_HIP, e.msg);
@@ -678,8 +701,10 @@ void render_wavefront(pt_renderer_s* h, int first_sample, int num_samples) {
 
 // The adjoint's record of hits: 28 bytes per path and bounce, for as many bounces
 // as RECORD_BYTES hold and RECORD_BOUNCES at least (a path that goes on for longer
-// is rare), within a sixteenth of the device's memory; none where that cannot be
-// had. The bounces beyond query the hits again. Render and gradient of 64
+// is rare), within a sixteenth of the device's memory; half as many, and so on,
+// where that cannot be had. The bounces beyond query the hits again. A record of
+// up to RECORD_BYTES is kept for the next call, a larger one given back, and any
+// where another call's memory cannot be had otherwise (Guard). Render and gradient of 64
 // materials, 512x512x16 samples at depth 4: 19.5 -> 16.0 ms (closest-hit stages
 // 9.9 -> 6.3); 200x150x4: 3.9 -> 2.6. Alpha-tested foliage, where paths may take
 // 64 bounces more than their depth, 256x192x8 with media: 106 -> 85 ms with 16
@@ -693,15 +718,15 @@ ptd::Record hit_record(pt_renderer_s* h, const Wavefront& w) {
     const size_t each = 28 * r.qrow;
     size_t n = std::max(static_cast<size_t>(RECORD_BOUNCES), RECORD_BYTES / each);
     n = std::min({n, static_cast<size_t>(w.D), h->device_bytes / 16 / each});
-    try {
-        h->r_hit.ensure(n * r.row);
-        h->r_hit2.ensure(n * r.row);
-        h->r_q.ensure(n * r.qrow);
-    } catch (const HipError&) {
-        (void)hipGetLastError();
-        h->r_hit.free(); h->r_hit2.free(); h->r_q.free();
-        n = 0;
-    }
+    for (; n > 0; n /= 2) try {
+            h->r_hit.ensure(n * r.row);
+            h->r_hit2.ensure(n * r.row);
+            h->r_q.ensure(n * r.qrow);
+            break;
+        } catch (const MemError&) {
+            (void)hipGetLastError();
+            h->drop_record();
+        }
     r.hit = h->r_hit.p;
     r.hit2 = h->r_hit2.p;
     r.q = h->r_q.p;
@@ -734,8 +759,6 @@ void adjoint_wavefront(pt_renderer_s* h, int first_sample, int num_samples, floa
     if (vis_words > static_cast<size_t>(INT32_MAX)) throw ArgError(PT_ERR_OVERFLOW, "too many paths per pass");
     h->a_rad.ensure(w.max_paths);
     h->a_vis.ensure(vis_words);
-    ptd::Record rec = hit_record(h, w);
-    rec.vis = h->a_vis.p;
     const ptd::PathBuf pb = path_buf(h);
     ptd::PathBuf pb2 = pb;
     pb2.rad = h->a_rad.p;
@@ -754,6 +777,8 @@ void adjoint_wavefront(pt_renderer_s* h, int first_sample, int num_samples, floa
     const int D = w.D;
     const size_t ncells = static_cast<size_t>(counter_cells(D)) * ptd::CELL;
     h->counters.ensure(2 * ncells);
+    ptd::Record rec = hit_record(h, w);  // last, from what memory is left
+    rec.vis = h->a_vis.p;
     rec.counts = Cells{h->counters.p, D}.hits(0);
     const Cells cells{h->counters.p + ncells, D};  // the replay's own
     const int cadence = std::max(1, h->opts.compact_every);
@@ -1188,7 +1213,8 @@ int query(pt_handle h, const float* origins, const float* dirs, const float* rea
     lanes.each(parts, [&](ptx::Lane& l, int k) {
         const int m = std::min(n - k * per, per);
         const size_t first = static_cast<size_t>(k) * per, um = static_cast<size_t>(m);
-        HIPCHK(l.ensure_spill((um + 255) / 256 * 256 * static_cast<size_t>(ptd::MAXD - S + 1)));
+        if (l.ensure_spill((um + 255) / 256 * 256 * static_cast<size_t>(ptd::MAXD - S + 1)) != hipSuccess)
+            throw MemError("device memory for a query's traversal stacks");
         int* flag = reinterpret_cast<int*>(l.pinned);  // first line: the overflow flag
         float* in = reinterpret_cast<float*>(l.pinned + 64);
         float* out = in + um * in_words;
@@ -1916,6 +1942,7 @@ static int adjoint_call(pt_handle h, int32_t first_sample, int32_t num_samples, 
         HIPCHK(hipMemcpyAsync(g.data(), h->a_grad.p, ng * sizeof(float), hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipMemcpyAsync(flags, h->a_flags.p, sizeof(flags), hipMemcpyDeviceToHost, h->stream));
         h->resolve_events();
+        if (h->r_hit.n * 16 + h->r_hit2.n * 8 + h->r_q.n * 4 > RECORD_BYTES) h->drop_record();
         h->stats.adjoint_dropped = flags[1];
         if (flags[0]) return Fail(h, PT_ERR_STATE, "adjoint: a path vertex named a material outside the scene's table");
         for (size_t i = 0; i < np; ++i) d_params[i] += g[i];

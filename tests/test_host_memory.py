@@ -1,5 +1,5 @@
-"""What the renderer's host code does with memory: calls where pinned memory
-cannot be had. CPU build over a stand-in HIP runtime."""
+"""What the renderer's host code does with memory: calls where pinned memory or the
+adjoint's record cannot be had. CPU build over a stand-in HIP runtime."""
 import numpy as np
 import pytest
 
@@ -55,3 +55,51 @@ def test_renders_without_pinned_memory(renderer):
     job = dict(camera=sc.camera(), width=20, height=10, spp=2, max_depth=3)
     assert renderer.batch_render([job])[0].shape == (10, 20, 4)
     renderer.adjoint(0, 1, np.zeros((rs.height, rs.width, 3), np.float32))
+
+
+def adjoint_call(r, size, depth):
+    sc, rs = small_instanced()
+    rs.width = rs.height = size
+    rs.max_depth = depth
+    r.upload_scene(sc)
+    r.set_options(options_for(rs, wave_spp=1, compact_every=2))
+    r.set_camera(sc.camera())
+    r.adjoint(0, 1, np.zeros((size, size, 3), np.float32))
+
+
+SIDE = 2400  # 5.8M paths: 184 MB of record per bounce
+EACH = 28 * (SIDE * SIDE + SIDE * SIDE // 7 + 64)
+
+
+def test_record_kept_between_calls_is_bounded(renderer):
+    """16 recorded bounces of 5.8M paths are 2.9 GB; at most 2 GB of them stay."""
+    lib = hostabi.lib()
+    adjoint_call(renderer, SIDE, 0)
+    one = lib.fake_device_used()
+    lib.fake_device_peak()
+    adjoint_call(renderer, SIDE, 15)
+    assert lib.fake_device_peak() - one > 14 * EACH * 0.85
+    assert lib.fake_device_used() - one <= (2 << 30)
+
+
+def test_record_of_fewer_bounces(renderer):
+    """Where 16 bounces cannot be had but 6 can, some are recorded, and a call
+    that needs the room gets it from the record."""
+    lib = hostabi.lib()
+    adjoint_call(renderer, SIDE, 0)
+    one = lib.fake_device_used()
+    limit = one + 6 * EACH
+    lib.fake_device_limit(limit)
+    lib.fake_device_peak()
+    adjoint_call(renderer, SIDE, 15)
+    assert lib.fake_device_peak() - one > 2 * EACH * 0.85
+    kept = lib.fake_device_used()
+    assert kept > one + EACH
+    # a scene whose textures take all but what the record holds
+    texels = (limit - kept) // 4 + (1 << 20)
+    sc, rs = small_instanced()
+    v = sc.view()
+    tex = np.zeros(4 * texels, np.uint8)
+    v.num_textures, v.tex_width, v.tex_height = 1, 1 << 10, (texels >> 10) - 1
+    v.texture_maps = tex.ctypes.data_as(type(v.texture_maps))
+    renderer._check("pt_upload_scene", lib.pt_upload_scene(renderer._h, hostabi.C.byref(v)))
