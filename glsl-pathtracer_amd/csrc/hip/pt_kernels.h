@@ -212,6 +212,7 @@ inline LayoutSizes layout_sizes_here() {
 }
 void launch_env_cdf(hipStream_t s, const float* img, int n, float* cdf, float* total, int* ok, void* scratch);
 void launch_zero_cells(hipStream_t s, int* cells, int n);  // cells 0..n-1, CELL ints apart
+void launch_roll_cells(hipStream_t s, int* cells, int n, const int* from);  // the same, then cell 0 = *from (one of them)
 void launch_fill(hipStream_t s, int* p, int n, int v);
 void launch_query_closest(hipStream_t s, const ptd::DevScene& sc, const ptd::DevOpts& op, const float* o,
                           const float* d, int n, float* t, int* inst, int* tri, int* light, float* uv, int S,

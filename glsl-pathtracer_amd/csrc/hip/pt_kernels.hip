@@ -1494,7 +1494,15 @@ __global__ void __launch_bounds__(ENV_SCAN_THREADS) k_env_scan(float* cdf, int n
 // The counter cells of a pass.
 __global__ void k_zero_cells(int* cells, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) cells[i * CELL] = 0;
+    if (i < n) cells[static_cast<size_t>(i) * CELL] = 0;
+}
+
+// The same between bounces of a pass (one block): the count at `from`, a cell of
+// these, becomes the first.
+__global__ void __launch_bounds__(256) k_roll_cells(int* cells, int n, const int* from) {
+    const int first = *from;
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += blockDim.x) cells[i * CELL] = i == 0 ? first : 0;
 }
 
 __global__ void k_fill_int(int* p, int n, int v) {
@@ -1790,6 +1798,10 @@ void launch_env_cdf(hipStream_t s, const float* img, int n, float* cdf, float* t
 
 void launch_zero_cells(hipStream_t s, int* cells, int n) {
     hipLaunchKernelGGL(k_zero_cells, dim3((n + 63) / 64), dim3(64), 0, s, cells, n);
+}
+
+void launch_roll_cells(hipStream_t s, int* cells, int n, const int* from) {
+    hipLaunchKernelGGL(k_roll_cells, dim3(1), dim3(256), 0, s, cells, n, from);
 }
 
 void launch_fill(hipStream_t s, int* p, int n, int v) {

@@ -425,26 +425,40 @@ void check_ready(pt_renderer_s* h) {
     if (!h->has_cam) throw ArgError(PT_ERR_STATE, "no camera set (pt_set_camera)");
 }
 
-// Counters of one wavefront pass of D bounces (all zeroed per pass), each on a
-// cache line of its own (ptd::CELL):
-//   [0, D+1)            paths entering extend at bounce b
-//   [D+1, 2D+2)         hits entering shade at bounce b
-//   [2D+2, 3D+3)        shadow records of bounce b
-//   [3D+3, 4D+3)        stopped traversals of bounce b
-//   4D+3                the work counter of k_finish
-//   from 4D+4           work counters (ptd::SHARDS each) of the extend, shade,
+// Counters of n staged bounces of a wavefront pass (all zeroed per pass), each on
+// a cache line of its own (ptd::CELL):
+//   [0, n+1)            paths entering extend at bounce b
+//   [n+1, 2n+2)         hits entering shade at bounce b
+//   [2n+2, 3n+3)        shadow records of bounce b
+//   [3n+3, 4n+3)        stopped traversals of bounce b
+//   4n+3                the work counter of k_finish
+//   from 4n+4           work counters (ptd::SHARDS each) of the extend, shade,
 //                       shadow and resume stages of bounce b
-int counter_cells(int D) { return 4 * D + 4 + 4 * D * ptd::SHARDS; }
+// A pass that stages more bounces than CELL_BOUNCES uses the cells again and
+// again: before bounces CELL_BOUNCES, 2 CELL_BOUNCES, ... they are cleared and
+// the count of the paths that enter moves to the first (launch_roll_cells), so
+// that a depth of a million does not take 4.6 GB of counters.
+constexpr int CELL_BOUNCES = 256;
+int counter_cells(int n) { return 4 * n + 4 + 4 * n * ptd::SHARDS; }
 struct Cells {
     int* base;
-    int D;
+    int n;
     int* at(int i) const { return base + static_cast<size_t>(i) * ptd::CELL; }
     int* paths(int b) const { return at(b); }
-    int* hits(int b) const { return at(D + 1 + b); }
-    int* shadows(int b) const { return at(2 * (D + 1) + b); }
-    int* conts(int b) const { return at(3 * (D + 1) + b); }
-    int* finish() const { return at(4 * D + 3); }
-    int* work(int b, int stage) const { return at(4 * D + 4 + (4 * b + stage) * ptd::SHARDS); }
+    int* hits(int b) const { return at(n + 1 + b); }
+    int* shadows(int b) const { return at(2 * (n + 1) + b); }
+    int* conts(int b) const { return at(3 * (n + 1) + b); }
+    int* finish() const { return at(4 * n + 3); }
+    int* work(int b, int stage) const { return at(4 * n + 4 + (4 * b + stage) * ptd::SHARDS); }
+    // Index of bounce b's cells; c_ext: the count of the paths that enter it.
+    int bounce(int b, int*& c_ext, hipStream_t s) const {
+        const int i = b % CELL_BOUNCES;
+        if (b > 0 && i == 0) {
+            ptk::launch_roll_cells(s, base, counter_cells(n), c_ext);
+            c_ext = paths(0);
+        }
+        return i;
+    }
 };
 
 // k_finish takes a pass over from the stages at the first later bounce whose
@@ -550,6 +564,7 @@ const int2* tile_entries(pt_renderer_s* h, const DevOpts& op, const ptd::JobDev*
 // spp_pass samples of every pixel.
 struct Wavefront {
     int npix, spp_pass, D, bs, S, b_ext, b_sha, b_sdw;
+    int nb;             // bounces that the stages run (0: k_finish runs the passes whole)
     bool cw, inline_nee;
     size_t max_paths;
     int cap;            // extend_cap of later bounces (0: off)
@@ -578,7 +593,8 @@ Wavefront wavefront_setup(pt_renderer_s* h, const DevOpts& op, int num_samples, 
     if (staged && !w.inline_nee) ensure_shadow(h, max_paths);
     // Bounce iterations: maxDepth + 1 closest hits; alpha pass-through repeats a depth.
     w.D = op.max_depth + 1 + ((op.flags & ptd::OPT_ALPHA_TEST) ? 64 : 0);
-    h->counters.ensure(static_cast<size_t>(counter_cells(w.D)) * ptd::CELL);
+    w.nb = !staged ? 0 : w.fin.leave > 0 ? std::min(w.D, FINISH_BOUNCES) : w.D;
+    h->counters.ensure(static_cast<size_t>(counter_cells(std::min(w.nb, CELL_BOUNCES))) * ptd::CELL);
     h->ensure_misc();
     w.bs = h->block_size();
     w.S = h->stack_S();
@@ -596,31 +612,44 @@ Wavefront wavefront_setup(pt_renderer_s* h, const DevOpts& op, int num_samples, 
     return w;
 }
 
-// Where the hits of bounce b go: the record's row, or the path buffer's place.
+// Where the hits of bounce b go: the record's row, or the path buffer's place and
+// the pass's count.
 struct HitPlace {
     ptd::PathBuf pb;
     int* q;
+    int* count;
 };
-HitPlace hit_place(pt_renderer_s* h, const ptd::PathBuf& pb, const ptd::Record* rec, int b) {
-    HitPlace p{pb, h->hq.p};
+HitPlace hit_place(pt_renderer_s* h, const ptd::PathBuf& pb, const ptd::Record* rec, int b, int* count) {
+    HitPlace p{pb, h->hq.p, count};
     if (rec && b < rec->bounces) {
         p.pb.hit = rec->hit + static_cast<size_t>(b) * rec->row;
         p.pb.hit2 = rec->hit2 + static_cast<size_t>(b) * rec->row;
         p.q = rec->q + static_cast<size_t>(b) * rec->qrow;
+        p.count = rec->counts + static_cast<size_t>(b) * ptd::CELL;
     }
     return p;
+}
+
+// Instrumented runs: adds the hits per bounce of bounces [first, first + n).
+void count_hits(pt_renderer_s* h, const Cells& cells, int first, int n) {
+    std::vector<int> hits(n);
+    HIPCHK(hipMemcpy2DAsync(hits.data(), sizeof(int), cells.hits(0), ptd::CELL * sizeof(int), sizeof(int), n,
+                            hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
+    for (int b = 0; b < n; ++b) h->stats.bounce_hits[std::min(first + b, 15)] += hits[b];
 }
 
 // Every bounce of one pass (paths [0, npaths), samples fs...): extend, shade,
 // shadow per bounce. rec (the adjoint's primal pass, else null): what the replay
 // takes from it; hits of the bounces beyond rec->bounces go to the usual buffers.
+// The counters of the pass (and the record's) are zero.
 void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const ptd::PathBuf& pb0,
                  const ptd::ShadowBuf& sb, int npaths, int fs, const ptd::Record* rec) {
     hipStream_t s = h->stream;
     const int D = w.D;
-    const Cells cells{h->counters.p, D};
+    const Cells cells{h->counters.p, std::min(w.nb, CELL_BOUNCES)};
+    const bool count = w.cw && !rec;  // hits per bounce
     hipEvent_t ev;
-    ptk::launch_zero_cells(s, cells.base, counter_cells(D));
     int* qin = h->qa.p;
     int* qout = h->qb.p;
     int* c_ext = cells.paths(0);  // count of the current extend queue
@@ -632,38 +661,39 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
                            refill_lanes(h, w.inline_nee, npaths), rec);
         h->stage_end(PT_STAGE_PLAIN, ev);
     };
-    if (w.fin.whole > 0 && w.max_paths <= static_cast<size_t>(w.fin.whole)) {
+    if (w.nb == 0) {
         finish(true, 0);
         return;
     }
-    const int nb = w.fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
-    for (int b = 0; b < nb; ++b) {
-        const HitPlace hp = hit_place(h, pb0, rec, b);
-        int* c_hit = cells.hits(b);
-        int* c_sh = cells.shadows(b);
+    for (int b = 0; b < w.nb; ++b) {
+        if (count && b > 0 && b % CELL_BOUNCES == 0) count_hits(h, cells, b - CELL_BOUNCES, CELL_BOUNCES);
+        const int k = cells.bounce(b, c_ext, s);
+        const HitPlace hp = hit_place(h, pb0, rec, b, cells.hits(k));
+        int* c_hit = hp.count;
+        int* c_sh = cells.shadows(k);
         const bool primary = b == 0;
         // bounce 0 always compacts (its input is the implicit slot range);
         // later bounces compact every `cadence`-th time, otherwise the next
         // extend re-reads this queue and skips ended paths.
         const bool compact = primary || (b % cadence) == 0;
-        int* c_next = compact ? cells.paths(b + 1) : c_ext;
+        int* c_next = compact ? cells.paths(k + 1) : c_ext;
         const bool capped = w.cap > 0 && !primary;
         h->stage_begin(PT_STAGE_EXTEND, ev);
         ptk::launch_extend(s, w.b_ext, w.bs, h->sc, op, hp.pb, primary, qin, c_ext, npaths, w.npix, fs, hp.q, c_hit,
-                           cells.work(b, 0), w.S, h->spill.p, h->work_counts.p, h->ovf.p, w.cw, capped ? w.cap : 0, &w.cb,
-                           cells.conts(b), w.fin.leave, w.tiles);
+                           cells.work(k, 0), w.S, h->spill.p, h->work_counts.p, h->ovf.p, w.cw, capped ? w.cap : 0, &w.cb,
+                           cells.conts(k), w.fin.leave, w.tiles);
         if (capped)
-            ptk::launch_extend_resume(s, w.b_ext, w.bs, h->sc, op, hp.pb, w.cb, cells.conts(b), hp.q, cells.work(b, 3), w.S,
+            ptk::launch_extend_resume(s, w.b_ext, w.bs, h->sc, op, hp.pb, w.cb, cells.conts(k), hp.q, cells.work(k, 3), w.S,
                                       h->spill.p, h->ovf.p);
         h->stage_end(PT_STAGE_EXTEND, ev);
         h->stage_begin(PT_STAGE_SHADE, ev);
         ptk::launch_shade(s, w.b_sha, w.bs, h->sc, op, hp.pb, sb, nullptr, primary, w.inline_nee, hp.q, c_hit, w.npix,
-                          fs, qout, c_next, c_sh, cells.work(b, 1), compact, w.S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
+                          fs, qout, c_next, c_sh, cells.work(k, 1), compact, w.S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
         h->stage_end(PT_STAGE_SHADE, ev);
         if (!w.inline_nee) {
             unsigned* vb = rec ? rec->vis + static_cast<size_t>(b / ptd::VIS_BOUNCES_PER_WORD) * w.max_paths : nullptr;
             h->stage_begin(PT_STAGE_SHADOW, ev);
-            ptk::launch_shadow(s, w.b_sdw, w.bs, h->sc, op, hp.pb, sb, c_sh, cells.work(b, 2), w.S, h->spill.p,
+            ptk::launch_shadow(s, w.b_sdw, w.bs, h->sc, op, hp.pb, sb, c_sh, cells.work(k, 2), w.S, h->spill.p,
                                h->work_counts.p + 8, h->ovf.p, w.cw, vb, 2 * (b % ptd::VIS_BOUNCES_PER_WORD));
             h->stage_end(PT_STAGE_SHADOW, ev);
         }
@@ -672,7 +702,11 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
             c_ext = c_next;
         }
     }
-    if (w.fin.leave > 0) finish(false, nb);
+    if (count) {
+        const int first = (w.nb - 1) / CELL_BOUNCES * CELL_BOUNCES;
+        count_hits(h, cells, first, w.nb - first);
+    }
+    if (w.fin.leave > 0) finish(false, w.nb);
 }
 
 void render_wavefront(pt_renderer_s* h, int first_sample, int num_samples) {
@@ -682,20 +716,13 @@ void render_wavefront(pt_renderer_s* h, int first_sample, int num_samples) {
     const ptd::ShadowBuf sb = shadow_buf(h);
     for (int s0 = 0; s0 < num_samples; s0 += w.spp_pass) {
         const int ns = std::min(w.spp_pass, num_samples - s0);
+        ptk::launch_zero_cells(h->stream, h->counters.p, counter_cells(std::min(w.nb, CELL_BOUNCES)));
         run_bounces(h, op, w, pb, sb, w.npix * ns, first_sample + s0, nullptr);
         hipEvent_t ev;
         h->stage_begin(PT_STAGE_ACCUM, ev);
         ptk::launch_accum(h->stream, op, pb, h->accum.p, w.npix, ns);
         h->stage_end(PT_STAGE_ACCUM, ev);
         HIPCHK(hipGetLastError());
-        if (w.cw) {  // instrumented runs: hits per bounce of this pass (the counters are reused per pass)
-            std::vector<int> hits(w.D);
-            const Cells cells{h->counters.p, w.D};
-            HIPCHK(hipMemcpy2DAsync(hits.data(), sizeof(int), cells.hits(0), ptd::CELL * sizeof(int), sizeof(int), w.D,
-                                    hipMemcpyDeviceToHost, h->stream));
-            HIPCHK(hipStreamSynchronize(h->stream));
-            for (int b = 0; b < w.D; ++b) h->stats.bounce_hits[std::min(b, 15)] += hits[b];
-        }
     }
 }
 
@@ -711,13 +738,16 @@ void render_wavefront(pt_renderer_s* h, int first_sample, int num_samples) {
 // bounces recorded, 57 with all.
 constexpr int RECORD_BOUNCES = 16;
 constexpr size_t RECORD_BYTES = size_t{2} << 30;
+size_t record_bounces(const pt_renderer_s* h, const Wavefront& w) {
+    const size_t each = 28 * ptd::queue_room(w.max_paths);
+    const size_t n = std::max(static_cast<size_t>(RECORD_BOUNCES), RECORD_BYTES / each);
+    return std::min({n, static_cast<size_t>(w.D), h->device_bytes / 16 / each});
+}
 ptd::Record hit_record(pt_renderer_s* h, const Wavefront& w) {
     ptd::Record r{};
     r.row = w.max_paths;
     r.qrow = ptd::queue_room(w.max_paths);
-    const size_t each = 28 * r.qrow;
-    size_t n = std::max(static_cast<size_t>(RECORD_BOUNCES), RECORD_BYTES / each);
-    n = std::min({n, static_cast<size_t>(w.D), h->device_bytes / 16 / each});
+    size_t n = record_bounces(h, w);
     for (; n > 0; n /= 2) try {
             h->r_hit.ensure(n * r.row);
             h->r_hit2.ensure(n * r.row);
@@ -775,43 +805,46 @@ void adjoint_wavefront(pt_renderer_s* h, int first_sample, int num_samples, floa
     rb.lds = lds ? 1 : 0;
     hipStream_t s = h->stream;
     const int D = w.D;
-    const size_t ncells = static_cast<size_t>(counter_cells(D)) * ptd::CELL;
-    h->counters.ensure(2 * ncells);
+    // the primal pass's counters, the replay's own and the record's
+    const int n1 = counter_cells(std::min(w.nb, CELL_BOUNCES)), win = std::min(D, CELL_BOUNCES), n2 = counter_cells(win);
+    const size_t ncells = static_cast<size_t>(n1) + n2 + record_bounces(h, w);
+    h->counters.ensure(ncells * ptd::CELL);
     ptd::Record rec = hit_record(h, w);  // last, from what memory is left
     rec.vis = h->a_vis.p;
-    rec.counts = Cells{h->counters.p, D}.hits(0);
-    const Cells cells{h->counters.p + ncells, D};  // the replay's own
+    const Cells cells{h->counters.p + static_cast<size_t>(n1) * ptd::CELL, win};
+    rec.counts = cells.base + static_cast<size_t>(n2) * ptd::CELL;
     const int cadence = std::max(1, h->opts.compact_every);
     for (int s0 = 0; s0 < num_samples; s0 += w.spp_pass) {
         const int ns = std::min(w.spp_pass, num_samples - s0);
         const int npaths = w.npix * ns, fs = first_sample + s0;
         ptk::launch_fill(s, reinterpret_cast<int*>(h->a_vis.p), static_cast<int>(vis_words), 0);
+        ptk::launch_zero_cells(s, h->counters.p, n1 + n2 + rec.bounces);
         run_bounces(h, op, w, pb, sb, npaths, fs, &rec);
         // replay: beyond the recorded bounces the extend stage of the forward
         // renderer, then the replay stage
-        ptk::launch_zero_cells(s, cells.base, counter_cells(D));
         int* qin = h->qa.p;
         int* qout = h->qb.p;
         int* c_ext = cells.paths(0);
         hipEvent_t ev;
         for (int b = 0; b < D; ++b) {
-            const HitPlace hp = hit_place(h, pb2, &rec, b);
+            const int k = cells.bounce(b, c_ext, s);
+            const HitPlace hp = hit_place(h, pb2, &rec, b, cells.hits(k));
             const bool recorded = b < rec.bounces;
-            int* c_hit = recorded ? rec.counts + static_cast<size_t>(b) * ptd::CELL : cells.hits(b);
+            int* c_hit = hp.count;
             const bool primary = b == 0;
             const bool compact = primary || (b % cadence) == 0;
-            int* c_next = compact ? cells.paths(b + 1) : c_ext;
+            int* c_next = compact ? cells.paths(k + 1) : c_ext;
             if (!recorded) {
                 h->stage_begin(PT_STAGE_EXTEND, ev);
                 ptk::launch_extend(s, w.b_ext, w.bs, h->sc, op, pb2, primary, qin, c_ext, npaths, w.npix, fs, h->hq.p,
-                                   c_hit, cells.work(b, 0), w.S, h->spill.p, h->work_counts.p, h->ovf.p, false, 0, nullptr,
+                                   c_hit, cells.work(k, 0), w.S, h->spill.p, h->work_counts.p, h->ovf.p, false, 0, nullptr,
                                    nullptr, 0, w.tiles);
                 h->stage_end(PT_STAGE_EXTEND, ev);
             }
             rb.vis = h->a_vis.p + static_cast<size_t>(b / ptd::VIS_BOUNCES_PER_WORD) * w.max_paths;
             h->stage_begin(PT_STAGE_ADJOINT, ev);
             ptk::launch_replay_shade(s, b_rep, w.bs, h->sc, op, hp.pb, primary, hp.q, c_hit, w.npix, fs, qout, c_next,
-                                     cells.work(b, 1), compact, rb, 2 * (b % ptd::VIS_BOUNCES_PER_WORD));
+                                     cells.work(k, 1), compact, rb, 2 * (b % ptd::VIS_BOUNCES_PER_WORD));
             h->stage_end(PT_STAGE_ADJOINT, ev);
             if (compact) {
                 std::swap(qin, qout);
@@ -1002,7 +1035,8 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     if (!whole) ensure_paths(h, max_paths);
     if (!whole && !inl) ensure_shadow(h, max_paths);
     const int D = P.max_depth + 1 + ((op.flags & ptd::OPT_ALPHA_TEST) ? 64 : 0);
-    const int ncells = counter_cells(D);
+    const int nb = whole ? 0 : fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;  // bounces that the stages run
+    const int ncells = counter_cells(std::min(nb, CELL_BOUNCES));
     h->counters.ensure(static_cast<size_t>(ncells) * ptd::CELL);
     h->ensure_misc();
     const int bs = h->block_size(), S = h->stack_S();
@@ -1027,7 +1061,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
     const ptd::PathBuf pb = path_buf(h);
     const ptd::ShadowBuf sb = shadow_buf(h);
     const int2* tiles = tile_entries(h, op, h->b_jobs.p, n, static_cast<int>(P.items / 64), P.max_side, P.samples);
-    const Cells cells{h->counters.p, D};
+    const Cells cells{h->counters.p, std::min(nb, CELL_BOUNCES)};
     const int cadence = std::max(1, h->opts.compact_every);
     const bool graph = h->opts.use_graph != 0;
 
@@ -1051,33 +1085,33 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
                                    refill_lanes(h, inl, P.max_paths));
             });
         };
-        const int nb = whole ? 0 : fin.leave > 0 ? std::min(D, FINISH_BOUNCES) : D;
         if (whole) finish(true, 0);
         for (int b = 0; b < nb; ++b) {
-            int* c_hit = cells.hits(b);
-            int* c_sh = cells.shadows(b);
+            const int k = cells.bounce(b, c_ext, s);
+            int* c_hit = cells.hits(k);
+            int* c_sh = cells.shadows(k);
             const bool primary = b == 0;
             const bool compact = primary || (b % cadence) == 0;
-            int* c_next = compact ? cells.paths(b + 1) : c_ext;
+            int* c_next = compact ? cells.paths(k + 1) : c_ext;
             stage(PT_STAGE_EXTEND, [&] {
                 if (primary) {
-                    ptk::launch_extend_batch(s, b_ext, bs, h->sc, op, pb, bb, h->hq.p, c_hit, cells.work(b, 0), S, h->spill.p, h->ovf.p,
+                    ptk::launch_extend_batch(s, b_ext, bs, h->sc, op, pb, bb, h->hq.p, c_hit, cells.work(k, 0), S, h->spill.p, h->ovf.p,
                                              tiles);
                 } else {
-                    ptk::launch_extend(s, b_ext, bs, h->sc, op, pb, false, qin, c_ext, 0, 0, 0, h->hq.p, c_hit, cells.work(b, 0), S,
-                                       h->spill.p, h->work_counts.p, h->ovf.p, false, cap, &cb, cells.conts(b), fin.leave);
+                    ptk::launch_extend(s, b_ext, bs, h->sc, op, pb, false, qin, c_ext, 0, 0, 0, h->hq.p, c_hit, cells.work(k, 0), S,
+                                       h->spill.p, h->work_counts.p, h->ovf.p, false, cap, &cb, cells.conts(k), fin.leave);
                     if (cap > 0)
-                        ptk::launch_extend_resume(s, b_ext, bs, h->sc, op, pb, cb, cells.conts(b), h->hq.p, cells.work(b, 3),
+                        ptk::launch_extend_resume(s, b_ext, bs, h->sc, op, pb, cb, cells.conts(k), h->hq.p, cells.work(k, 3),
                                                   S, h->spill.p, h->ovf.p);
                 }
             });
             stage(PT_STAGE_SHADE, [&] {
                 ptk::launch_shade(s, b_sha, bs, h->sc, op, pb, sb, &bb, primary, inl, h->hq.p, c_hit, 0, 0, qout,
-                                  c_next, c_sh, cells.work(b, 1), compact, S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
+                                  c_next, c_sh, cells.work(k, 1), compact, S, h->spill.p, h->work_counts.p + 8, h->ovf.p);
             });
             if (!inl)
                 stage(PT_STAGE_SHADOW, [&] {
-                    ptk::launch_shadow(s, b_sdw, bs, h->sc, op, pb, sb, c_sh, cells.work(b, 2), S, h->spill.p,
+                    ptk::launch_shadow(s, b_sdw, bs, h->sc, op, pb, sb, c_sh, cells.work(k, 2), S, h->spill.p,
                                        h->work_counts.p + 8, h->ovf.p, false);
                 });
             if (compact) {

@@ -71,6 +71,11 @@ void launch_env_cdf(hipStream_t, const float*, int, float*, float*, int*, void*)
 void launch_zero_cells(hipStream_t, int* cells, int n) {
     for (int i = 0; i < n; ++i) cells[static_cast<size_t>(i) * CELL] = 0;
 }
+void launch_roll_cells(hipStream_t s, int* cells, int n, const int* from) {
+    const int first = *from;
+    launch_zero_cells(s, cells, n);
+    cells[0] = first;
+}
 void launch_fill(hipStream_t, int* p, int n, int v) { std::fill_n(p, n, v); }
 void launch_tonemap(hipStream_t, const float4*, int, int, float, int, int, int, int, const float*, uchar4*) {}
 void launch_tlas_rebuild(hipStream_t, const TlasBuild&) {}

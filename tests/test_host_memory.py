@@ -103,3 +103,32 @@ def test_record_of_fewer_bounces(renderer):
     v.num_textures, v.tex_width, v.tex_height = 1, 1 << 10, (texels >> 10) - 1
     v.texture_maps = tex.ctypes.data_as(type(v.texture_maps))
     renderer._check("pt_upload_scene", lib.pt_upload_scene(renderer._h, hostabi.C.byref(v)))
+
+
+@pytest.mark.parametrize("kind", ["whole", "staged", "counted", "batch", "batch staged", "adjoint", "adjoint staged"])
+def test_depth_takes_little_memory(renderer, kind):
+    """The counters of a pass are not held for every bounce that a depth allows
+    (paths end by Russian roulette long before)."""
+    lib = hostabi.lib()
+    used = []
+    for depth in (8, 20000):
+        sc, rs = small_instanced()
+        rs.max_depth = depth
+        renderer.upload_scene(sc)
+        renderer.set_options(options_for(rs, compact_every=2 if "staged" in kind else 1, count_work=kind == "counted"))
+        renderer.set_camera(sc.camera())
+        lib.fake_device_peak()
+        if "batch" in kind:
+            renderer.batch_render([dict(camera=sc.camera(), width=64, height=64, spp=2, max_depth=depth)])
+        elif "adjoint" in kind:
+            if depth > 8:  # the record and the visibility words, 28 bytes and two bits per path and bounce, aside
+                rs.width = rs.height = 1
+                renderer.set_options(options_for(rs, compact_every=2 if "staged" in kind else 1, wave_spp=1))
+            renderer.adjoint(0, 1, np.zeros((rs.height, rs.width, 3), np.float32))
+        else:
+            renderer.clear()
+            renderer.render(0, 2)
+            renderer.synchronize()
+        used.append(lib.fake_device_peak())
+    room = 28 * 150 * 20000 + 128 * 20001 if "adjoint" in kind else 0
+    assert used[1] - used[0] < (2 << 20) + room
