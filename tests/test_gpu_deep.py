@@ -1,5 +1,6 @@
 """Deep passes in a closed room without Russian roulette, where paths go on to
-the last bounce: passes that use their counters several times over give the
+the last bounce: passes that use their counters several times over, and the
+takeover by k_finish after 40 bounces with more paths than its grid, give the
 plain form's image bit for bit."""
 import numpy as np
 import pytest
@@ -84,3 +85,41 @@ def test_counters_used_again_in_the_adjoint(renderer):
     for other in g[1:]:
         # 2e5 terms per sum in fp32: 2e5^0.5 * 6e-8 with threefold cancellation
         assert np.abs(g[0] - other).max() <= 1e-4 * np.abs(g[0]).max()
+
+
+@pytest.mark.parametrize("depth", [39, 40, 45, 60])
+@pytest.mark.parametrize("kind", ["frame", "batch", "adjoint"])
+def test_takeover_of_many_paths(renderer, kind, depth):
+    """3.1M paths in a pass, staged up to bounce 40 (nearly all of them alive
+    there, many times what the grid of k_finish holds at once) and taken over then."""
+    size, spp = (1200, 864), 3
+    sc, rs = closed_room(*size, spp, depth)
+    renderer.upload_scene(sc)
+    if kind == "adjoint":
+        dl = np.random.default_rng(5).normal(size=(size[1], size[0], 3)).astype(np.float32)
+        g = []
+        for cadence in (1, 2):
+            renderer.set_options(options_for(rs, wave_spp=spp, compact_every=cadence))
+            renderer.set_camera(sc.camera())
+            g.append(renderer.adjoint(0, spp, dl).astype(np.float64))
+        assert np.abs(g[0]).max() > 0
+        # up to 1e8 terms per sum in fp32, summed per block first: 1e4 of them in
+        # a row at most, 1e4 * 6e-8 if their roundings all agreed
+        assert np.abs(g[0] - g[1]).max() <= 6e-4 * np.abs(g[1]).max()
+        return
+    jobs = [dict(camera=sc.camera(), width=size[0], height=size[1], spp=spp, max_depth=depth)]
+    if kind == "frame":
+        want = image(renderer, sc, rs, PT_MODE_PLAIN, spp)
+    else:
+        renderer.set_options(options_for(rs, mode=PT_MODE_PLAIN))
+        want, = renderer.batch_render(jobs)
+    for cadence in (1, 2):
+        if kind == "frame":
+            renderer.reset_stats()
+            got = image(renderer, sc, rs, PT_MODE_WAVEFRONT, spp, wave_spp=spp, compact_every=cadence)
+            assert renderer.stats()["ms_stage"]["extend"] > 0
+        else:
+            renderer.set_options(options_for(rs, mode=PT_MODE_WAVEFRONT, wave_spp=spp, compact_every=cadence,
+                                             use_graph=cadence - 1))
+            got, = renderer.batch_render(jobs)
+        assert np.array_equal(got, want)
