@@ -152,7 +152,7 @@ struct Relayout {
     std::vector<int> inst_blas4_ref;        // each instance's four-wide BLAS root reference
     int tlas4_base = 0;                     // first four-wide TLAS entry in wide.nodes (at least max(n - 1, 1) follow)
     int root4 = 0;                          // four-wide TLAS root reference
-    long long traced_tris = 0;              // triangles over all instances (an estimate)
+    long long traced_tris = 0;              // triangles over all instances
     float local_max = 0.f;                  // local_reach of inst_local
     bool far = false;                       // a TLAS box or a BLAS root's box has a far plane
     // The TLAS as the device rebuild writes it: one instance per leaf, every
@@ -179,12 +179,15 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
     if (top < 0 || top >= num_nodes) throw ArgError(PT_ERR_INVALID_ARG, "top_level_index out of range");
     st.push_back(top);
     std::vector<char> blas_seen(num_nodes, 0);
+    std::unordered_map<int, long long> blas_tris;  // triangles of each BLAS, by its root
+    long long* tris = nullptr;                     // of the BLAS walked: its nodes follow its root
     while (!st.empty()) {
         int i = st.back();
         st.pop_back();
         if (i < 0 || i >= num_nodes) throw ArgError(PT_ERR_INVALID_ARG, "node child index out of range");
         if (reach[i]) throw ArgError(PT_ERR_INVALID_ARG, "node reachable twice (not a tree)");
         reach[i] = 1;
+        if (blas_seen[i]) tris = &blas_tris[i];
         int k = kind(i);
         if (k == 0) {
             st.push_back(as_int(flat[i].LRLeaf[0]));
@@ -204,6 +207,7 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
             if (count < 1 || count > 3) throw ArgError(PT_ERR_UNSUPPORTED, "BLAS leaves must hold 1..3 triangles");
             if (first < 0 || first + count > num_tris) throw ArgError(PT_ERR_INVALID_ARG, "BLAS leaf triangle range out of bounds");
             if (first >= (1 << 28)) throw ArgError(PT_ERR_UNSUPPORTED, "too many triangles for the leaf encoding");
+            if (tris) *tris += count;
         }
     }
     int n = 0;
@@ -234,6 +238,7 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
             const int root = as_int(flat[i].LRLeaf[0]);
             R.inst_blas_ref[inst] = ref_of(root);
             R.root_ref[root] = R.inst_blas_ref[inst];
+            R.traced_tris += blas_tris[root];
             R.inst_material[inst] = as_int(flat[i].LRLeaf[1]);
             for (int j = 0; j < 3; ++j) {
                 R.inst_local[6 * inst + j] = flat[root].bboxmin[j];
@@ -269,14 +274,6 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
         R.tlas_rebuildable = ok && leaves == num_instances && internal == num_instances - 1 && base + internal == n;
         R.tlas_base = base;
     }
-    {
-        // Triangles below every node, children first: the reference's trees are
-        // in preorder (another order only makes the estimate smaller).
-        std::vector<int> below(R.nodes.size(), 0);
-        auto tris_of = [&](int ref) { return ref < 0 ? (-1 - ref) & 3 : below[ref]; };
-        for (int i = n - 1; i >= 0; --i) below[i] = tris_of(R.nodes[i].d.x) + tris_of(R.nodes[i].d.y);
-        for (int i = 0; i < num_instances; ++i) R.traced_tris += tris_of(R.inst_blas_ref[i]);
-    }
     R.local_max = local_reach(R.inst_local);
     R.far = R.local_max > FAR_PLANE;
     for (st.assign(1, R.root); !st.empty() && !R.far;) {  // the inner TLAS nodes
@@ -288,6 +285,7 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
         st.push_back(R.nodes[r].d.y);
     }
     R.inst_blas4_ref.assign(num_instances, 0);
+    R.wide.nodes.reserve(R.nodes.size() + std::max(num_instances, 1));
     for (int i = 0; i < num_instances; ++i) {
         collapse4_root(R.nodes, R.inst_blas_ref[i], R.wide);
         R.inst_blas4_ref[i] = R.wide.root4[R.inst_blas_ref[i]];
