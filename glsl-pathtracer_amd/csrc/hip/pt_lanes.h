@@ -27,7 +27,7 @@ namespace ptx {
 constexpr size_t LANE_PINNED = size_t{4} << 20;  // pinned bytes of a lane,
 constexpr size_t LANE_SMALL = size_t{64} << 10;  // or these (4 MB take 0.1 ms to pin, 0.1 to give back)
 constexpr int LANES_PER_CALL = 8;
-constexpr size_t POOL_LANES = 16;
+constexpr int POOL_LANES = 16;
 
 struct Lane {
     int device = 0;
@@ -81,12 +81,14 @@ public:
         ++users_;
     }
     void drop_user() {
-        std::vector<Lane*> gone;
+        Lane* gone[POOL_LANES];
+        int n = 0;
         {
             std::lock_guard<std::mutex> g(m_);
-            if (--users_ == 0) gone.swap(idle_);
+            if (--users_ == 0)
+                while (idle_n_ > 0) gone[n++] = idle_[--idle_n_];
         }
-        for (Lane* l : gone) discard(l);
+        for (int i = 0; i < n; ++i) discard(gone[i]);
     }
     // An idle lane of the device or a new one, with `bytes` of pinned memory; null
     // where that cannot be had.
@@ -94,10 +96,11 @@ public:
         Lane* l = nullptr;
         {
             std::lock_guard<std::mutex> g(m_);
-            for (size_t i = idle_.size(); i-- > 0 && !l;)
+            for (int i = idle_n_; i-- > 0 && !l;)
                 if (idle_[i]->device == device) {
                     l = idle_[i];
-                    idle_.erase(idle_.begin() + static_cast<std::ptrdiff_t>(i));
+                    std::copy(idle_ + i + 1, idle_ + idle_n_, idle_ + i);
+                    --idle_n_;
                 }
         }
         const bool made = !l;
@@ -112,8 +115,8 @@ public:
     void give(Lane* l) {
         {
             std::lock_guard<std::mutex> g(m_);
-            if (users_ > 0 && idle_.size() < POOL_LANES) {
-                idle_.push_back(l);
+            if (users_ > 0 && idle_n_ < POOL_LANES) {
+                idle_[idle_n_++] = l;
                 return;
             }
         }
@@ -129,7 +132,8 @@ private:
         (void)hipSetDevice(current);
     }
     std::mutex m_;
-    std::vector<Lane*> idle_;
+    Lane* idle_[POOL_LANES];  // no container: a lane is given back where nothing may throw
+    int idle_n_ = 0;
     int users_ = 0;
 };
 
@@ -140,19 +144,19 @@ public:
         for (int i = 0; i < std::min(want, LANES_PER_CALL); ++i) {
             Lane* l = Pool::get().take(device, bytes);
             if (!l) break;
-            l_.push_back(l);
+            l_[n_++] = l;
         }
     }
     Lanes(const Lanes&) = delete;
     Lanes& operator=(const Lanes&) = delete;
     ~Lanes() {
-        for (Lane* l : l_) {
-            (void)hipStreamSynchronize(l->stream);  // nothing in flight on a lane that is given back
-            Pool::get().give(l);
+        for (int i = 0; i < n_; ++i) {
+            (void)hipStreamSynchronize(l_[i]->stream);  // nothing in flight on a lane that is given back
+            Pool::get().give(l_[i]);
         }
     }
-    int size() const { return static_cast<int>(l_.size()); }
-    Lane& operator[](int i) { return *l_[static_cast<size_t>(i)]; }
+    int size() const { return n_; }
+    Lane& operator[](int i) { return *l_[i]; }
 
     // part(lane, k) for k = 0..n-1, the lanes on threads of their own taking
     // the next part each; the first error ends it and is thrown here.
@@ -186,7 +190,8 @@ public:
     }
 
 private:
-    std::vector<Lane*> l_;
+    Lane* l_[LANES_PER_CALL];
+    int n_ = 0;
 };
 
 // Touches the pages of [p, p + n) (values kept) while `busy` says the device is

@@ -10,10 +10,11 @@
 #include "pt_path.h"
 
 namespace fake {
-thread_local bool no_host_memory = false;
+thread_local long until_failure = -1;  // allocations of this thread before the one that fails (-1: none does)
 }
 void* operator new(size_t n) {
-    void* p = fake::no_host_memory ? nullptr : std::malloc(n ? n : 1);
+    const bool fail = fake::until_failure >= 0 && fake::until_failure-- == 0;
+    void* p = fail ? nullptr : std::malloc(n ? n : 1);
     if (!p) throw std::bad_alloc();
     return p;
 }
@@ -30,6 +31,8 @@ size_t fake_device_peak() {
     return p;
 }
 void fake_refuse_pinned(int on) { fake::state().refuse_pinned = on != 0; }
+void fake_fail_new(long after) { fake::until_failure = after; }
+long fake_fail_new_left() { return fake::until_failure; }
 int fake_pinned() { return fake::state().pinned; }
 }
 

@@ -1,10 +1,15 @@
 """What the renderer's host code does with memory: calls where pinned memory or the
 adjoint's record cannot be had. CPU build over a stand-in HIP runtime."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 import hostabi
 from common import random_dirs, small_instanced
+from glslpt._capi import PtError
 from glslpt.renderer import options_for
 
 
@@ -132,3 +137,65 @@ def test_depth_takes_little_memory(renderer, kind):
         used.append(lib.fake_device_peak())
     room = 28 * 150 * 20000 + 128 * 20001 if "adjoint" in kind else 0
     assert used[1] - used[0] < (2 << 20) + room
+
+
+CALLS = {
+    "upload": lambda r, sc, rs, q: r.upload_scene(sc),
+    "closest 49": lambda r, sc, rs, q: r.closest_hit(q[0][:49], q[1][:49]),
+    "closest 140000": lambda r, sc, rs, q: r.closest_hit(*q[:2]),
+    "any 140000": lambda r, sc, rs, q: r.any_hit(*q),
+    "render": lambda r, sc, rs, q: (r.render(0, 2), r.synchronize()),
+    "image": lambda r, sc, rs, q: r.read_accum(),
+    "batch": lambda r, sc, rs, q: r.batch_render(
+        [dict(camera=sc.camera(), width=600 + k, height=500, spp=2, max_depth=3) for k in range(3)]),
+    "adjoint": lambda r, sc, rs, q: r.adjoint(0, 1, np.zeros((rs.height, rs.width, 3), np.float32)),
+}
+
+
+def sweep(name):
+    """Every host allocation of a call fails once: the call reports it, or does
+    without, and the next one runs."""
+    lib = hostabi.lib()
+    lib.fake_fail_new.argtypes = [hostabi.C.c_long]
+    lib.fake_fail_new.restype = None
+    lib.fake_fail_new_left.restype = hostabi.C.c_long
+    rng = np.random.default_rng(1)
+    n = 140000
+    q = (rng.uniform(-6, 6, (n, 3)).astype(np.float32), random_dirs(rng, n), np.ones(n, np.float32))
+    r = hostabi.HostRenderer()
+    sc, rs = scene(r)
+    rs.width, rs.height = 700, 640  # an image of several parts
+    r.set_options(options_for(rs))
+    r.clear()
+    failed = 0
+    for k in range(100000):
+        lib.fake_fail_new(k)
+        try:
+            CALLS[name](r, sc, rs, q)
+        except PtError:
+            failed += 1
+        left = lib.fake_fail_new_left()
+        lib.fake_fail_new(-1)
+        if k % 7 == 0:
+            CALLS[name](r, sc, rs, q)
+        if left >= 0:  # the call made fewer allocations
+            break
+        if k % 5 == 4:  # again without idle lanes
+            r.close()
+            r.__init__()
+            scene(r)
+            r.set_options(options_for(rs))
+            r.clear()
+    r.close()
+    assert lib.fake_device_used() == 0 and lib.fake_pinned() == 0
+    print(f"{k} allocations, {failed} calls failed")
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_host_allocations_that_fail(name):
+    """In a process of its own: a call that cannot handle it ends the process."""
+    code = f"import test_host_memory as t; t.sweep({name!r})"
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join(sys.path))
+    p = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=600)
+    print(p.stdout)
+    assert p.returncode == 0, p.stderr[-2000:]
