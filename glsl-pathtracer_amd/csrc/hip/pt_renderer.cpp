@@ -976,7 +976,9 @@ void batch_images(pt_renderer_s* h, const pt_job* jobs, const BatchPlan& P) {
     std::sort(by_dst.begin(), by_dst.end(), [](const Part& a, const Part& b) { return a.dst < b.dst; });
     bool shared = false;
     for (size_t j = 1; j < by_dst.size(); ++j) shared |= by_dst[j].dst < by_dst[j - 1].dst + by_dst[j - 1].n;
-    ptx::Lanes lanes(h->device, shared ? 1 : static_cast<int>(std::min<size_t>(parts.size(), 64)), IMAGE_PART);
+    size_t largest = 0;
+    for (const Part& p : parts) largest = std::max(largest, p.n);
+    ptx::Lanes lanes(h->device, shared ? 1 : static_cast<int>(std::min<size_t>(parts.size(), 64)), largest);
     if (lanes.size() == 0) {
         for (const Part& p : parts) HIPCHK(hipMemcpyAsync(p.dst, p.src, p.n, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));

@@ -25,7 +25,7 @@ def lib():
                 getattr(_lib, fn).restype = C.c_int
         _lib.pt_last_error.argtypes = [C.c_void_p]
         _lib.pt_last_error.restype = C.c_char_p
-        for fn in ("fake_device_used", "fake_device_peak"):
+        for fn in ("fake_device_used", "fake_device_peak", "fake_pinned"):
             getattr(_lib, fn).restype = C.c_size_t
         _lib.fake_device_limit.argtypes = [C.c_size_t]
         _lib.fake_device_limit.restype = None

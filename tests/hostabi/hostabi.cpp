@@ -33,7 +33,7 @@ size_t fake_device_peak() {
 void fake_refuse_pinned(int on) { fake::state().refuse_pinned = on != 0; }
 void fake_fail_new(long after) { fake::until_failure = after; }
 long fake_fail_new_left() { return fake::until_failure; }
-int fake_pinned() { return fake::state().pinned; }
+size_t fake_pinned() { return fake::state().pinned; }
 }
 
 namespace ptk {

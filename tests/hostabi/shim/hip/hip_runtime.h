@@ -22,9 +22,9 @@ namespace fake {
 constexpr size_t MARK = 0x9e3779b97f4a7c15;
 struct State {
     std::mutex m;
-    size_t used = 0, peak = 0, limit = SIZE_MAX;
+    size_t used = 0, peak = 0, limit = SIZE_MAX, pinned = 0;
     bool refuse_pinned = false;
-    int pinned = 0, streams = 0;
+    int streams = 0;
 };
 inline State& state() {
     static State s;
@@ -69,15 +69,19 @@ inline hipError_t hipFree(void* p) {
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     fake::State& s = fake::state();
     std::lock_guard<std::mutex> g(s.m);
-    *p = s.refuse_pinned ? nullptr : std::malloc(n);
-    if (*p) ++s.pinned;
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    size_t* at = s.refuse_pinned ? nullptr : static_cast<size_t*>(std::malloc(n + 64));
+    *p = at ? reinterpret_cast<char*>(at) + 64 : nullptr;
+    if (!at) return hipErrorOutOfMemory;
+    at[0] = n;
+    s.pinned += n;
+    return hipSuccess;
 }
 inline hipError_t hipHostFree(void* p) {
     fake::State& s = fake::state();
     std::lock_guard<std::mutex> g(s.m);
-    --s.pinned;
-    std::free(p);
+    size_t* at = reinterpret_cast<size_t*>(static_cast<char*>(p) - 64);
+    s.pinned -= at[0];
+    std::free(at);
     return hipSuccess;
 }
 inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }

@@ -139,6 +139,17 @@ def test_depth_takes_little_memory(renderer, kind):
     assert used[1] - used[0] < (2 << 20) + room
 
 
+@pytest.mark.parametrize("mode", [0, 1])
+def test_small_batches_pin_little(renderer, mode):
+    """What a lane pins follows the largest part that the call copies."""
+    sc, rs = scene(renderer, mode=mode)
+    jobs = [dict(camera=sc.camera(), width=40 + k, height=64, spp=1, max_depth=2) for k in range(6)]
+    renderer.batch_render(jobs)
+    assert hostabi.lib().fake_pinned() <= 6 * (64 << 10) + 64
+    renderer.batch_render([dict(jobs[0], width=500, height=600)])
+    assert hostabi.lib().fake_pinned() <= 9 * (4 << 20)
+
+
 CALLS = {
     "upload": lambda r, sc, rs, q: r.upload_scene(sc),
     "closest 49": lambda r, sc, rs, q: r.closest_hit(q[0][:49], q[1][:49]),
