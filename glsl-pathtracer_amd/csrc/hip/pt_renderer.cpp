@@ -411,6 +411,8 @@ void supply_while_busy(pt_renderer_s* h, void* dst, size_t bytes) {
     (void)hipGetLastError();
 }
 
+bool blends(const pt_material& m) { return static_cast<int>(m.alphaMode) == ptd::ALPHA_MODE_BLEND; }
+
 ptd::PathBuf path_buf(pt_renderer_s* h) {
     ptd::PathBuf pb;
     pb.ro = h->p_ro.p; pb.rd = h->p_rd.p; pb.thr = h->p_thr.p; pb.rad = h->p_rad.p; pb.rng = h->p_rng.p;
@@ -1440,10 +1442,10 @@ int pt_upload_scene(pt_handle h, const pt_scene_view* v) {
         h->mats.upload(reinterpret_cast<const float4*>(v->materials), 8 * static_cast<size_t>(v->num_materials), s);
         h->inst.upload(insts.data(), insts.size(), s);
         h->lights.upload(lights.data(), lights.size(), s);
-        h->any_alpha = h->any_medium = h->any_blend = false;
+        h->any_alpha = h->any_medium = false;
+        h->any_blend = std::any_of(v->materials, v->materials + v->num_materials, blends);
         for (int i = 0; i < v->num_materials; ++i) {
             if (static_cast<int>(v->materials[i].alphaMode) != 0) h->any_alpha = true;
-            if (static_cast<int>(v->materials[i].alphaMode) == ptd::ALPHA_MODE_BLEND) h->any_blend = true;
             if (static_cast<int>(v->materials[i].mediumType) != 0) h->any_medium = true;
         }
         if (v->num_textures > 0 && v->texture_maps) {
@@ -1587,7 +1589,13 @@ int pt_update_instances(pt_handle h, const float* transforms, int32_t num_instan
                                      h->inst_blas4[i]);
         }
         h->inst.upload(insts.data(), insts.size(), h->stream);
-        if (materials) h->mats.upload(reinterpret_cast<const float4*>(materials), 8 * static_cast<size_t>(num_materials), h->stream);
+        if (materials) {
+            h->mats.upload(reinterpret_cast<const float4*>(materials), 8 * static_cast<size_t>(num_materials), h->stream);
+            // which kernels and which tree stochastic alpha takes follows the table in
+            // use (OPT_ALPHA_TEST and OPT_MEDIUM stay as the upload set them)
+            h->any_blend = std::any_of(materials, materials + num_materials, blends);
+            h->select_bvh();
+        }
         h->sc.inst = h->inst.p;
         h->sc.mats = h->mats.p;
         HIPCHK(hipStreamSynchronize(h->stream));
