@@ -551,8 +551,10 @@ __device__ __forceinline__ int tlas_kids(const DevScene& sc, int r, Kid k[4]) {
     k[1] = Kid{g.d.y, {g.b.z, g.b.w, g.c.x}, {g.c.y, g.c.z, g.c.w}};
     return 2;
 }
+// (planes in order, as slab() takes them: two-wide boxes are the caller's own)
 __device__ __forceinline__ bool outside(const Pyramid& P, const Kid& k) {
-    return outside(P, k.lo[0], k.lo[1], k.lo[2], k.hi[0], k.hi[1], k.hi[2]);
+    return outside(P, fminf(k.lo[0], k.hi[0]), fminf(k.lo[1], k.hi[1]), fminf(k.lo[2], k.hi[2]),
+                   fmaxf(k.lo[0], k.hi[0]), fmaxf(k.lo[1], k.hi[1]), fmaxf(k.lo[2], k.hi[2]));
 }
 // Entry of a tile. stack: CULL_STACK entries at stride `step`; a TLAS deeper
 // than that is not searched further and counts as hit.

@@ -101,3 +101,25 @@ def test_instance_boxes_are_tested(freq, far, width4):
     differ, hits, culled = tile_hits(sc, rs, sc.camera(), (0, 0, 50, 38), 16, bvh_width=width4)
     print(f"{differ} of {hits} hits differ, {culled} tiles culled")
     assert differ == 0 and hits > 1000 and culled > 100
+
+
+@pytest.mark.parametrize("width4", [2, 4])
+def test_boxes_with_swapped_planes(width4):
+    """A TLAS whose boxes have their planes swapped on some axes, which the slab
+    test takes as they are meant: the tiles do too."""
+    rng = np.random.default_rng(12)
+    sc, rs = scenes.instanced_spheres(num_instances=24, freq=3, width=160, height=96, spp=16, max_depth=1, extent=12.0)
+    v, cam = sc.view(), sc.camera()
+    nodes = np.ctypeslib.as_array(C.cast(v.nodes, C.POINTER(C.c_float)), (v.num_nodes, 9)).copy()
+    swap = rng.random((v.num_nodes, 3)) < 0.5
+    swap[:v.top_level_index] = False
+    lo, hi = nodes[:, :3].copy(), nodes[:, 3:6].copy()
+    nodes[:, :3], nodes[:, 3:6] = np.where(swap, hi, lo), np.where(swap, lo, hi)
+    v.nodes = C.cast(nodes.ctypes.data, type(v.nodes))
+    o = options_for(rs, bvh_width=width4)
+    out = [C.c_int(0) for _ in range(3)]
+    assert hostpath.lib().host_tile_hits(C.byref(v), C.byref(o), C.byref(cam), 0, 0, 20, 12, 16,
+                                         *(C.byref(c) for c in out)) == 0
+    differ, hits, culled = (c.value for c in out)
+    print(f"{differ} of {hits} hits differ")
+    assert differ == 0 and hits > 1000 and culled > 20
