@@ -123,3 +123,23 @@ def test_takeover_of_many_paths(renderer, kind, depth):
                                              use_graph=cadence - 1))
             got, = renderer.batch_render(jobs)
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("cadence", [1, 2])
+@pytest.mark.parametrize("depth", [15, 16, 24])
+def test_record_boundary(renderer, depth, cadence):
+    """The adjoint's record holds 16 bounces of 5.2M paths (2 GB hold 12) and all
+    bounces of a sixth of them: queried again beyond bounce 15 or recorded, the
+    gradient is the same up to the order of the sums (tolerance as above). A
+    seventh of the light and more comes from the bounces beyond at depth 24."""
+    size, spp = (1200, 864), 5
+    sc, rs = closed_room(*size, spp, depth)
+    renderer.upload_scene(sc)
+    dl = np.random.default_rng(6).normal(size=(size[1], size[0], 3)).astype(np.float32)
+    g = []
+    for wave_spp in (5, 1):
+        renderer.set_options(options_for(rs, wave_spp=wave_spp, compact_every=cadence))
+        renderer.set_camera(sc.camera())
+        g.append(renderer.adjoint(0, spp, dl).astype(np.float64))
+    assert np.abs(g[1]).max() > 0
+    assert np.abs(g[0] - g[1]).max() <= 6e-4 * np.abs(g[1]).max()
