@@ -179,8 +179,8 @@ inline Relayout relayout(const pt_bvh_node* flat, int num_nodes, int top, int nu
     if (top < 0 || top >= num_nodes) throw ArgError(PT_ERR_INVALID_ARG, "top_level_index out of range");
     st.push_back(top);
     std::vector<char> blas_seen(num_nodes, 0);
-    std::unordered_map<int, long long> blas_tris;  // triangles of each BLAS, by its root
-    long long* tris = nullptr;                     // of the BLAS walked: its nodes follow its root
+    std::vector<int> blas_tris(num_nodes, 0);  // triangles of each BLAS, at its root
+    int* tris = nullptr;                       // of the BLAS walked: its nodes follow its root
     while (!st.empty()) {
         int i = st.back();
         st.pop_back();
