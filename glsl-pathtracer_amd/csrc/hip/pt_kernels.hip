@@ -725,7 +725,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))
 // 0.94 -> 1.07. A wave takes its next paths up to 64 at a time, fewer towards the
 // end of the work (640x360 boxes 1.57 -> 1.42 ms), but with INLINE_NEE, where
 // the vertices' work keeps the SIMDs busy, never fewer (1001x563x2 volume MIS 2.26
-// ms against 2.37).
+// ms against 2.37). But for the last two batches per wave, which shrink, batches are
+// claimed from SHARDS counters as WorkCursor's are: with one for all, waves whose
+// camera rays see nothing waited for it (2560x1440 with one small sphere 0.73 ->
+// 0.30 ms). Longer claims cost views that see something more than they save (boxes
+// 640x360x4 1.9 -> 2.7 ms at up to 256 paths).
 template <bool PRIMARY, bool BATCH, bool INLINE_NEE, bool RECORD>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, const int* cells, int nb, int limit,
@@ -748,6 +752,9 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
     bool ovf = false, alive = false;
     int at = static_cast<int>(blockIdx.x) * per, end = min(at + per, count);  // the wave's items
     bool more = nw * per < count;
+    const int first = nw * per;  // of the claimed items
+    const int runs = max(0, (count - first) / 64 - 2 * nw), tail = first + 64 * runs;
+    int share = static_cast<int>(blockIdx.x) % SHARDS, left = runs > 0 ? SHARDS : 0;
     int slot = -1, max_depth = op0.max_depth;
     int tile = -1;  // of a camera ray that has an entry
     PathRegs p;
@@ -756,12 +763,32 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
         const int idle = 64 - __popcll(live);
         if (!live || idle >= refill) {
             if (at >= end && more) {
-                const int part = INLINE_NEE ? 64 : max(8, min(64, (count - end) / (2 * nw)));
-                int next = 0;
-                if (l == 0) next = atomicAdd(work, part);
-                at = __builtin_amdgcn_readfirstlane(next) + nw * per;
-                end = min(at + part, count);
-                more = at + part < count;
+                int run = runs;
+                while (left > 0) {
+                    int* c = work + (1 + share) * CELL;
+                    int n = 0;
+                    if (left < SHARDS)  // another share's counter is read before it is claimed from
+                        n = __builtin_amdgcn_readfirstlane(
+                            __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                    if (n * SHARDS + share < runs) {
+                        if (l == 0) n = atomicAdd(c, 1);
+                        run = __builtin_amdgcn_readfirstlane(n) * SHARDS + share;
+                        if (run < runs) break;
+                    }
+                    --left;
+                    share = share + 1 == SHARDS ? 0 : share + 1;
+                }
+                if (left > 0) {
+                    at = first + 64 * run;
+                    end = at + 64;
+                } else {
+                    const int part = INLINE_NEE ? 64 : max(8, min(64, (count - max(end, tail)) / (2 * nw)));
+                    int next = 0;
+                    if (l == 0) next = atomicAdd(work, part);
+                    at = __builtin_amdgcn_readfirstlane(next) + tail;
+                    end = min(at + part, count);
+                    more = at + part < count;
+                }
             }
             if (at < end) {
                 const int i = at + __popcll(~live & ((1ull << l) - 1));

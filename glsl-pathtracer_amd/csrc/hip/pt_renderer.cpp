@@ -433,15 +433,15 @@ void check_ready(pt_renderer_s* h) {
 //   [n+1, 2n+2)         hits entering shade at bounce b
 //   [2n+2, 3n+3)        shadow records of bounce b
 //   [3n+3, 4n+3)        stopped traversals of bounce b
-//   4n+3                the work counter of k_finish
-//   from 4n+4           work counters (ptd::SHARDS each) of the extend, shade,
+//   from 4n+3           the work counters of k_finish (1 + ptd::SHARDS)
+//   after them          work counters (ptd::SHARDS each) of the extend, shade,
 //                       shadow and resume stages of bounce b
 // A pass that stages more bounces than CELL_BOUNCES uses the cells again and
 // again: before bounces CELL_BOUNCES, 2 CELL_BOUNCES, ... they are cleared and
 // the count of the paths that enter moves to the first (launch_roll_cells), so
 // that a depth of a million does not take 4.6 GB of counters.
 constexpr int CELL_BOUNCES = 256;
-int counter_cells(int n) { return 4 * n + 4 + 4 * n * ptd::SHARDS; }
+int counter_cells(int n) { return 4 * n + 4 + (4 * n + 1) * ptd::SHARDS; }
 struct Cells {
     int* base;
     int n;
@@ -451,7 +451,7 @@ struct Cells {
     int* shadows(int b) const { return at(2 * (n + 1) + b); }
     int* conts(int b) const { return at(3 * (n + 1) + b); }
     int* finish() const { return at(4 * n + 3); }
-    int* work(int b, int stage) const { return at(4 * n + 4 + (4 * b + stage) * ptd::SHARDS); }
+    int* work(int b, int stage) const { return at(4 * n + 4 + (4 * b + 1 + stage) * ptd::SHARDS); }
     // Index of bounce b's cells; c_ext: the count of the paths that enter it.
     int bounce(int b, int*& c_ext, hipStream_t s) const {
         const int i = b % CELL_BOUNCES;
