@@ -782,7 +782,7 @@ k_finish(DevScene sc, DevOpts op0, PathBuf pb, const int* qa, const int* qb, con
                     at = first + 64 * run;
                     end = at + 64;
                 } else {
-                    const int part = INLINE_NEE ? 64 : max(8, min(64, (count - max(end, tail)) / (2 * nw)));
+                    const int part = INLINE_NEE ? 64 : max(8, min(64, (count - end) / (2 * nw)));
                     int next = 0;
                     if (l == 0) next = atomicAdd(work, part);
                     at = __builtin_amdgcn_readfirstlane(next) + tail;

@@ -527,13 +527,18 @@ struct Finish { int blocks, leave, whole; };
 // alpha lets paths go on without counting (1280x720x20 in the plain form, all lanes
 // / 8: Cornell box at depth 2 11.5 / 15.5 ms, 3 16.8 / 19.5, 4 21.3 / 21.6, 5 25.3 /
 // 23.0; media at depth 2 17.4 / 19.0, 3 22.8 / 21.4; 400x300x4 in k_finish, Cornell
-// box: 0.41 / 0.49, 0.58 / 0.57, 0.72 / 0.64, 0.85 / 0.68). inl (visibility inside the
-// vertices): only from 16 paths per lane of the two waves per SIMD on (900x700x8
-// volume MIS 7.1 -> 6.3 ms, blended alpha 7.1 -> 6.6; 1001x563x2 volume MIS 2.26 ->
-// 2.35, 1640x900 2.42 -> 2.41).
-int refill_lanes(const pt_renderer_s* h, const DevOpts& op, int max_depth, bool inl, long long paths) {
-    if (h->traced_tris > FEW_TRIS || max_depth <= ((op.flags & ptd::OPT_ALPHA_TEST) ? 2 : 3)) return 64;
-    return !inl || paths >= 16LL * 512 * h->num_cu ? 8 : 64;
+// box: 0.41 / 0.49, 0.58 / 0.57, 0.72 / 0.64, 0.85 / 0.68). In k_finish only from three
+// paths per lane of the two waves per SIMD on, as the last batches are small ones
+// that are better joined (Cornell box at depth 2: 192k paths 0.29 / 0.26, 260k 0.34 /
+// 0.29, 400k 0.29 / 0.32, 1.2M 0.34 / 0.40). inl (visibility inside the vertices): only
+// from 16 such paths on (900x700x8 volume MIS 7.1 -> 6.3 ms, blended alpha 7.1 -> 6.6;
+// 1001x563x2 volume MIS 2.26 -> 2.35, 1640x900 2.42 -> 2.41).
+int refill_lanes(const pt_renderer_s* h, const DevOpts& op, int max_depth, bool inl, long long paths, bool plain) {
+    if (h->traced_tris > FEW_TRIS) return 64;
+    const long long lanes = 512LL * h->num_cu;
+    const bool shallow = max_depth <= ((op.flags & ptd::OPT_ALPHA_TEST) ? 2 : 3);
+    if (shallow && (plain || paths >= 3 * lanes)) return 64;
+    return !inl || paths >= 16 * lanes ? 8 : 64;
 }
 
 Finish finish_setup(pt_renderer_s* h, bool inl) {
@@ -666,7 +671,7 @@ void run_bounces(pt_renderer_s* h, const DevOpts& op, const Wavefront& w, const 
         h->stage_begin(PT_STAGE_PLAIN, ev);
         ptk::launch_finish(s, w.fin.blocks, h->sc, op, pb0, nullptr, primary, w.inline_nee, h->qa.p, h->qb.p, cells.base, nb,
                            w.fin.leave, D, npaths, w.npix, fs, cells.finish(), h->spill.p, h->ovf.p, w.tiles,
-                           refill_lanes(h, op, op.max_depth, w.inline_nee, npaths), rec);
+                           refill_lanes(h, op, op.max_depth, w.inline_nee, npaths, false), rec);
         h->stage_end(PT_STAGE_PLAIN, ev);
     };
     if (w.nb == 0) {
@@ -1019,7 +1024,7 @@ void batch_render_plain(pt_renderer_s* h, const pt_job* jobs, int n) {
     const int2* tiles = tile_entries(h, op, h->b_jobs.p, n, static_cast<int>(P.items / 64), P.max_side, P.samples);
     hipEvent_t ev;
     h->stage_begin(PT_STAGE_BATCH, ev);
-    ptk::launch_plain_batch(s, blocks, bs, h->sc, op, h->b_jobs.p, n, static_cast<int>(P.items), refill_lanes(h, op, P.max_depth, inl, P.samples),
+    ptk::launch_plain_batch(s, blocks, bs, h->sc, op, h->b_jobs.p, n, static_cast<int>(P.items), refill_lanes(h, op, P.max_depth, inl, P.samples, true),
                             h->b_accum.p, h->counters.p, S, h->spill.p, h->ovf.p, inl, tiles);
     h->stage_end(PT_STAGE_BATCH, ev);
     HIPCHK(hipGetLastError());
@@ -1092,7 +1097,7 @@ void batch_render(pt_renderer_s* h, const pt_job* jobs, int n) {
             stage(PT_STAGE_PLAIN, [&] {
                 ptk::launch_finish(s, fin.blocks, h->sc, op, pb, &bb, primary, inl, h->qa.p, h->qb.p, cells.base, nb, fin.leave,
                                    D, 0, 0, 0, cells.finish(), h->spill.p, h->ovf.p, tiles,
-                                   refill_lanes(h, op, P.max_depth, inl, P.max_paths));
+                                   refill_lanes(h, op, P.max_depth, inl, P.max_paths, false));
             });
         };
         if (whole) finish(true, 0);
@@ -1188,7 +1193,7 @@ void render_plain(pt_renderer_s* h, int first_sample, int num_samples) {
         ptk::launch_zero_cells(h->stream, h->counters.p, ptd::SHARDS);
         h->stage_begin(PT_STAGE_PLAIN, ev);
         ptk::launch_plain(h->stream, blocks, bs, h->sc, op, h->accum.p, first_sample + k, spp,
-                          refill_lanes(h, op, op.max_depth, inl, static_cast<long long>(items) * spp), items, h->counters.p, S, h->spill.p,
+                          refill_lanes(h, op, op.max_depth, inl, static_cast<long long>(items) * spp, true), items, h->counters.p, S, h->spill.p,
                           h->work_counts.p, h->ovf.p, cw, inl, tiles);
         h->stage_end(PT_STAGE_PLAIN, ev);
         HIPCHK(hipGetLastError());
