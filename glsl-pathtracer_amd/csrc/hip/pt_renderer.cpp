@@ -518,6 +518,10 @@ ptd::ShadowBuf shadow_buf(pt_renderer_s* h) { return ptd::ShadowBuf{h->s_idx.p, 
 //   0.2M to 1M triangles over all instances: 1M 3.6 / 4.9 and 2.0 / 2.9; 2M
 //     5.7 / 5.9 and 2.5 / 3.3; 4M 9.9 / 7.7 and 3.4 / 3.6;
 //   21M triangles with foliage: 0.23M 19.1 / 20.3; 0.5M 30 / 26; 1M 48 / 39.
+// Around the lines (spheres, device time): 16k triangles 4.2M 1.93 / 2.10, 8.4M 3.40 /
+// 3.05; 18k 2.1M 1.32 / 1.65, 4.2M 2.11 / 2.21, 8.4M 3.85 / 3.22; 3.6M 2.1M 1.88 / 1.93,
+// 4.2M 3.25 / 2.66; 4.4M 0.5M 0.95 / 1.33, 2.1M 2.01 / 1.98; 16M 0.26M 1.03 / 1.37, 1M
+// 2.02 / 1.99: compact meshes alone would move the last line to 16M, foliage holds it.
 struct Finish { int blocks, leave, whole; };
 
 // How many lanes of a wave wait before they begin new paths (64: all), in k_finish
@@ -527,17 +531,17 @@ struct Finish { int blocks, leave, whole; };
 // alpha lets paths go on without counting (1280x720x20 in the plain form, all lanes
 // / 8: Cornell box at depth 2 11.5 / 15.5 ms, 3 16.8 / 19.5, 4 21.3 / 21.6, 5 25.3 /
 // 23.0; media at depth 2 17.4 / 19.0, 3 22.8 / 21.4; 400x300x4 in k_finish, Cornell
-// box: 0.41 / 0.49, 0.58 / 0.57, 0.72 / 0.64, 0.85 / 0.68). In k_finish only from three
-// paths per lane of the two waves per SIMD on, as the last batches are small ones
-// that are better joined (Cornell box at depth 2: 192k paths 0.29 / 0.26, 260k 0.34 /
-// 0.29, 400k 0.29 / 0.32, 1.2M 0.34 / 0.40). inl (visibility inside the vertices): only
-// from 16 such paths on (900x700x8 volume MIS 7.1 -> 6.3 ms, blended alpha 7.1 -> 6.6;
-// 1001x563x2 volume MIS 2.26 -> 2.35, 1640x900 2.42 -> 2.41).
+// box: 0.41 / 0.49, 0.58 / 0.57, 0.72 / 0.64, 0.85 / 0.68). At depth 3 k_finish needs
+// three paths per lane of the two waves per SIMD for that (Cornell box: 260k paths
+// 0.38 / 0.35, 400k 0.39 / 0.38, 520k 0.37 / 0.39, 1.2M 0.43 / 0.48; at depth 2 260k 0.28 /
+// 0.29, 1.2M 0.34 / 0.40). inl (visibility inside the vertices): only from 16 such
+// paths on (900x700x8 volume MIS 7.1 -> 6.3 ms, blended alpha 7.1 -> 6.6; 1001x563x2
+// volume MIS 2.26 -> 2.35, 1640x900 2.42 -> 2.41).
 int refill_lanes(const pt_renderer_s* h, const DevOpts& op, int max_depth, bool inl, long long paths, bool plain) {
     if (h->traced_tris > FEW_TRIS) return 64;
     const long long lanes = 512LL * h->num_cu;
     const bool shallow = max_depth <= ((op.flags & ptd::OPT_ALPHA_TEST) ? 2 : 3);
-    if (shallow && (plain || paths >= 3 * lanes)) return 64;
+    if (shallow && (plain || max_depth < 3 || paths >= 3 * lanes)) return 64;
     return !inl || paths >= 16 * lanes ? 8 : 64;
 }
 
