@@ -405,11 +405,12 @@ __device__ __forceinline__ void save_cont(const ContBuf& cb, int r, int slot, co
 // hits are compacted into the shade queue. At bounce 0 (PRIMARY) the input is
 // every slot of the pass and the camera ray is generated in place; BATCH
 // (bounce 0 of a batched pass) takes the slot count and each slot's job,
-// sample and pixel from the device-side pass state. Seven waves per SIMD (72
-// registers): at eight (64) more values spill and the traversal loop reloads
-// them around its stack pushes, which costs issue slots in a stage bound by
-// VALU issue (1080p: 19.6 -> 17.9 ms per frame; 4K heavy scene: 630 -> 569 ms;
-// six waves, 80 registers, is slower on both). A later bounce that at most
+// sample and pixel from the device-side pass state. Six waves per SIMD (80
+// registers): at seven (72) and eight (64) more values spill and the traversal
+// loop reloads them, which keeps the L1 return path, the stage's limit, busier
+// (closest hits of the 1080p frame 10.7 ms at six, 10.8 and 12.5; of the 4K foliage
+// frame 232 ms, 241 and 264; the capped kernel spills 20, 55 and 94). A later
+// bounce that at most
 // `leave` paths enter is left to k_finish.
 // CAPPED (later bounces): a traversal runs at most `budget` loop iterations
 // here; a wave does not wait on its longest rays. Stopped traversals go to the
@@ -420,7 +421,7 @@ __device__ __forceinline__ void save_cont(const ContBuf& cb, int r, int slot, co
 // shade stage reads the paths of a batch together (k_extend_resume writes the
 // slot there, or -1 for a miss, which the shade stage skips).
 template <bool COUNT, bool PRIMARY, bool BATCH, bool CAPPED = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))) k_extend(DevScene sc, DevOpts op, PathBuf pb, const int* __restrict__ qin,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 6))) k_extend(DevScene sc, DevOpts op, PathBuf pb, const int* __restrict__ qin,
                                                 const int* count_in, int npaths, int npix, int first_sample,
                                                 int* hitq, int* hit_count, int* work, int S, int* spill,
                                                 unsigned long long* counters, int* ovf_flag, BatchBuf bb,
@@ -511,7 +512,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7))
 // stack back on this thread's stack, the traversal run to its end, then the
 // same finish as the extend stage (records [0, min(*cont_count, cap))); the
 // slot, or -1 for a miss, goes to the hit-queue position the record kept.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7, 7)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 6)))
 k_extend_resume(DevScene sc, DevOpts op, PathBuf pb, ContBuf cb, const int* cont_count, int* hitq,
                 int* work, int S, int* spill, int* ovf_flag) {
     extern __shared__ int lds[];
