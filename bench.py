@@ -226,7 +226,7 @@ def batch_throughput(reps):
 
 def batch_sequential(reps):
     """The same 32 jobs rendered one after another, one pt_render per job
-    (plain: one kernel launch per sample; wavefront: the C3 launch
+    (plain: one kernel launch per 16 samples; wavefront: the C3 launch
     configuration without batching). Each job's image is bit-identical to its
     batched image. Device time summed over the jobs, best of `reps`."""
     from glslpt import scenes

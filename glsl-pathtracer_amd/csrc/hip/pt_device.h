@@ -844,7 +844,7 @@ __device__ __forceinline__ bool odd_ray(vec3 o, vec3 inv) {
 // its time on two things here: the issue slots of this code and the 112 bytes
 // a lane reads per node, which keep the CU's L1 return path busy (16 cycles per
 // 16-byte load of a wave, whatever lanes are active; at 1080p its data unit is
-// busy for 95% of the camera rays' cycles and 96% of the later rays', with 1.15
+// busy for 95% of the camera rays' cycles and 97% of the later rays', with 1.1
 // VALU instructions per cycle and CU).
 // Against slab() per child, a count of hits before the sort and a bounds check
 // per push, the node step went from about 165 to 120 VALU instructions:

@@ -200,7 +200,8 @@ typedef struct pt_stats {
 #define PT_STAGE_SHADE 2
 #define PT_STAGE_SHADOW 3
 #define PT_STAGE_ACCUM 4
-#define PT_STAGE_PLAIN 5
+#define PT_STAGE_PLAIN 5     /* the plain form; in the wavefront forms the launch that runs a pass's
+                                (remaining) paths to their end */
 #define PT_STAGE_ADJOINT 6   /* replay shade stage of pt_adjoint */
 #define PT_STAGE_BATCH 7     /* whole pass sequence of pt_batch_render */
 

@@ -336,6 +336,7 @@ def summarize(root, out_json):
     from the rocprofv3 runs under ROOT:
       fetch, write, tcc, sq   --pmc FETCH_SIZE / WRITE_SIZE / TCC_REQ_sum / SQ
                               counters of `profiling.py c2 64`, k_extend only
+      ta                      --pmc TA_TA_BUSY_sum TD_TD_BUSY_sum GRBM_GUI_ACTIVE of the same
       copy_fetch, copy_write  FETCH_SIZE / WRITE_SIZE of `profiling.py copy 1073741824`
       l2req                   TCC_REQ_sum of `profiling.py l2read 2 256 3`
       valusq                  SQ counters and GRBM_GUI_ACTIVE of `profiling.py valu 4096 3`
@@ -368,6 +369,12 @@ def summarize(root, out_json):
                     k["dispatches"] += 1
                 for c, v in cv.items():
                     k["sums"][c] = k["sums"].get(c, 0.0) + v
+    busy = {}  # the texture path's address and data units, summed over the CUs
+    for name, ds in _one(root, "ta").items():
+        b = busy.setdefault("camera" if "k_extend<false, true, false" in name else "later", {})
+        for cv in ds.values():
+            for c, v in cv.items():
+                b[c] = b.get(c, 0.0) + v
     cf = _one(root, "copy_fetch")["__amd_rocclr_copyBuffer"]
     cw = _one(root, "copy_write")["__amd_rocclr_copyBuffer"]
     nbytes = 1 << 30
@@ -398,6 +405,8 @@ def summarize(root, out_json):
         # occupancy: SQ_WAVE_CYCLES counts resident wave-cycles in units of 4 cycles; GRBM_GUI_ACTIVE
         # sums the busy cycles of the 8 XCDs
         per["waves_per_simd"] = 4 * sm["SQ_WAVE_CYCLES"] / (sm["GRBM_GUI_ACTIVE"] / 8 * MI355X_SIMDS)
+        cycles = busy[kind]["GRBM_GUI_ACTIVE"] / 8 * (MI355X_SIMDS // 4)
+        per["ta_busy"], per["td_busy"] = (busy[kind][c] / cycles for c in ("TA_TA_BUSY_sum", "TD_TD_BUSY_sum"))
         per["waves_per_simd_launched"] = sm["SQ_WAVES"] / k["dispatches"] / MI355X_SIMDS
         summary["kinds"][kind] = {"kernels": sorted(k["kernels"]), "dispatches": k["dispatches"], "steps": n,
                                   "per_step": per}
